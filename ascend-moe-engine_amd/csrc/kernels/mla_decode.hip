@@ -663,58 +663,75 @@ __device__ __forceinline__ void ZeroFill(const AttnArgs& a, int z, int seq, int 
   }
 }
 
-// Merges the `n` partials of (sequence, head): out = sum_c w_c O_c / sum_c w_c with
-// w_c = 2^(lse2_c - max lse2), in the order of the sequence's tiles. One wave, 8 output columns
-// per lane. Partial 0 sits in slot `first_slot`, partial i > 0 in slot `u0 + i`. Every partial
-// carries an LSE (-inf for an empty one, whose O row is not data), so the loads of a group of
-// eight partials are issued together.
+// What the partials of one (sequence, head) add up to, as one wave holds it: 8 output columns per
+// lane, sum_c w_c O_c and sum_c w_c with w_c = 2^(lse2_c - m).
+struct MergeState {
+  float acc[8];
+  float m = -__builtin_inff(), denom = 0.0f;
+};
+
+// Takes partials first, first + step, ... < n of (sequence, head), in the order of the sequence's
+// tiles. Partial 0 sits in slot `first_slot`, partial i > 0 in slot `u0 + i`. Every partial carries
+// an LSE (-inf for an empty one, whose O row is not data), so the loads of a group of eight partials
+// are issued together; the group is a uniform count, and what it does not hold is not asked for.
 // AGENT: the partials were written by other CUs of this launch (agent-scope loads); otherwise by
 // an earlier launch (plain streaming loads).
-template <bool MXQ, bool AGENT>
-__device__ __forceinline__ void MergeHead(const AttnArgs& a, int z, int seq, int head_in_group, int first_slot, int u0, int n, int lane) {
-  const int head = 64 * z + head_in_group;
-  float acc[8];
+template <bool AGENT>
+__device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_in_group, int first_slot, int u0, int first, int step,
+                                             int n, int lane, MergeState& s) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
-  float m = -__builtin_inff(), denom = 0.0f;
-  for (int c0 = 0; c0 < n; c0 += 8) {
+  for (int j = 0; j < 8; ++j) s.acc[j] = 0.0f;
+  for (int c0 = first; c0 < n; c0 += 8 * step) {
     u32x4 v[8];
     float l[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int c = min(c0 + u, n - 1);
-      const int64_t row = PartialRow(a, z, c == 0 ? first_slot : u0 + c, head_in_group);
+      const int c = c0 + u * step;
       if constexpr (AGENT) {
-        l[u] = c0 + u < n ? LoadAgentF32(a.partial_lse + row) : -__builtin_inff();
+        const int64_t row = PartialRow(a, z, c == 0 || n == 1 ? first_slot : u0 + min(c, n - 1), head_in_group);
+        l[u] = c < n ? LoadAgentF32(a.partial_lse + row) : -__builtin_inff();
         v[u] = LoadAgent16(a.partial_out + row * (kLatentDim * 2) + lane * 16);
       } else {
-        l[u] = c0 + u < n ? a.partial_lse[row] : -__builtin_inff();
-        v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.partial_out + row * (kLatentDim * 2) + lane * 16));
+        l[u] = -__builtin_inff();
+        v[u] = u32x4{0u, 0u, 0u, 0u};
+        if (c < n) {
+          const int64_t row = PartialRow(a, z, c == 0 ? first_slot : u0 + c, head_in_group);
+          l[u] = a.partial_lse[row];
+          v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.partial_out + row * (kLatentDim * 2) + lane * 16));
+        }
       }
     }
     if constexpr (AGENT) WaitAgentLoads(v);
-    float group_max = m;
+    float group_max = s.m;
 #pragma unroll
     for (int u = 0; u < 8; ++u) group_max = fmaxf(group_max, l[u]);
     if (group_max == -__builtin_inff()) continue;  // nothing but empty partials so far
-    const float rescale = __builtin_amdgcn_exp2f(m - group_max);  // 0 on the first group
-    m = group_max;
-    denom *= rescale;
+    const float rescale = __builtin_amdgcn_exp2f(s.m - group_max);  // 0 on the first group
+    s.m = group_max;
+    s.denom *= rescale;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[j] *= rescale;
+    for (int j = 0; j < 8; ++j) s.acc[j] *= rescale;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       if (l[u] == -__builtin_inff()) continue;  // empty or padding slot
-      const float w = __builtin_amdgcn_exp2f(l[u] - m);
-      denom += w;
+      const float w = __builtin_amdgcn_exp2f(l[u] - s.m);
+      s.denom += w;
       const unsigned words[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        acc[2 * j] += w * __builtin_bit_cast(float, words[j] << 16);
-        acc[2 * j + 1] += w * __builtin_bit_cast(float, words[j] & 0xffff0000u);
+        s.acc[2 * j] += w * __builtin_bit_cast(float, words[j] << 16);
+        s.acc[2 * j + 1] += w * __builtin_bit_cast(float, words[j] & 0xffff0000u);
       }
     }
   }
+}
+
+// Writes the output row of (sequence, head): out = sum_c w_c O_c / sum_c w_c. One wave.
+template <bool MXQ>
+__device__ __forceinline__ void FinishHead(const AttnArgs& a, int z, int seq, int head_in_group, int lane, const MergeState& s) {
+  const int head = 64 * z + head_in_group;
+  const float (&acc)[8] = s.acc;
+  const float m = s.m, denom = s.denom;
   // Nothing but empty partials yields zeros and lse = -inf.
   const float inv = denom == 0.0f ? 0.0f : 1.0f / denom;
   u32x4 packed;
@@ -732,14 +749,14 @@ __device__ __forceinline__ void MergeHead(const AttnArgs& a, int z, int seq, int
     for (int i = 0; i < 4; ++i) magnitude = MxMagnitudeMax(packed[i], magnitude);
     magnitude = max(magnitude, static_cast<unsigned>(__shfl_xor(static_cast<int>(magnitude), 1)));
     magnitude = max(magnitude, static_cast<unsigned>(__shfl_xor(static_cast<int>(magnitude), 2)));
-    const MxScale s = MxScaleFromMaxBits(magnitude);
+    const MxScale scale = MxScaleFromMaxBits(magnitude);
     u32x2 codes;
-    codes.x = MxEncodeWord(packed.x, s) | (MxEncodeWord(packed.y, s) << 16);
-    codes.y = MxEncodeWord(packed.z, s) | (MxEncodeWord(packed.w, s) << 16);
+    codes.x = MxEncodeWord(packed.x, scale) | (MxEncodeWord(packed.y, scale) << 16);
+    codes.y = MxEncodeWord(packed.z, scale) | (MxEncodeWord(packed.w, scale) << 16);
     *reinterpret_cast<u32x2*>(a.out_codes + seq * a.out_codes_seq_stride + head * a.out_codes_head_stride + lane * 8) = codes;
     if ((lane & 3) == 0) {
       reinterpret_cast<unsigned char*>(a.out_scales + seq * a.out_scales_seq_stride + head * a.out_scales_head_stride)[lane >> 2] =
-          static_cast<unsigned char>(s.code);
+          static_cast<unsigned char>(scale.code);
     }
   }
   if (a.lse != nullptr && lane == 0) {
@@ -869,7 +886,11 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
       if (share != 0) {
         for (int u = share == 2 ? 0 : rank; u < merge_units; u += share == 2 ? 1 : n) {
           const int h = u * kMergeHeads + wave0;
-          if (h < heads_here) MergeHead<MXQ, true>(a, z, seq, h, a.max_units + seq, u0, n, lane0);
+          if (h < heads_here) {
+            MergeState state;
+            TakePartials<true>(a, z, h, a.max_units + seq, u0, 0, 1, n, lane0, state);
+            FinishHead<MXQ>(a, z, seq, h, lane0, state);
+          }
         }
       }
       __syncthreads();  // scalar_lds[1] is free again
@@ -1476,10 +1497,16 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
 }
 
 // The merge as a launch of its own, for launches that have no counters to meet on: block =
-// (eight heads, sequence, head group); every wave repeats the cut of the flat tile axis and merges
-// one head.
-template <bool MXQ, bool SPARSE>
+// (8 / WAYS heads, sequence, head group); every wave repeats the cut of the flat tile axis. WAYS
+// waves share a head, wave w of them takes partials w, w + WAYS, ..., and the first adds up what
+// they hold through LDS. What bounds it is the chain of memory trips (lengths, then a group of eight
+// rows at a time) and how many rows are on their way at once: one wave per head leaves a launch of
+// few sequences with few waves and many partials each. Measured (64 heads, FP8, 3 sequences of 15k
+// to 33k tokens, about 85 partials per head): 18.6 us with one wave per head, 6.9 us with eight.
+template <bool MXQ, bool SPARSE, int WAYS>
 __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
+  __shared__ float shared_acc[WAYS > 1 ? kMergeHeads : 1][8][64];
+  __shared__ float shared_ends[WAYS > 1 ? kMergeHeads : 1][2];  // reference maximum and denominator
   const int lane = threadIdx.x & 63, wave = Uniform(threadIdx.x >> 6);
   // Workgroups go to the XCDs round-robin by linear id. The main launch put the units of XCD x's
   // share of the flat tile axis on XCD x; with equal lengths that is the x-th eighth of the
@@ -1492,8 +1519,9 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
     seq = (linear & (kXcds - 1)) * (gridDim.y / kXcds) + within / static_cast<int>(gridDim.x);
     group = within % static_cast<int>(gridDim.x);
   }
-  const int h = group * kMergeHeads + wave;
-  if (h >= min(64, a.heads - 64 * z)) return;
+  const int h = group * (kMergeHeads / WAYS) + wave / WAYS, way = wave % WAYS;
+  const bool has_head = h < min(64, a.heads - 64 * z);
+  if (WAYS == 1 && !has_head) return;
   SeqWindow<SPARSE> win;
   win.Load(a, lane, 0, 0, 0);
   int end_tiles = 0, end_live = 0, seq_tiles = 0, common_tiles = 0;
@@ -1508,13 +1536,66 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
     if (win.base + 64 >= a.batch) break;
     win.Next(a, lane);
   }
-  if (seq_tiles == 0) return;
+  if (seq_tiles == 0) return;  // (as is all below, the same for the whole workgroup)
   const Cut cut = MakeCut(a, win.EndTiles(), win.EndLive(), common_tiles, a.work_groups);
   const int seq_end = end_tiles + cut.pad * end_live;
   const int first_unit = (seq_end - seq_tiles) / cut.tiles_per_unit;
   const int partials = (seq_end - 1) / cut.tiles_per_unit - first_unit + 1;
   if (partials == 1) return;  // written by the workgroup that held the whole sequence
-  MergeHead<MXQ, false>(a, z, seq, h, a.max_units + seq, first_unit, partials, lane);
+  MergeState state;
+  if (has_head) TakePartials<false>(a, z, h, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
+  if constexpr (WAYS > 1) {
+    if (way != 0 && has_head) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) shared_acc[wave][j][lane] = state.acc[j];
+      if (lane == 0) {
+        shared_ends[wave][0] = state.m;
+        shared_ends[wave][1] = state.denom;
+      }
+    }
+    __syncthreads();
+    if (way != 0 || !has_head) return;
+    float top = state.m;
+#pragma unroll
+    for (int w = 1; w < WAYS; ++w) top = fmaxf(top, shared_ends[wave + w][0]);
+    if (top != -__builtin_inff()) {
+      const float own = __builtin_amdgcn_exp2f(state.m - top);
+      state.m = top;
+      state.denom *= own;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) state.acc[j] *= own;
+#pragma unroll
+      for (int w = 1; w < WAYS; ++w) {
+        const float weight = __builtin_amdgcn_exp2f(shared_ends[wave + w][0] - top);  // 0 for a wave without partials
+        state.denom += weight * shared_ends[wave + w][1];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) state.acc[j] += weight * shared_acc[wave + w][j][lane];
+      }
+    }
+  }
+  FinishHead<MXQ>(a, z, seq, h, lane, state);
+}
+
+// Waves per head of the second-launch merge, from the partials a sequence has on average. Measured,
+// append + attention + merge of a layer at 64 heads with one wave per head / with the choice below:
+// 256 partials per sequence (1 x 32000 tokens) 59.5 / 28.0 us, 64 (4 x 8000) 32.5 / 26.0, 32 (8 x 4000)
+// 28.1 / 25.3, 21 (12 x 3000) 27.5 / 26.3, 16 (16 x 4096) 32.5 / 32.0, 12 (20 x 4000) 38.1 / 37.7. At 8
+// (32 x 2048) two waves per head took 6.2 us where one takes 5.9: a head's rows fit one group of loads.
+int MergeWays(const AttnArgs& a) {
+  const int partials = a.max_units / std::max(a.batch, 1);
+  return partials >= 32 ? 8 : (partials >= 12 ? 4 : 1);
+}
+
+template <bool MXQ, bool SPARSE>
+hipError_t LaunchMerge(const AttnArgs& args, int head_groups, hipStream_t stream) {
+  const int ways = MergeWays(args), heads_per_block = kMergeHeads / ways;
+  const dim3 grid((std::min(64, args.heads) + heads_per_block - 1) / heads_per_block, args.batch, head_groups), block(kMergeHeads * 64);
+  switch (ways) {
+    case 8: hipLaunchKernelGGL((MlaMergeKernel<MXQ, SPARSE, 8>), grid, block, 0, stream, args); break;
+    case 4: hipLaunchKernelGGL((MlaMergeKernel<MXQ, SPARSE, 4>), grid, block, 0, stream, args); break;
+    default: hipLaunchKernelGGL((MlaMergeKernel<MXQ, SPARSE, 1>), grid, block, 0, stream, args); break;
+  }
+  return hipGetLastError();
 }
 
 // ---- selected-token attention in whole-sequence units of 16 heads ----------------------------
@@ -2085,7 +2166,11 @@ hipError_t LaunchHeadBlock(const AttnArgs& args, const dim3& units, hipStream_t 
 template <bool MXQ, bool SPARSE>
 hipError_t PrepareMerge() {
   hipFuncAttributes attributes;
-  return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&MlaMergeKernel<MXQ, SPARSE>));
+  for (const void* kernel : {reinterpret_cast<const void*>(&MlaMergeKernel<MXQ, SPARSE, 1>), reinterpret_cast<const void*>(&MlaMergeKernel<MXQ, SPARSE, 4>),
+                             reinterpret_cast<const void*>(&MlaMergeKernel<MXQ, SPARSE, 8>)}) {
+    if (hipError_t e = hipFuncGetAttributes(&attributes, kernel); e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 template <bool FP8, bool ALIGNED, bool MXQ, bool SPARSE>
@@ -2237,15 +2322,8 @@ hipError_t LaunchAttnDecode(const AttnArgs& args_in, hipStream_t stream) {
   }
   if (e != hipSuccess || merge_in_launch) return e;
   if (!AnySequenceSplit(args)) return hipSuccess;  // every sequence is written by the one unit that holds it
-  const dim3 merge_grid((std::min(64, args.heads) + kMergeHeads - 1) / kMergeHeads, args.batch, head_groups);
-  if (sparse) {
-    hipLaunchKernelGGL((MlaMergeKernel<false, true>), merge_grid, dim3(kMergeHeads * 64), 0, stream, args);
-  } else if (quantise) {
-    hipLaunchKernelGGL((MlaMergeKernel<true, false>), merge_grid, dim3(kMergeHeads * 64), 0, stream, args);
-  } else {
-    hipLaunchKernelGGL((MlaMergeKernel<false, false>), merge_grid, dim3(kMergeHeads * 64), 0, stream, args);
-  }
-  return hipGetLastError();
+  if (sparse) return LaunchMerge<false, true>(args, head_groups, stream);
+  return quantise ? LaunchMerge<true, false>(args, head_groups, stream) : LaunchMerge<false, false>(args, head_groups, stream);
 }
 
 // Split-KV partials for callers that cannot allocate: one array per GPU, held from module load to

@@ -1,0 +1,56 @@
+"""GPU parity of the variants of the split-KV decode attention, at the sizes where the choice between
+them changes, against the CPU oracle (float64 accumulation) with the tolerances of
+test_gpu_attention.py: 2e-2 of the peak for bf16 KV, 6e-2 for FP8 KV."""
+import math
+
+import numpy as np
+import pytest
+
+import kv_testing as kt
+
+pytestmark = pytest.mark.gpu
+
+LATENT, ROPE = kt.LATENT, kt.ROPE
+SCALE = 1.0 / math.sqrt(192.0)
+TOL_BF16, TOL_FP8 = 2e-2, 6e-2
+
+
+def _cache(ctxs, bs, seed, fp8=False, grow=None):
+    """A filled one-layer cache and its table; `grow(position)` scales the rows of a sequence."""
+    blocks = sum(-(-c // bs) for c in ctxs) + 3
+    table = kt.build_tables(ctxs, bs, blocks, seed=seed).table()
+    cache = kt.PagedCache(1, blocks, bs, fp8=fp8)
+    total = sum(ctxs)
+    latent, rope = kt.randn_bf16((1, total, LATENT), seed=seed + 1), kt.randn_bf16((1, total, ROPE), seed=seed + 2)
+    if grow is not None:
+        at = np.concatenate([np.arange(n) for n in ctxs])
+        factor = kt.torch.as_tensor(grow(at), dtype=kt.torch.float32)[None, :, None]
+        latent, rope = (latent.float() * factor).bfloat16(), (rope.float() * factor).bfloat16()
+    kt.append(cache, latent.cuda(), rope.cuda(), kt.dev_i32(kt.slots_for(table, ctxs, bs)))
+    return cache, table
+
+
+def _check(cache, table, ctxs, heads, seed, fp8=False, sparse=None, **options):
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=seed).cuda()
+    expected, expected_lse = kt.oracle_attention(cache, 0, q, table, ctxs, SCALE, sparse_indices=sparse)
+    if sparse is None:
+        out, lse, _ = kt.attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE, **options)
+    else:
+        out, lse, _ = kt.sparse_attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), kt.dev_i32(sparse), SCALE, **options)
+    got, peak = out.float().cpu().numpy(), np.abs(expected).max()
+    assert np.isfinite(got).all()
+    assert np.abs(got - expected).max() <= (TOL_FP8 if fp8 else TOL_BF16) * peak
+    live = np.asarray(ctxs) > 0
+    assert np.abs(lse.cpu().numpy()[live] - expected_lse[live]).max() <= 2e-2
+
+
+# Partials per sequence on average (256 units on a full chip): 85 (eight waves per head in the merge),
+# 36 with 128 heads in two groups, 19 and 12 (four), 10 (one); empty sequences and sequences of one
+# unit among them, head counts that leave waves of the merge without a head.
+@pytest.mark.parametrize("ctxs,heads,fp8", [([3000, 1, 1900], 64, True), ([900, 2100, 40], 128, False), ([4096], 16, False),
+                                            ([300] * 12 + [0], 48, False), ([130] * 21, 64, True), ([200] * 24 + [1700], 32, False)])
+def test_merge_with_several_waves_per_head(ctxs, heads, fp8):
+    cache, table = _cache(ctxs, 64, seed=901, fp8=fp8)
+    # units of one tile as well: more partials than one round of the waves takes
+    for options in ({"selection_units": 1}, {"chunk_tiles": 1}):
+        _check(cache, table, ctxs, heads, seed=905, fp8=fp8, **options)
