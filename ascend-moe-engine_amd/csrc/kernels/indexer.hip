@@ -275,24 +275,10 @@ __global__ __launch_bounds__(kScoreThreads) void IndexerScoreKernel(IndexerArgs 
 
 constexpr int kSelectThreads = 1024;
 constexpr int kSelectWaves = kSelectThreads / 64;
-constexpr int kKeysPerThread = 8;                              // one 16-byte load
-constexpr int kKeysPerPass = kSelectThreads * kKeysPerThread;  // 8192
-
-// kKeysPerThread consecutive keys of a sequence starting at `first` (a multiple of 8; rows are
-// 256-byte aligned); keys past the end read as -1, below every real key.
-__device__ __forceinline__ void LoadKeys(const unsigned short* keys, int first, int n, int (&out)[kKeysPerThread]) {
-#pragma unroll
-  for (int part = 0; part < kKeysPerThread / 8; ++part) {
-    const int at = first + 8 * part;
-    u32x4 v = {0u, 0u, 0u, 0u};
-    if (at < n) v = *reinterpret_cast<const u32x4*>(keys + at);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      out[8 * part + 2 * i] = at + 2 * i < n ? static_cast<int>(v[i] & 0xffffu) : -1;
-      out[8 * part + 2 * i + 1] = at + 2 * i + 1 < n ? static_cast<int>(v[i] >> 16) : -1;
-    }
-  }
-}
+constexpr int kHeldPieces = 4;                                   // 16-byte pieces (eight keys) a thread keeps in registers
+constexpr int kKeysPerPiece = kSelectThreads * 8;                // 8192
+constexpr int kHistogramCopies = 32;
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 
 // Inclusive prefix sum over the 64 lanes with data-parallel-primitive moves (no LDS crossbar, no
 // wait per step): four shifted adds inside each row of 16 lanes, then lane 15 of rows 0 and 2 onto
@@ -307,41 +293,57 @@ __device__ __forceinline__ int WaveInclusiveScan(int v) {
   return v;
 }
 
-// The byte value that holds the `wanted`-th largest entry of a 256-bin histogram, and the number
-// of entries above that bin, found by the first wavefront (four bins per lane, a suffix sum over
-// the lanes) and handed to everyone through `result`.
-__device__ __forceinline__ void FindBin(const int* histogram, int wanted, int* result, int tid) {
-  if (tid < 64) {
-    int bins[4], mine = 0;
+// Adds up the copies of the histogram and finds the byte value that holds the `wanted`-th largest
+// entry and the number of entries above it. Thread t owns counters 8 t .. 8 t + 7, a quarter of bin
+// t / 4, and leaves them cleared; behind the barrier every wavefront looks for the bin itself (four
+// bins per lane, a prefix sum over the lanes), so the answer needs no second one.
+__device__ __forceinline__ void FindBin(int* counters, int* totals, int wanted, int tid, int* bin, int* entries_above) {
+  u32x4* own = reinterpret_cast<u32x4*>(counters + 8 * tid);
+  const u32x4 lo = own[0], hi = own[1];
+  own[0] = own[1] = u32x4{0u, 0u, 0u, 0u};
+  int sum = static_cast<int>(((lo.x + lo.y) + (lo.z + lo.w)) + ((hi.x + hi.y) + (hi.z + hi.w)));
+  sum += __builtin_amdgcn_update_dpp(0, sum, 0xb1, 0xf, 0xf, false);  // quad_perm:[1,0,3,2]
+  sum += __builtin_amdgcn_update_dpp(0, sum, 0x4e, 0xf, 0xf, false);  // quad_perm:[2,3,0,1]
+  if ((tid & 3) == 0) totals[tid >> 2] = sum;
+  __syncthreads();
+  const int lane = tid & 63;
+  const u32x4 four = *reinterpret_cast<const u32x4*>(totals + 4 * lane);
+  const int mine = static_cast<int>((four.x + four.y) + (four.z + four.w));
+  // the sum over the lanes above this one: everything minus this lane's inclusive prefix
+  const int inclusive = WaveInclusiveScan(mine);
+  int above = __builtin_amdgcn_readlane(inclusive, 63) - inclusive;
+  int found = -1, found_above = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      bins[i] = histogram[4 * tid + i];
-      mine += bins[i];
+  for (int i = 3; i >= 0; --i) {
+    const int here = static_cast<int>(four[i]);
+    if (above < wanted && wanted <= above + here) {
+      found = 4 * lane + i;
+      found_above = above;
     }
-    // the sum over the lanes above this one: everything minus this lane's inclusive prefix
-    const int inclusive = WaveInclusiveScan(mine);
-    int above = __builtin_amdgcn_readlane(inclusive, 63) - inclusive;
-#pragma unroll
-    for (int i = 3; i >= 0; --i) {
-      if (above < wanted && wanted <= above + bins[i]) {
-        result[0] = 4 * tid + i;
-        result[1] = above;
-      }
-      above += bins[i];
-    }
+    above += here;
   }
+  const int holder = __builtin_ctzll(__builtin_amdgcn_ballot_w64(found >= 0));  // exactly one lane: 1 <= wanted <= entries
+  *bin = __builtin_amdgcn_readlane(found, holder);
+  *entries_above = __builtin_amdgcn_readlane(found_above, holder);
 }
 
 // One workgroup per sequence. The k-th largest key is found by its high and then its low byte (two
 // 256-bin histograms); then an ordered compaction writes the positions above it and the first ones
-// equal to it. Thread t holds keys 8t .. 8t+7 of each pass of 8192, so thread order is position
-// order. (Measured at 8192 keys: this 7.1 us; 256 threads of 32 keys 10.0 us; sixteen one-bit
-// counting rounds 14 us; one atomic per key with a serial bin search 31.6 us.)
+// equal to it. Thread t holds `pieces` consecutive groups of eight keys, as many as the sequence
+// needs for all threads together (1 up to 8192 keys, 4 up to 32768), so thread order is position
+// order and the keys are read once; longer sequences go in sweeps of 32768 that are read again, from
+// the L2, for each of the three steps.
+// What bounds it is one CU's time for a sequence: the chain of its steps and the counting. Scores
+// crowd into a few exponents, so one histogram is a handful of hot counters: with 32 copies, lane L
+// counting in copy L % 32, the 64 lanes of an addition meet at most in pairs and never in a bank.
+// Measured, top 512 of 8192 keys (32 sequences) and top 2048 of up to 32768 (9 sequences):
+// 5.8 -> 5.7 us and 18.7 -> 10.3 us against one histogram and passes of 8192 keys that re-read the later
+// ones in every step. (A separate path without the per-key end tests measured the same.)
 __global__ __launch_bounds__(kSelectThreads) void IndexerSelectKernel(IndexerArgs a) {
-  __shared__ int histograms[2][256];  // of the high bytes, then of the low bytes among the keys with the high byte found
-  __shared__ int founds[2][2];
-  __shared__ int wave_counts[kSelectWaves];
-  const int seq = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ __attribute__((aligned(16))) int counters[256 * kHistogramCopies];  // copy c of bin b at 32 b + c
+  __shared__ __attribute__((aligned(16))) int totals[2][256];  // one per byte, so that no barrier separates the rounds
+  __shared__ unsigned wave_counts[kSelectWaves];
+  const int seq = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = max(min(a.seq_lens[seq], a.max_seq_len), 0);
   const int k = a.sparse_count;
   int32_t* out = a.indices_out + seq * a.indices_seq_stride;
@@ -350,90 +352,111 @@ __global__ __launch_bounds__(kSelectThreads) void IndexerSelectKernel(IndexerArg
     return;
   }
   const unsigned short* keys = a.keys + seq * a.keys_stride;
-  const int passes = (n + kKeysPerPass - 1) / kKeysPerPass;
-  int first[kKeysPerThread];  // the keys of pass 0 stay in registers; later passes are read again from L2
-  LoadKeys(keys, tid * kKeysPerThread, n, first);
-
-  int prefix = 0, wanted = k;  // the bytes of the k-th largest key decided so far; how many of the candidates are wanted
-  // both histograms are cleared here and each round has its own result words, so a round is two
-  // barriers: the counts complete, the bin found
-  if (tid < 512) histograms[tid >> 8][tid & 255] = 0;
-  __syncthreads();
+  const int pieces = min((n + kKeysPerPiece - 1) / kKeysPerPiece, kHeldPieces);
+  const int sweep_keys = pieces * kKeysPerPiece, sweeps = (n + sweep_keys - 1) / sweep_keys;
+  u32x4 held[kHeldPieces];
+  // The keys of one sweep; a row starts on 256 bytes and is a multiple of them long, so a piece that
+  // begins inside the sequence can be read whole.
+  const auto load = [&](int sweep) __attribute__((always_inline)) {
+    const int first = sweep * sweep_keys + tid * (8 * pieces);
 #pragma unroll
-  for (int shift = 8; shift >= 0; shift -= 8) {
-    int* histogram = histograms[shift == 8 ? 0 : 1];
-    int* found = founds[shift == 8 ? 0 : 1];
-    for (int pass = 0; pass < passes; ++pass) {
-      int more[kKeysPerThread];
-      if (pass > 0) LoadKeys(keys, pass * kKeysPerPass + tid * kKeysPerThread, n, more);
-      const int (&mine)[kKeysPerThread] = pass == 0 ? first : more;
-      // Candidates: real keys (shift 8) or keys whose high byte is the one found (shift 0).
-      // Scores crowd into a few exponents, so the candidates that share the byte of the thread's
-      // first key go in as one addition instead of one each to the same counter.
-      const int lead = (mine[0] >> shift) & 255;
-      int same = 0;
-#pragma unroll
-      for (int i = 0; i < kKeysPerThread; ++i) {
-        const int key = mine[i];
-        const bool candidate = shift == 8 ? key >= 0 : (key >> 8) == prefix;
-        const int byte = (key >> shift) & 255;
-        if (candidate && byte == lead) {
-          ++same;
-        } else if (candidate) {
-          atomicAdd(&histogram[byte], 1);
-        }
-      }
-      if (same > 0) atomicAdd(&histogram[lead], same);
+    for (int p = 0; p < kHeldPieces; ++p) {
+      held[p] = u32x4{0u, 0u, 0u, 0u};
+      if (p < pieces && first + 8 * p < n) held[p] = *reinterpret_cast<const u32x4*>(keys + first + 8 * p);
     }
-    __syncthreads();
-    FindBin(histogram, wanted, found, tid);
-    __syncthreads();
-    prefix = shift == 8 ? found[0] : (prefix << 8) | found[0];
-    wanted -= found[1];
+    return first;
+  };
+  int first = load(0);
+  {
+    u32x4* own = reinterpret_cast<u32x4*>(counters + 8 * tid);
+    own[0] = own[1] = u32x4{0u, 0u, 0u, 0u};
   }
-  const int threshold = prefix, equal_wanted = wanted, greater_total = k - wanted;
+  __syncthreads();
 
+  int* const copy = counters + (lane & (kHistogramCopies - 1));
+  int high = 0, low = 0, above_high = 0, above_low = 0;
+  for (int sweep = 0; sweep < sweeps; ++sweep) {
+    if (sweep > 0) first = load(sweep);
+#pragma unroll
+    for (int p = 0; p < kHeldPieces; ++p) {
+      if (p >= pieces) break;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const unsigned byte = (held[p][i >> 1] >> (i & 1 ? 24 : 8)) & 255u;
+        if (first + 8 * p + i < n) atomicAdd(copy + byte * kHistogramCopies, 1);
+      }
+    }
+  }
+  __syncthreads();
+  FindBin(counters, totals[0], k, tid, &high, &above_high);
+  if (sweeps > 1) first = load(0);
+  for (int sweep = 0; sweep < sweeps; ++sweep) {
+    if (sweep > 0) first = load(sweep);
+#pragma unroll
+    for (int p = 0; p < kHeldPieces; ++p) {
+      if (p >= pieces) break;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const unsigned key = (held[p][i >> 1] >> (i & 1 ? 16 : 0)) & 0xffffu;
+        if ((key >> 8) == static_cast<unsigned>(high) && first + 8 * p + i < n) atomicAdd(copy + (key & 255u) * kHistogramCopies, 1);
+      }
+    }
+  }
+  __syncthreads();
+  FindBin(counters, totals[1], k - above_high, tid, &low, &above_low);
+  const unsigned short threshold = static_cast<unsigned short>((high << 8) | low);
+  const int greater_total = above_high + above_low, equal_wanted = k - greater_total;
+
+  if (sweeps > 1) first = load(0);
   int greater_done = 0, equal_done = 0;
-  for (int pass = 0; pass < passes; ++pass) {
-    int mine[kKeysPerThread];
-    if (pass == 0) {
+  for (int sweep = 0; sweep < sweeps; ++sweep) {
+    if (sweep > 0) first = load(sweep);
+    // bit i of the masks: whether the thread's i-th key is above the threshold, or equal to it
+    unsigned greater = 0u, equal = 0u;
 #pragma unroll
-      for (int i = 0; i < kKeysPerThread; ++i) mine[i] = first[i];
-    } else {
-      LoadKeys(keys, pass * kKeysPerPass + tid * kKeysPerThread, n, mine);
-    }
-    int greater = 0, equal = 0;
+    for (int p = 0; p < kHeldPieces; ++p) {
+      if (p >= pieces) break;
 #pragma unroll
-    for (int i = 0; i < kKeysPerThread; ++i) {
-      greater += mine[i] > threshold ? 1 : 0;
-      equal += mine[i] == threshold ? 1 : 0;
+      for (int pair = 0; pair < 4; ++pair) {
+        const u16x2 two = __builtin_bit_cast(u16x2, static_cast<unsigned>(held[p][pair]));
+        const u16x2 limit = {threshold, threshold}, one = {1, 1};
+        const unsigned above = __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_elementwise_sub_sat(two, limit), one));
+        const unsigned other = __builtin_bit_cast(unsigned, __builtin_elementwise_min(static_cast<u16x2>(two ^ limit), one));
+        greater |= ((above | (above >> 15)) & 3u) << (8 * p + 2 * pair);
+        equal |= (((other | (other >> 15)) & 3u) ^ 3u) << (8 * p + 2 * pair);
+      }
     }
-    // exclusive prefix over the threads of both counts at once (each below 2^16 per pass)
-    const int packed = greater | (equal << 16);
-    const int inclusive = WaveInclusiveScan(packed);
-    __syncthreads();  // wave_counts of the previous pass have been read
+    const int real = n - first;
+    if (real < 8 * kHeldPieces) {
+      const unsigned mask = real <= 0 ? 0u : (1u << real) - 1u;
+      greater &= mask;
+      equal &= mask;
+    }
+    // exclusive prefix over the threads of both counts at once (each at most 32768 per sweep)
+    const unsigned packed = static_cast<unsigned>(__builtin_popcount(greater)) | (static_cast<unsigned>(__builtin_popcount(equal)) << 16);
+    const unsigned inclusive = static_cast<unsigned>(WaveInclusiveScan(static_cast<int>(packed)));
+    if (sweep > 0) __syncthreads();  // wave_counts of the previous sweep have been read
     if (lane == 63) wave_counts[wave] = inclusive;
     __syncthreads();
-    int before = inclusive - packed, all = 0;
+    unsigned before = inclusive - packed, all = 0u;
 #pragma unroll
     for (int v = 0; v < kSelectWaves; ++v) {
-      const int c = wave_counts[v];
+      const unsigned c = wave_counts[v];
       if (v < wave) before += c;
       all += c;
     }
-    int greater_at = greater_done + (before & 0xffff), equal_at = equal_done + (before >> 16);
-    const int base = pass * kKeysPerPass + tid * kKeysPerThread;
-#pragma unroll
-    for (int i = 0; i < kKeysPerThread; ++i) {
-      if (mine[i] > threshold) {
-        out[greater_at++] = base + i;
-      } else if (mine[i] == threshold) {
-        if (equal_at < equal_wanted) out[greater_total + equal_at] = base + i;
-        ++equal_at;
-      }
+    int32_t* to = out + greater_done + static_cast<int>(before & 0xffffu);
+    while (greater != 0u) {
+      *to++ = first + __builtin_ctz(greater);
+      greater &= greater - 1u;
     }
-    greater_done += all & 0xffff;
-    equal_done += all >> 16;
+    int rank = equal_done + static_cast<int>(before >> 16);
+    while (equal != 0u && rank < equal_wanted) {
+      out[greater_total + rank++] = first + __builtin_ctz(equal);
+      equal &= equal - 1u;
+    }
+    greater_done += static_cast<int>(all & 0xffffu);
+    equal_done += static_cast<int>(all >> 16);
   }
 }
 

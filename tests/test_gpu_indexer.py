@@ -148,6 +148,16 @@ def test_index_key_append_matches_the_oracle_quantiser(bs):
     assert lib.mlakvIndexKeyAppend(C.byref(view), rows_d.data_ptr(), D * 2, slots_d.data_ptr(), 0, kt.stream_ptr()) == 0
 
 
+# One piece of eight keys per thread up to 8192 keys, four up to 32768, sweeps of 32768 beyond; the
+# edges of each, a last piece that is not full, selections that end inside a run of equal keys.
+@pytest.mark.parametrize("seq_lens,k", [([8191, 8192, 8193], 2048), ([16384, 16385, 24577], 700), ([32761, 32768, 32769], 2048),
+                                        ([2, 70001], 1)])
+def test_selection_at_the_edges_of_pieces_and_sweeps(seq_lens, k):
+    _run(seq_lens, 64, 16, k, seed=140)
+    got = _run(seq_lens, 64, 16, k, seed=141, zero_query=True)
+    assert all(row.tolist() == list(range(k)) for row in got)
+
+
 def test_all_equal_scores_select_the_first_positions():
     got = _run([1000, 300], 64, 64, 256, seed=102, zero_query=True)
     assert got[0].tolist() == list(range(256)) and got[1].tolist() == list(range(256))
