@@ -751,8 +751,8 @@ __device__ __forceinline__ void FinishHead(const AttnArgs& a, int z, int seq, in
     magnitude = max(magnitude, static_cast<unsigned>(__shfl_xor(static_cast<int>(magnitude), 2)));
     const MxScale scale = MxScaleFromMaxBits(magnitude);
     u32x2 codes;
-    codes.x = MxEncodeWord(packed.x, scale) | (MxEncodeWord(packed.y, scale) << 16);
-    codes.y = MxEncodeWord(packed.z, scale) | (MxEncodeWord(packed.w, scale) << 16);
+    codes.x = MxEncodeFour(packed.x, packed.y, scale);
+    codes.y = MxEncodeFour(packed.z, packed.w, scale);
     *reinterpret_cast<u32x2*>(a.out_codes + seq * a.out_codes_seq_stride + head * a.out_codes_head_stride + lane * 8) = codes;
     if ((lane & 3) == 0) {
       reinterpret_cast<unsigned char*>(a.out_scales + seq * a.out_scales_seq_stride + head * a.out_scales_head_stride)[lane >> 2] =
@@ -1409,7 +1409,7 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
                   const MxScale s = MxScaleFromMaxBits(magnitude);
   #pragma unroll
                   for (int half = 0; half < 2; ++half) {
-                    const unsigned four = MxEncodeWord(packed[half].x, s) | (MxEncodeWord(packed[half].y, s) << 16);
+                    const unsigned four = MxEncodeFour(packed[half].x, packed[half].y, s);
                     __builtin_nontemporal_store(four, reinterpret_cast<unsigned*>(codes_row + 16 * (kDvPerWave * hw + 2 * k + half) + 4 * g));
                   }
                   scale_codes |= s.code << (8 * k);

@@ -33,16 +33,19 @@ __device__ __forceinline__ unsigned MxMagnitudeMax(unsigned word, unsigned runni
   return max(running, max(lo, hi));
 }
 
-// Two bf16 values (one dword, low half first) -> their two codes in the low 16 bits.
+// Four bf16 values (two dwords, low halves first) -> their four codes.
 // v_cvt_pk_fp8_f32 rounds to nearest even onto the E4M3 grid for |v| < 464 and returns NaN beyond,
-// so the clamp supplies the saturation.
-__device__ __forceinline__ unsigned MxEncodeWord(unsigned word, const MxScale& s) {
-  if (s.nan) return ((word >> 8) & 0x80u) | ((word >> 16) & 0x8000u) | 0x7f7fu;
-  float lo = __builtin_bit_cast(float, word << 16) * s.inverse;
-  float hi = __builtin_bit_cast(float, word & 0xffff0000u) * s.inverse;
-  lo = fminf(fmaxf(lo, -448.0f), 448.0f);
-  hi = fminf(fmaxf(hi, -448.0f), 448.0f);
-  return static_cast<unsigned>(__builtin_amdgcn_cvt_pk_fp8_f32(lo, hi, 0, false)) & 0xffffu;
+// so the clamp (one median of three per value) supplies the saturation; a block with a NaN does not
+// get there. The second conversion writes the upper half of the first one's destination.
+__device__ __forceinline__ unsigned MxEncodeFour(unsigned first, unsigned second, const MxScale& s) {
+  if (s.nan) {
+    return ((first >> 8) & 0x80u) | ((first >> 16) & 0x8000u) | ((second << 8) & 0x800000u) | (second & 0x80000000u) | 0x7f7f7f7fu;
+  }
+  const auto scaled = [&](unsigned bits) __attribute__((always_inline)) {
+    return __builtin_amdgcn_fmed3f(__builtin_bit_cast(float, bits) * s.inverse, -448.0f, 448.0f);
+  };
+  const int low = __builtin_amdgcn_cvt_pk_fp8_f32(scaled(first << 16), scaled(first & 0xffff0000u), 0, false);
+  return static_cast<unsigned>(__builtin_amdgcn_cvt_pk_fp8_f32(scaled(second << 16), scaled(second & 0xffff0000u), low, true));
 }
 
 }  // namespace mlakv

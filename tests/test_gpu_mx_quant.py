@@ -79,6 +79,18 @@ def test_standalone_strided_rows_ragged_row_count_and_argument_checks():
     torch.cuda.synchronize()
 
 
+# 524,288 items of eight values are dealt one per thread, one row more two per thread: narrow rows
+# (several in a workgroup), rows a little longer than a workgroup's items, rows of a whole attention output.
+@pytest.mark.parametrize("rows,cols", [(131072, 32), (131073, 32), (3737, 1120), (1021, 4128), (128, 32768), (129, 32768)])
+def test_standalone_where_items_per_thread_change_and_rows_wrap(rows, cols):
+    x = kt.randn_bf16((rows, cols), seed=79, outlier_fraction=0.01)
+    x[rows - 1, cols - 1] = float("nan")
+    codes, scales = _quant(x.cuda())
+    want_codes, want_scales = orc.mx_quant_rows(kt.bits16(x))
+    assert np.array_equal(scales, want_scales)
+    assert np.array_equal(codes, want_codes)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("options", [{}, {"chunk_tiles": 2}, {"chunk_tiles": 100}, {"chunk_tiles": 1, "merge_mode": 1}])
 def test_attention_epilogue_equals_quantising_the_bf16_output(fp8, options):
