@@ -149,7 +149,7 @@ __device__ __forceinline__ void StoreStepWords(const WORDS& w) {
   }
 }
 
-constexpr int kAppendRows = 4;      // FP8: rows per wavefront
+constexpr int kAppendRows = 4;      // FP8: rows per wavefront of a large append
 constexpr int kAppendRowsBf16 = 1;  // bf16: a pure copy ran fastest with one row per wavefront (8 layers x 311k rows: 984 us, 1081 with two, 1106 with four)
 
 template <typename WORDS>
@@ -312,28 +312,28 @@ __device__ __forceinline__ void QuantizeRowAndStore(const AppendArgs& a, int lay
 // Quantize-on-append: per-row absmax over latent+rope by wave shuffles, scale = absmax/448,
 // code = e4m3(x / scale) with the correctly rounded quotient. Each lane quantizes the 8 latent
 // values it loaded (8-byte store) and one of the 64 rope values (1-byte store).
-template <typename WORDS>
+template <int ROWS, typename WORDS>
 __global__ __launch_bounds__(kThreads) void AppendFp8Kernel(AppendArgs a, WORDS w) {
   static_assert(kRopeDim == kWave, "one rope element per lane");
   StoreStepWords(w);
   const int lane = threadIdx.x & (kWave - 1);
-  const int token0 = Uniform((blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)) * kAppendRows);
+  const int token0 = Uniform((blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)) * ROWS);
   const int layer = blockIdx.y;
   if (token0 >= a.num_tokens) return;
   int my_slot = -1;
-  if (lane < kAppendRows && token0 + lane < a.num_tokens) my_slot = SlotOf(a, w, token0 + lane);
+  if (lane < ROWS && token0 + lane < a.num_tokens) my_slot = SlotOf(a, w, token0 + lane);
   // the usual block sizes are powers of two: a shift then, not a division per row
   const int block_shift = (a.block_size & (a.block_size - 1)) == 0 ? __builtin_ctz(static_cast<unsigned>(a.block_size)) : -1;
-  u32x4 lv[kAppendRows];
-  unsigned short rv[kAppendRows];
+  u32x4 lv[ROWS];
+  unsigned short rv[ROWS];
 #pragma unroll
-  for (int i = 0; i < kAppendRows; ++i) {
+  for (int i = 0; i < ROWS; ++i) {
     const int token = min(token0 + i, a.num_tokens - 1);  // a repeated row is loaded and never stored
     lv[i] = Load16(a.latent_src.base + layer * a.latent_src.layer_stride + token * a.latent_src.row_stride + lane * 16);
     rv[i] = *reinterpret_cast<const unsigned short*>(a.rope_src.base + layer * a.rope_src.layer_stride + token * a.rope_src.row_stride + lane * 2);
   }
 #pragma unroll
-  for (int i = 0; i < kAppendRows; ++i) {
+  for (int i = 0; i < ROWS; ++i) {
     const int slot = __builtin_amdgcn_readlane(my_slot, i);
     if (slot < 0) continue;
     const int block = block_shift >= 0 ? slot >> block_shift : slot / a.block_size;
@@ -663,11 +663,28 @@ __global__ __launch_bounds__(kThreads) void StoreWordsKernel(StoreWordsArgs args
 
 }  // namespace
 
+namespace {
+// Rows per wavefront of the quantising append. Up to 8192 rows the chip holds a wavefront for each,
+// and the launch is one chain of loads, reduction and stores: a second, third and fourth row in the
+// same wavefront only make it longer (64 rows: 4.8 us with
+// four, 2.9 us with one).
+template <typename WORDS>
+void LaunchAppendFp8(const AppendArgs& args, const WORDS& words, hipStream_t stream) {
+  constexpr int64_t kResidentWaves = 8192;
+  if (static_cast<int64_t>(args.num_tokens) * args.num_layers <= kResidentWaves) {
+    const dim3 grid(DivUp(args.num_tokens, kWavesPerGroup), args.num_layers);
+    hipLaunchKernelGGL((AppendFp8Kernel<1, WORDS>), grid, dim3(kThreads), 0, stream, args, words);
+  } else {
+    const dim3 grid(DivUp(args.num_tokens, kWavesPerGroup * kAppendRows), args.num_layers);
+    hipLaunchKernelGGL((AppendFp8Kernel<kAppendRows, WORDS>), grid, dim3(kThreads), 0, stream, args, words);
+  }
+}
+}  // namespace
+
 hipError_t LaunchAppend(const AppendArgs& args, hipStream_t stream) {
   if (args.num_tokens <= 0 || args.num_layers <= 0) return hipSuccess;
   if (args.fp8) {
-    const dim3 grid(DivUp(args.num_tokens, kWavesPerGroup * kAppendRows), args.num_layers);
-    hipLaunchKernelGGL(AppendFp8Kernel<NoStepWords>, grid, dim3(kThreads), 0, stream, args, NoStepWords{});
+    LaunchAppendFp8(args, NoStepWords{}, stream);
   } else {
     const dim3 grid(DivUp(args.num_tokens, kWavesPerGroup * kAppendRowsBf16), args.num_layers);
     hipLaunchKernelGGL(AppendBf16Kernel<NoStepWords>, grid, dim3(kThreads), 0, stream, args, NoStepWords{});
@@ -689,8 +706,7 @@ hipError_t LaunchAppendWithWords(const AppendArgs& args, const int32_t* host_wor
   words.dst = dst;
   words.scatter_dst = scatter_dst;
   if (args.fp8) {
-    const dim3 grid(DivUp(args.num_tokens, kWavesPerGroup * kAppendRows), args.num_layers);
-    hipLaunchKernelGGL(AppendFp8Kernel<StepWords>, grid, dim3(kThreads), 0, stream, args, words);
+    LaunchAppendFp8(args, words, stream);
   } else {
     const dim3 grid(DivUp(args.num_tokens, kWavesPerGroup * kAppendRowsBf16), args.num_layers);
     hipLaunchKernelGGL(AppendBf16Kernel<StepWords>, grid, dim3(kThreads), 0, stream, args, words);
@@ -796,7 +812,8 @@ hipError_t PreparePagedCopyKernels() {
   if (once.state[device] == 1) return hipSuccess;
   const void* kernels[] = {
       reinterpret_cast<const void*>(&AppendBf16Kernel<NoStepWords>), reinterpret_cast<const void*>(&AppendBf16Kernel<StepWords>),
-      reinterpret_cast<const void*>(&AppendFp8Kernel<NoStepWords>),  reinterpret_cast<const void*>(&AppendFp8Kernel<StepWords>),
+      reinterpret_cast<const void*>(&AppendFp8Kernel<1, NoStepWords>), reinterpret_cast<const void*>(&AppendFp8Kernel<1, StepWords>),
+      reinterpret_cast<const void*>(&AppendFp8Kernel<kAppendRows, NoStepWords>), reinterpret_cast<const void*>(&AppendFp8Kernel<kAppendRows, StepWords>),
       reinterpret_cast<const void*>(&GatherBf16TileKernel<kGatherTileRows>), reinterpret_cast<const void*>(&GatherBf16Kernel),
       reinterpret_cast<const void*>(&GatherFp8Kernel), reinterpret_cast<const void*>(&CopyBlocksKernel<64, 8>),
       reinterpret_cast<const void*>(&CopyBlocksKernel<32, 4>), reinterpret_cast<const void*>(&StoreWordsKernel)};

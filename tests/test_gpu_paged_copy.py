@@ -253,6 +253,28 @@ def test_fp8_quantize_on_append_and_dequant_gather_bit_exact(bs):
     assert bool(((x - y).abs() <= bound).all())
 
 
+# One row per wavefront up to 8192 rows over all layers, four beyond (a last wavefront of one to three rows).
+@pytest.mark.parametrize("layers,tokens", [(2, 4096), (3, 2731), (1, 8193), (1, 8194), (1, 8195)])
+def test_fp8_append_on_both_sides_of_the_rows_per_wavefront_bit_exact(layers, tokens):
+    bs = 64
+    blocks = -(-tokens // bs) + 1
+    cache = kt.PagedCache(layers, blocks, bs, fp8=True)
+    latent_src = kt.randn_bf16((layers, tokens, LATENT), seed=12, outlier_fraction=0.01).cuda()
+    rope_src = kt.randn_bf16((layers, tokens, ROPE), seed=13, outlier_fraction=0.01).cuda()
+    slots = np.random.default_rng(14).permutation(blocks * bs)[:tokens].astype(np.int32)
+    slots[tokens - 2] = -1
+    kt.append(cache, latent_src, rope_src, kt.dev_i32(slots))
+    torch.cuda.synchronize()
+    lat, rop, scl = _oracle_planes(layers, blocks, bs, fp8=True)
+    live = slots >= 0
+    for layer in range(layers):
+        orc.append_rows_fp8(lat[layer], rop[layer], scl[layer], bs, kt.bits16(latent_src[layer])[live],
+                            kt.bits16(rope_src[layer])[live], slots[live])
+        assert cache.scale_np(layer).tobytes() == scl[layer].tobytes()
+        assert cache.latent_np(layer).tobytes() == lat[layer].tobytes()
+        assert cache.rope_np(layer).tobytes() == rop[layer].tobytes()
+
+
 def test_fp8_quantize_rows_at_the_edges_of_the_arithmetic_bit_exact():
     """Rows where the quantiser's shortcuts do not apply or must not matter, against the oracle bit
     for bit: magnitudes so small that the scale's reciprocal leaves the normal range (every lane
