@@ -54,7 +54,7 @@ struct NormRopeAppendArgs {
   int64_t q_rope_token_stride;
   int64_t q_rope_head_stride;
   int num_heads;
-  int items_per_token;       // set by the launcher: 1 + groups of eight query heads
+  int items_per_token;       // set by the launcher: 1 + groups of query heads
 };
 
 struct GatherArgs {

@@ -167,3 +167,33 @@ def test_query_rope_slices_rotate_in_place_with_the_key(heads):
     rope_plane = np.zeros((blocks * bs, ROPE), dtype=np.uint16)
     rope_plane[slots] = got_kv[:, LATENT:]
     assert np.array_equal(cache.rope_np(0), rope_plane.reshape(-1))
+
+
+# 2048 wavefronts with eight heads each at most, 32 heads each beyond: both sides of the line, head
+# counts that leave a wavefront part of its heads, values so small that the products are subnormal
+# (bf16 keeps 7 bits of them: the bound is one bf16 step or one step of the subnormal grid).
+@pytest.mark.parametrize("tokens,heads", [(1024, 1), (1025, 1), (409, 32), (410, 32), (410, 33), (700, 9), (300, 100), (1, 128)])
+def test_query_heads_on_both_sides_of_the_split(tokens, heads):
+    bs, max_pos = 64, 128
+    cache = kt.PagedCache(1, -(-tokens // bs), bs)
+    lib = ffi.load()
+    kv_d = kt.randn_bf16((tokens, LATENT + ROPE), seed=41).cuda()
+    q = kt.randn_bf16((tokens, heads, ROPE), seed=42)
+    q[tokens // 2] *= 2.0 ** -126
+    q_d, gamma_d = q.cuda(), torch.ones(LATENT, dtype=torch.bfloat16, device="cuda")
+    cos, sin = _tables(max_pos)
+    cos_d, sin_d = cos.cuda(), sin.cuda()
+    positions = np.random.default_rng(43).integers(0, max_pos, tokens).astype(np.int32)
+    positions_d, slots_d = kt.dev_i32(positions), kt.dev_i32(np.arange(tokens, dtype=np.int32))
+    row = (LATENT + ROPE) * 2
+    ffi.check(lib.mlakvNormRopeAppend(C.byref(cache.view), 0, kv_d.data_ptr(), row, gamma_d.data_ptr(), EPS, cos_d.data_ptr(),
+                                      sin_d.data_ptr(), ROPE * 2, positions_d.data_ptr(), slots_d.data_ptr(), tokens,
+                                      None, 0, None, 0, q_d.data_ptr(), heads * ROPE * 2, ROPE * 2, heads, kt.stream_ptr()))
+    torch.cuda.synchronize()
+    x = q.double().numpy()
+    c, s = (table.double().numpy()[positions][:, None] for table in (cos, sin))
+    half = ROPE // 2
+    want = x * c + np.concatenate([-x[..., half:], x[..., :half]], axis=-1) * s
+    # half a bf16 step of the result, and the fp32 rounding of two products that may cancel
+    bound = 2.0 ** -8 * np.abs(want) + 2.0 ** -23 * (np.abs(x) + np.abs(np.roll(x, half, axis=-1))) + 2.0 ** -133
+    assert (np.abs(q_d.double().cpu().numpy() - want) <= bound).all()
