@@ -344,6 +344,12 @@ int64_t CapUnitTiles(int32_t block_size, bool sparse) {
   return cap < 1 ? 1 : cap;
 }
 
+// What the workgroups that share a unit of 16 heads leave in the workspace: `parts` partials of 16
+// rows per (sequence, 16 heads) and, behind the rows of all of them, their LSEs (4 x 16 floats each).
+uint64_t HeadBlockPartialBytes(int32_t batch, int32_t heads, int32_t parts) {
+  return static_cast<uint64_t>(batch) * (heads / 16) * parts * (16 * mlakv::kLatentDim * 2 + 4 * 16 * sizeof(float));
+}
+
 struct PlanShape {
   int64_t max_tiles, head_groups, cap, units;
   uint64_t workspace;
@@ -368,15 +374,19 @@ PlanShape ShapeOf(int32_t batch, int32_t heads, int32_t max_seq_len, int32_t blo
   const uint64_t rows = static_cast<uint64_t>(shape.head_groups) * static_cast<uint64_t>(shape.units + batch) * 64;
   // bf16 partial outputs, then fp32 partial log-sum-exps
   shape.workspace = rows * mlakv::kLatentDim * 2 + ((rows * sizeof(float) + 255) & ~255ull);
-  // Halved whole-selection units: two partials of 16 rows per (sequence, 16 heads) and, behind the
-  // rows of all of them, their LSEs (2 x 4 x 16 floats each).
-  const uint64_t halved = static_cast<uint64_t>(batch) * (heads / 16) * (32 * mlakv::kLatentDim * 2 + 2 * 4 * 16 * sizeof(float));
+  const uint64_t halved = HeadBlockPartialBytes(batch, heads, 2);
   if (halved_units && halved > shape.workspace) shape.workspace = halved;
   return shape;
 }
 
+// Workgroups of a unit of 16 heads that is shared: four while four per unit fit the CUs once, else
+// two. Measured, append + attention of a layer, whole contexts (us, one / two / four workgroups): batch 8,
+// 64 heads, bf16, 256 tokens 13.1 / 13.3 / 13.3; 384: 16.5 / 14.9 / 14.5; 512: 19.3 / 16.5 / 15.4; 768: 24.6 /
+// 19.2 / 16.9; batch 16, 600: 21.5 / 18.3 / 16.5; 7 x 128 heads, 600: 21.3 / 18.0 / 16.5; FP8 alike.
+int32_t SharedUnitParts(int64_t pairs) { return 4 * pairs <= ComputeUnits() ? 4 : 2; }
+
 // How a whole-context launch whose longest context is `bound` tokens cuts its work: 0 = the
-// 64-head kernel's flat cut, 1 = one workgroup per (sequence, 16 heads), 2 = two. Measured on
+// 64-head kernel's flat cut, 1 = one workgroup per (sequence, 16 heads), 2 or 4 = that many. Measured on
 // MI355X, bf16 and FP8 caches alike (64 heads unless said; us, 64-head kernel / one workgroup per
 // unit / two): batch 1 .. 32 (and 16 x 128, 64 x 16 heads), 128 tokens 14.5-16.8 / 8.3-8.5 / 8.7-9.9;
 // 256: 17.0-19.2 / 10.3-11.4 / 10.1-11.6; 512: 16.4-21.4 / 15.4-17.7 / 12.8-15.0; 768: 16.5-22.5 /
@@ -389,7 +399,7 @@ int32_t ShortContextUnits(const mlakvAttnPlan* plan, int32_t bound) {
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK) return 1;
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) return 2;
   const int64_t pairs = static_cast<int64_t>(plan->batch) * (plan->heads / 16);
-  if (2 * pairs <= ComputeUnits()) return bound <= 256 ? 1 : (bound <= 768 ? 2 : 0);
+  if (2 * pairs <= ComputeUnits()) return bound <= 256 ? 1 : (bound <= 768 ? SharedUnitParts(pairs) : 0);
   if (pairs <= ComputeUnits()) return bound <= 512 ? 1 : 0;
   if (pairs <= 2 * ComputeUnits()) return bound <= 256 ? 1 : 0;
   return 0;
@@ -686,6 +696,17 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
   args.merge_in_launch = plan->merge_mode == MLAKV_ATTN_MERGE_IN_LAUNCH;
   args.fp8 = cache->dtype == MLAKV_DTYPE_FP8_E4M3;
   args.head_block_units = plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK ? 1 : (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES ? 2 : 0);
+  const int64_t pairs = static_cast<int64_t>(plan->batch) * (plan->heads / 16);
+  // (the parts' partials must fit the plan's workspace, which is sized for the split and, with a
+  // selection, for two parts)
+  const auto partial_bytes = [&]() { return HeadBlockPartialBytes(plan->batch, plan->heads, args.head_block_units); };
+  const auto shrink_to_workspace = [&]() {
+    while (args.head_block_units > 1 && partial_bytes() > plan->workspace_bytes) args.head_block_units /= 2;
+  };
+  if (sparse && args.head_block_units == 2 && args.sparse_count > 256) {
+    args.head_block_units = SharedUnitParts(pairs);
+    shrink_to_workspace();
+  }
   if (!sparse) {
     // A whole context that is short: the units of the selected-token attention (one workgroup, or
     // two, per sequence and 16 heads; no selection, every position of the context) are ahead of the
@@ -698,13 +719,12 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
       for (int32_t i = 0; i < plan->batch; ++i) bound = std::max(bound, std::min(std::max(host_lens[i], 0), args.max_tokens));
     }
     args.head_block_units = ShortContextUnits(plan, bound);
-    const uint64_t halved = static_cast<uint64_t>(plan->batch) * (plan->heads / 16) * (32 * mlakv::kLatentDim * 2 + 2 * 4 * 16 * sizeof(float));
-    if (args.head_block_units == 2 && halved > plan->workspace_bytes) args.head_block_units = 1;  // (the halves' partials must fit what the plan sized for the split)
+    shrink_to_workspace();
     if (quant != nullptr && args.head_block_units != 0) {
       // The units have no quantising epilogue: they write bf16 rows (the caller's, or rows of the
-      // workspace behind the halves' partials) and the standalone quantiser follows in the same
+      // workspace behind the parts' partials) and the standalone quantiser follows in the same
       // stream; its codes are those of the fused epilogue, by construction of both from the bf16 rows.
-      const uint64_t rows_offset = args.head_block_units == 2 ? ((halved + 255) & ~255ull) : 0;
+      const uint64_t rows_offset = args.head_block_units > 1 ? ((partial_bytes() + 255) & ~255ull) : 0;
       const uint64_t rows_bytes = static_cast<uint64_t>(plan->batch) * plan->heads * mlakv::kLatentDim * 2;
       const bool own_rows = out == nullptr;
       const bool uniform = (own_rows || out_seq_stride == plan->heads * out_head_stride) &&

@@ -1616,15 +1616,15 @@ hipError_t LaunchMerge(const AttnArgs& args, int head_groups, hipStream_t stream
 //     multiplies it with its 128 columns of V.
 // The tile ring, the operand layouts and the barrier per tile are those of the kernel above.
 //
-// HALVES: two workgroups per (sequence, 16 heads), neighbours on one XCD, each with one half of the
-// selection's tiles, so that twice as many CUs (and twice as many rows in flight) work on a launch
-// that has fewer units than the chip has CUs. The exchange is a matter between the two output waves
-// that hold the same 128 columns, one in each workgroup: each leaves its normalised slice (bf16
-// rows and a log2-domain LSE per head, agent-scope stores) in the workspace and counts itself on
-// the word of (pair, slice); the one that finds the other's count there reads that slice back,
-// combines the two and writes the output. Nobody waits, no barrier is involved: the first to
-// arrive leaves. The words are zero between launches (the second to arrive clears its word). A
-// selection of a single tile is taken by the first workgroup alone.
+// PARTS: two or four workgroups per (sequence, 16 heads), neighbours on one XCD, each with an equal
+// share of the selection's tiles, so that more CUs (and more rows in flight) work on a launch that
+// has fewer units than the chip has CUs. The exchange is a matter between the output waves that hold
+// the same 128 columns, one in each workgroup: each leaves its normalised slice (bf16 rows and a
+// log2-domain LSE per head, agent-scope stores) in the workspace and counts itself on the word of
+// (unit, slice); the one that finds every other count there reads the slices back, combines them and
+// writes the output. Nobody waits, no barrier is involved: those that arrive earlier leave. The words
+// are zero between launches (the last to arrive clears its word). A selection of fewer tiles than
+// parts is taken by the first of them, one tile each.
 constexpr int kHbWaves = kWaves, kHbThreads = kHbWaves * 64;
 constexpr int kHbLoaders = kScoreWaves;  // the waves that fetch the tiles when every row is a plain row
 template <bool FP8>
@@ -1644,7 +1644,7 @@ struct GeomHeadBlock {
 template <bool FP8>
 constexpr int kHeadBlockKSteps = FP8 ? 10 : kKSteps / 2;
 
-template <bool HALVES, bool FP8>
+template <int PARTS, bool FP8>
 __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArgs a) {
   using G = GeomHeadBlock<FP8>;
   using T = Geom<FP8>;
@@ -1657,8 +1657,8 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
   // the head blocks of a sequence are neighbours among them.
   const int head_blocks = a.heads >> 4;  // heads is a multiple of 16
   const int rest = blockIdx.x >> 3;
-  const int half = HALVES ? rest & 1 : 0;
-  const int unit = HALVES ? rest >> 1 : rest;
+  const int part = rest % PARTS;
+  const int unit = rest / PARTS;
   const int hb = unit % head_blocks;
   const int seq = (unit / head_blocks) * kXcds + (blockIdx.x & (kXcds - 1));
   if (seq >= a.batch) return;
@@ -1754,11 +1754,12 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
   // Every row a real row of the pool (the usual case): the tile loads need no case distinction.
   const bool plain_rows = Uniform(outside) == 0;
   const int all_tiles = (seq_len + kTileTokens - 1) / kTileTokens;
-  // two workgroups share a selection of at least two tiles: the first ceil(all / 2), then the rest
-  const bool shared = HALVES && all_tiles >= 2;
-  if (HALVES && !shared && half != 0) return;
-  const int first_tile = shared && half != 0 ? (all_tiles + 1) >> 1 : 0;
-  const int ntiles = shared ? (half != 0 ? all_tiles >> 1 : (all_tiles + 1) >> 1) : all_tiles;
+  // the workgroups that take part, at most one per tile, share the tiles evenly
+  const int parts = min(PARTS, max(all_tiles, 1));
+  if (part >= parts) return;
+  const bool shared = parts > 1;
+  const int first_tile = (part * all_tiles + parts - 1) / parts;
+  const int ntiles = ((part + 1) * all_tiles + parts - 1) / parts - first_tile;
   if (ntiles == 0) {  // nothing selected: zeros, lse = -inf
     for (int h = wave; h < 16; h += kHbWaves) {
       *reinterpret_cast<u32x4*>(a.out + seq * a.out_seq_stride + (16 * hb + h) * a.out_head_stride + lane * 16) = u32x4{0u, 0u, 0u, 0u};
@@ -2094,48 +2095,62 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
     };
     u32x4 v[4];
     if (shared) {
-      // This half's partial at (pair, half) of the workspace: 16 rows of 1 KB, and behind the rows
-      // of all pairs the 16 LSEs once per slice, so that each wave's count covers what its partner reads.
+      // This part's partial at (unit, part) of the workspace: 16 rows of 1 KB, and behind the rows
+      // of all units the 16 LSEs once per slice, so that each wave's count covers what its partners read.
       const int pair = seq * head_blocks + hb;
-      const int64_t row0 = static_cast<int64_t>(2 * pair + half) * 16, other0 = static_cast<int64_t>(2 * pair + (half ^ 1)) * 16;
-      float* lses = reinterpret_cast<float*>(a.partial_out + static_cast<int64_t>(a.batch) * head_blocks * 32 * (kLatentDim * 2));
+      const int64_t unit_row0 = static_cast<int64_t>(pair) * (PARTS * 16);
+      float* lses = reinterpret_cast<float*>(a.partial_out + static_cast<int64_t>(a.batch) * head_blocks * (PARTS * 16) * (kLatentDim * 2)) +
+                    unit_row0 * 4 + 16 * hw + i16;                                      // + part * 64
+      char* slices = a.partial_out + unit_row0 * (kLatentDim * 2) + kSliceBytes * hw + piece * 16;  // + (16 part + row) KB
       rows_of_o(v);
-      char* mine = a.partial_out + row0 * (kLatentDim * 2) + kSliceBytes * hw + piece * 16;
 #pragma unroll
-      for (int it = 0; it < 4; ++it) StoreAgent16(mine + (4 * it + sub) * (kLatentDim * 2), v[it]);
-      if (g == 0) StoreAgentF32(lses + (row0 * 4 + 16 * hw) + i16, lse2);
+      for (int it = 0; it < 4; ++it) StoreAgent16(slices + (16 * part + 4 * it + sub) * (kLatentDim * 2), v[it]);
+      if (g == 0) StoreAgentF32(lses + part * 64, lse2);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partial stores are complete
       unsigned* word = a.sync + 4 * pair + hw;
       unsigned arrived = 0u;
       if (lane == 0) arrived = __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (Uniform(arrived) == 0u) return;  // the other half's wave will find this slice
+      if (Uniform(arrived) != static_cast<unsigned>(parts - 1)) return;  // the last part's wave will find this slice
       if (lane == 0) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const float lse2_other = LoadAgentF32(lses + (other0 * 4 + 16 * hw) + i16);
-      const char* theirs = a.partial_out + other0 * (kLatentDim * 2) + kSliceBytes * hw + piece * 16;
+      // Whichever part arrives last, the result is the same: every partial enters as the bf16 rows
+      // that were stored, in the order of the parts (this wave's own among them, read back as well;
+      // a part that does not exist repeats the last one with weight 0).
+      float lses2[PARTS], top = lse2;
+      u32x4 slice[PARTS][4];
 #pragma unroll
-      for (int it = 0; it < 4; ++it) v[it] = LoadAgent16(theirs + (4 * it + sub) * (kLatentDim * 2));
-      asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : : "memory");
+      for (int p = 0; p < PARTS; ++p) {
+        const int from = min(p, parts - 1);
+        lses2[p] = LoadAgentF32(lses + from * 64);
 #pragma unroll
-      for (int it = 0; it < 4; ++it) *reinterpret_cast<u32x4*>(stage + (4 * it + sub) * kStageRow + piece * 16) = v[it];
-      // Whichever half arrives second, the result is the same: both partials enter as the bf16
-      // rows that were stored, the first half's term first.
-      const float top = fmaxf(lse2, lse2_other);
-      const float w_mine = __builtin_amdgcn_exp2f(lse2 - top), w_theirs = __builtin_amdgcn_exp2f(lse2_other - top);
-      const float inv_w = 1.0f / (w_mine + w_theirs);
-      const bool second_half = half != 0;
-      const float c_first = (second_half ? w_theirs : w_mine) * inv_w, c_second = (second_half ? w_mine : w_theirs) * inv_w;
+        for (int it = 0; it < 4; ++it) slice[p][it] = LoadAgent16(slices + (16 * from + 4 * it + sub) * (kLatentDim * 2));
+      }
 #pragma unroll
-      for (int n = 0; n < kDvPerWave; ++n) {
-        const u32x2 packed = *reinterpret_cast<const u32x2*>(stage + i16 * kStageRow + (16 * n + 4 * g) * 2);
-        const float theirs[4] = {__builtin_bit_cast(float, packed.x << 16), __builtin_bit_cast(float, packed.x & 0xffff0000u),
-                                 __builtin_bit_cast(float, packed.y << 16), __builtin_bit_cast(float, packed.y & 0xffff0000u)};
+      for (int p = 0; p < PARTS; ++p) {
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(slice[p][0]), "+v"(slice[p][1]), "+v"(slice[p][2]), "+v"(slice[p][3]) : : "memory");
+        top = fmaxf(top, lses2[p]);
+      }
+      float weight[PARTS], total = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float mine = static_cast<float>(static_cast<__bf16>(o[n][j]));
-          o[n][j] = (second_half ? theirs[j] : mine) * c_first + (second_half ? mine : theirs[j]) * c_second;
+      for (int p = 0; p < PARTS; ++p) {
+        weight[p] = p < parts ? __builtin_amdgcn_exp2f(lses2[p] - top) : 0.0f;
+        total += weight[p];
+      }
+      const float inv_w = 1.0f / total;
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p) {
+#pragma unroll
+        for (int it = 0; it < 4; ++it) *reinterpret_cast<u32x4*>(stage + (4 * it + sub) * kStageRow + piece * 16) = slice[p][it];
+        const float c = weight[p] * inv_w;
+#pragma unroll
+        for (int n = 0; n < kDvPerWave; ++n) {
+          const u32x2 packed = *reinterpret_cast<const u32x2*>(stage + i16 * kStageRow + (16 * n + 4 * g) * 2);
+          const float values[4] = {__builtin_bit_cast(float, packed.x << 16), __builtin_bit_cast(float, packed.x & 0xffff0000u),
+                                   __builtin_bit_cast(float, packed.y << 16), __builtin_bit_cast(float, packed.y & 0xffff0000u)};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) o[n][j] = p == 0 ? values[j] * c : o[n][j] + values[j] * c;
         }
       }
-      lse2 = top + __builtin_amdgcn_logf(w_mine + w_theirs);
+      lse2 = top + __builtin_amdgcn_logf(total);
     }
     if (hw == 0 && g == 0 && a.lse != nullptr) a.lse[seq * a.heads + head] = lse2 * 0.6931471805599453f;
     rows_of_o(v);
@@ -2153,14 +2168,14 @@ hipError_t PrepareDecode() {
   return hipFuncSetAttribute(reinterpret_cast<const void*>(&MlaDecodeKernel<FP8, ALIGNED, MXQ, SPARSE>),
                              hipFuncAttributeMaxDynamicSharedMemorySize, Geom<FP8>::kLdsBytes);
 }
-template <bool HALVES, bool FP8>
+template <int PARTS, bool FP8>
 hipError_t PrepareHeadBlock() {
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(&MlaSelectedHeadBlockKernel<HALVES, FP8>),
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&MlaSelectedHeadBlockKernel<PARTS, FP8>),
                              hipFuncAttributeMaxDynamicSharedMemorySize, GeomHeadBlock<FP8>::kLdsBytes);
 }
-template <bool HALVES, bool FP8>
+template <int PARTS, bool FP8>
 hipError_t LaunchHeadBlock(const AttnArgs& args, const dim3& units, hipStream_t stream) {
-  hipLaunchKernelGGL((MlaSelectedHeadBlockKernel<HALVES, FP8>), units, dim3(kHbThreads), GeomHeadBlock<FP8>::kLdsBytes, stream, args);
+  hipLaunchKernelGGL((MlaSelectedHeadBlockKernel<PARTS, FP8>), units, dim3(kHbThreads), GeomHeadBlock<FP8>::kLdsBytes, stream, args);
   return hipGetLastError();
 }
 template <bool MXQ, bool SPARSE>
@@ -2228,7 +2243,8 @@ hipError_t PrepareAttnKernels() {
       PrepareDecode<true, true, true, false>(),   PrepareDecode<true, false, true, false>(),
       PrepareDecode<false, false, false, true>(), PrepareDecode<true, false, false, true>(),
       PrepareMerge<false, false>(), PrepareMerge<true, false>(), PrepareMerge<false, true>(),
-      PrepareHeadBlock<false, false>(), PrepareHeadBlock<true, false>(), PrepareHeadBlock<false, true>(), PrepareHeadBlock<true, true>()};
+      PrepareHeadBlock<1, false>(), PrepareHeadBlock<2, false>(), PrepareHeadBlock<4, false>(),
+      PrepareHeadBlock<1, true>(), PrepareHeadBlock<2, true>(), PrepareHeadBlock<4, true>()};
   for (const hipError_t e : results) {
     if (e != hipSuccess) return e;
   }
@@ -2269,21 +2285,24 @@ bool AnySequenceSplit(const AttnArgs& a) {
   return false;
 }
 
-// Whole-selection units of 16 heads, one workgroup per unit or two (head_block_units 1 / 2).
+// Whole-selection units of 16 heads, taken by one, two or four workgroups each (head_block_units).
 static hipError_t LaunchHeadBlockUnits(AttnArgs& args, hipStream_t stream) {
   const int sequences_per_xcd = (args.batch + kXcds - 1) / kXcds;
   const int64_t pairs = static_cast<int64_t>(args.batch) * (args.heads / 16);
-  // Two workgroups per unit meet on four words each of this launch's counters and leave their
-  // partials in the first 2 x 16 x pairs rows of the workspace, the LSEs behind them (the plan
-  // sizes the workspace for that).
-  const bool halves = args.head_block_units == 2 && pairs * 4 <= kAttnSyncSequences * 2 && args.partial_out != nullptr;
-  if (halves) {
+  // The workgroups of a unit meet on four words each of this launch's counters and leave their
+  // partials in the first parts x 16 x pairs rows of the workspace, the LSEs behind them (the caller
+  // has checked that the workspace holds them).
+  const bool together = args.head_block_units > 1 && pairs * 4 <= kAttnSyncSequences * 2 && args.partial_out != nullptr;
+  const int parts = together ? args.head_block_units : 1;
+  if (together) {
     if (hipError_t sync_error = SyncRegion(&args.sync); sync_error != hipSuccess) return sync_error;
-    const dim3 units(kXcds * (args.heads / 16) * 2 * sequences_per_xcd);
-    return args.fp8 ? LaunchHeadBlock<true, true>(args, units, stream) : LaunchHeadBlock<true, false>(args, units, stream);
   }
-  const dim3 units(kXcds * (args.heads / 16) * sequences_per_xcd);
-  return args.fp8 ? LaunchHeadBlock<false, true>(args, units, stream) : LaunchHeadBlock<false, false>(args, units, stream);
+  const dim3 units(kXcds * (args.heads / 16) * parts * sequences_per_xcd);
+  switch (parts) {
+    case 4: return args.fp8 ? LaunchHeadBlock<4, true>(args, units, stream) : LaunchHeadBlock<4, false>(args, units, stream);
+    case 2: return args.fp8 ? LaunchHeadBlock<2, true>(args, units, stream) : LaunchHeadBlock<2, false>(args, units, stream);
+    default: return args.fp8 ? LaunchHeadBlock<1, true>(args, units, stream) : LaunchHeadBlock<1, false>(args, units, stream);
+  }
 }
 
 hipError_t LaunchAttnDecode(const AttnArgs& args_in, hipStream_t stream) {

@@ -202,10 +202,11 @@ mlakvStatus mlakvAttnPlanInit(int32_t batch, int32_t heads, int32_t max_seq_len,
  *   unit; units that hold part of a selection leave partials that a merge puts together.
  * HEAD_BLOCK: one unit = the whole selection of one sequence for 16 heads; nothing to merge and the
  *   workspace stays untouched. sparse_count up to MLAKV_ATTN_HEAD_BLOCK_TOKENS.
- * HEAD_BLOCK_HALVES: the same unit taken by two workgroups, half of the selection's tiles each; each
+ * HEAD_BLOCK_HALVES: the same unit shared by two workgroups, half of the selection's tiles each (or by
+ *   four, a quarter each, above 256 selected tokens while four per unit fit the CUs once); each
  *   leaves a partial (16 rows) in the workspace and counts itself on a word of the library's
  *   counters (those of MLAKV_ATTN_MERGE_IN_LAUNCH, with their limit on launches in flight); the
- *   second to finish combines the two inside the launch, nobody waits. Up to 2048 (sequence, 16
+ *   last to finish combines them inside the launch, nobody waits. Up to 2048 (sequence, 16
  *   heads) pairs.
  * AUTO, unless chunk_tiles, work_groups or merge_mode ask for properties of the split, takes what
  * was measured ahead. bf16 caches: HEAD_BLOCK_HALVES from 257 to 768 selected tokens while two
@@ -218,7 +219,8 @@ mlakvStatus mlakvAttnPlanInit(int32_t batch, int32_t heads, int32_t max_seq_len,
  * contexts: a unit then takes every position of its sequence. AUTO decides at every launch from
  * the longest context the launch can see -- the lengths themselves with mlakvAttnDecodeHostLens,
  * the plan's max_seq_len with lengths in device memory: while two workgroups per unit fit the CUs
- * once, HEAD_BLOCK up to 256 tokens and HEAD_BLOCK_HALVES up to 768; while one per unit fits,
+ * once, HEAD_BLOCK up to 256 tokens and HEAD_BLOCK_HALVES (with four workgroups per unit while those
+ * fit) up to 768; while one per unit fits,
  * HEAD_BLOCK up to 512; while they fit twice, up to 256; the 64-head kernel otherwise and whenever
  * chunk_tiles, work_groups or merge_mode ask for properties of the split. SPLIT keeps the 64-head
  * kernel always; HEAD_BLOCK and HEAD_BLOCK_HALVES ask for the units (max_seq_len up to

@@ -54,3 +54,20 @@ def test_merge_with_several_waves_per_head(ctxs, heads, fp8):
     # units of one tile as well: more partials than one round of the waves takes
     for options in ({"selection_units": 1}, {"chunk_tiles": 1}):
         _check(cache, table, ctxs, heads, seed=905, fp8=fp8, **options)
+
+
+# Units of 16 heads shared by four workgroups (whole contexts and selections of 257 tokens and more while four
+# per unit fit the 256 CUs): fewer tiles than workgroups, shares of different sizes, the last batch
+# that fits (16 x 64 heads) and the first that is shared by two (17).
+@pytest.mark.parametrize("ctxs,heads,fp8", [([768, 1, 0, 32, 33, 65, 96, 97, 129, 300], 64, True), ([257, 600, 40], 128, False),
+                                            ([400, 31, 700], 16, True), ([320 + 7 * i for i in range(16)], 64, False),
+                                            ([280] * 17, 64, False)])
+def test_units_shared_by_four_workgroups(ctxs, heads, fp8):
+    cache, table = _cache(ctxs, 64, seed=911, fp8=fp8)
+    _check(cache, table, ctxs, heads, seed=915, fp8=fp8)
+    rng = np.random.default_rng(917)
+    for k in (257, 704):
+        sparse = np.full((len(ctxs), k), -1, dtype=np.int32)
+        for s, n in enumerate(ctxs):
+            sparse[s, :min(n, k)] = rng.permutation(n)[:k]
+        _check(cache, table, ctxs, heads, seed=919, fp8=fp8, sparse=sparse)
