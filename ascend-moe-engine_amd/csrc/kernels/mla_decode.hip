@@ -1017,24 +1017,49 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
           const int context = static_cast<int>(
               min(static_cast<int64_t>(max(Uniform(LiveLength(a, seq)), 0)), static_cast<int64_t>(a.table_stride) * a.block_size));
           const int32_t* selection = a.sparse_indices + static_cast<int64_t>(seq) * a.sparse_seq_stride;
+          // All loads of a step go out together: the segment's own entries, then the whole list for its
+          // end, then (once the first have arrived) the block-table entries of the own ones, which do
+          // not wait for where the list ends. One load and its wait at a time this was up to seven
+          // memory trips in front of the first tile (2048 selected tokens of 9 FP8 sequences: 20.2 -> 19.9 us).
+          constexpr int kOwn = kTableEntries / kThreads, kList = kAttnSelectionMax / kThreads;
+          const int32_t* table_row = a.block_table + static_cast<int64_t>(seq) * a.table_stride;
+          int own[kOwn], listed[kList];
+  #pragma unroll
+          for (int j = 0; j < kOwn; ++j) {
+            const int i = tid + kThreads * j;
+            own[j] = i < segment_tiles * kTileTokens && map.first_pos + i < a.sparse_count ? selection[map.first_pos + i] : -1;
+          }
+  #pragma unroll
+          for (int j = 0; j < kList; ++j) {
+            const int i = tid + kThreads * j;
+            listed[j] = i < a.sparse_count ? selection[i] : 0;
+          }
           if (tid == 0) scalar_lds[0] = a.sparse_count;
+          int packed[kOwn];
+  #pragma unroll
+          for (int j = 0; j < kOwn; ++j) {
+            packed[j] = -1;
+            if (own[j] >= 0 && own[j] < context) {
+              const int logical = own[j] / a.block_size;
+              const int entry = table_row[logical];
+              if (static_cast<unsigned>(entry) < static_cast<unsigned>(a.num_blocks)) {
+                packed[j] = (entry << map.slot_bits) | (own[j] - logical * a.block_size);
+              }
+            }
+          }
           __syncthreads();
-          for (int i = tid; i < a.sparse_count; i += kThreads) {
-            const int index = selection[i];
-            if (index < 0 || index >= context) atomicMin(scalar_lds, i);
+  #pragma unroll
+          for (int j = 0; j < kList; ++j) {
+            const int i = tid + kThreads * j;
+            if (i < a.sparse_count && (listed[j] < 0 || listed[j] >= context)) atomicMin(scalar_lds, i);
+          }
+  #pragma unroll
+          for (int j = 0; j < kOwn; ++j) {
+            const int i = tid + kThreads * j;
+            if (i < segment_tiles * kTileTokens) table_lds[i] = packed[j];  // <= kTableEntries, ensured by the plan's cap
           }
           __syncthreads();
           seq_len = Uniform(scalar_lds[0]);
-          const int32_t* table_row = a.block_table + static_cast<int64_t>(seq) * a.table_stride;
-          const int segment_tokens = min(segment_tiles * kTileTokens, seq_len - map.first_pos);  // <= kTableEntries, ensured by the plan's cap
-          for (int i = tid; i < segment_tokens; i += kThreads) {
-            const int index = selection[map.first_pos + i];  // inside [0, context): before the end of the selection
-            const int logical = index / a.block_size;
-            const int entry = table_row[logical];
-            table_lds[i] = static_cast<unsigned>(entry) < static_cast<unsigned>(a.num_blocks)
-                               ? (entry << map.slot_bits) | (index - logical * a.block_size)
-                               : -1;
-          }
         }
         map.seq_len = seq_len;
         const int num_tiles = (seq_len + kTileTokens - 1) / kTileTokens;
@@ -2318,7 +2343,7 @@ hipError_t LaunchAttnDecode(const AttnArgs& args_in, hipStream_t stream) {
   const bool sparse = args.sparse_indices != nullptr;
   hipError_t e;
   if (sparse) {
-    if (quantise) return hipErrorInvalidValue;
+    if (quantise || args.sparse_count > kAttnSelectionMax) return hipErrorInvalidValue;
     // a selected token is staged as (block << ceil(log2(block_size))) | slot in 31 bits
     int slot_bits = 0;
     while ((int64_t{1} << slot_bits) < args.block_size) ++slot_bits;
