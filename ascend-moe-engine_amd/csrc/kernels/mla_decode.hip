@@ -677,7 +677,9 @@ struct MergeState {
 // loads: 0.3 to 0.5 us less per launch).
 // AGENT: the partials were written by other CUs of this launch (agent-scope loads); otherwise by
 // an earlier launch (plain streaming loads).
-template <bool AGENT>
+// SHARED: other waves hold partials of the same head. A wave whose partials are all NaN then says so
+// with its denominator: beside finite partials of the others the row is NaN.
+template <bool AGENT, bool SHARED>
 __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_in_group, int first_slot, int u0, int first, int step,
                                              int n, int lane, MergeState& s) {
 #pragma unroll
@@ -703,7 +705,15 @@ __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_
     float group_max = s.m;
 #pragma unroll
     for (int u = 0; u < 8; ++u) group_max = fmaxf(group_max, l[u]);
-    if (group_max == -__builtin_inff()) continue;  // nothing but empty partials so far
+    if (group_max == -__builtin_inff()) {  // nothing but empty partials so far, or NaN ones, which no maximum shows
+      if constexpr (SHARED) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if (l[u] != l[u]) s.denom = l[u];
+        }
+      }
+      continue;
+    }
     const float rescale = __builtin_amdgcn_exp2f(s.m - group_max);  // 0 on the first group
     s.m = group_max;
     s.denom *= rescale;
@@ -886,7 +896,7 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
           const int h = u * kMergeHeads + wave0;
           if (h < heads_here) {
             MergeState state;
-            TakePartials<true>(a, z, h, a.max_units + seq, u0, 0, 1, n, lane0, state);
+            TakePartials<true, false>(a, z, h, a.max_units + seq, u0, 0, 1, n, lane0, state);
             FinishHead<MXQ>(a, z, seq, h, lane0, state);
           }
         }
@@ -1566,7 +1576,7 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
   const int partials = (seq_end - 1) / cut.tiles_per_unit - first_unit + 1;
   if (partials == 1) return;  // written by the workgroup that held the whole sequence
   MergeState state;
-  if (has_head) TakePartials<false>(a, z, h, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
+  if (has_head) TakePartials<false, (WAYS > 1)>(a, z, h, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
   if constexpr (WAYS > 1) {
     if (way != 0 && has_head) {
 #pragma unroll
@@ -1594,6 +1604,8 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) state.acc[j] += weight * shared_acc[wave + w][j][lane];
       }
+    } else {
+      state.denom = 0.0f;  // no finite partial at all: zeros, as from one wave
     }
   }
   FinishHead<MXQ>(a, z, seq, h, lane, state);

@@ -71,3 +71,20 @@ def test_units_shared_by_four_workgroups(ctxs, heads, fp8):
         for s, n in enumerate(ctxs):
             sparse[s, :min(n, k)] = rng.permutation(n)[:k]
         _check(cache, table, ctxs, heads, seed=919, fp8=fp8, sparse=sparse)
+
+
+# A row of NaN spoils every head of its sequence, also where the merge's waves take one partial each
+# and the one that holds it holds nothing else (three partials of the short sequence, eight waves).
+# No tolerance: NaN everywhere in that sequence, the other sequence as without it.
+@pytest.mark.parametrize("ctxs", [[32000, 300], [9000, 900] + [9000] * 10])
+def test_merge_keeps_a_nan(ctxs):
+    cache, table = _cache(ctxs, 64, seed=921)
+    q = kt.randn_bf16((len(ctxs), 64, LATENT + ROPE), seed=925).cuda()
+    arguments = (q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE)
+    clean = kt.attention(cache, 0, *arguments, selection_units=1)[0]
+    block, slot = int(table[1, 0]), 10
+    cache.latent[0, block, slot, :] = float("nan")
+    out, lse, _ = kt.attention(cache, 0, *arguments, selection_units=1)
+    others = [s for s in range(len(ctxs)) if s != 1]
+    assert kt.torch.isnan(out[1].float()).all() and kt.torch.isnan(lse[1]).all()
+    assert kt.torch.equal(out[others], clean[others])
