@@ -273,11 +273,9 @@ __global__ __launch_bounds__(kScoreThreads) void IndexerScoreKernel(IndexerArgs 
   if (token < seq_len) a.keys[seq * a.keys_stride + token] = static_cast<unsigned short>(ScoreKey(mine * my_scale));
 }
 
-constexpr int kSelectThreads = 1024;
-constexpr int kSelectWaves = kSelectThreads / 64;
-constexpr int kHeldPieces = 4;                                   // 16-byte pieces (eight keys) a thread keeps in registers
-constexpr int kKeysPerPiece = kSelectThreads * 8;                // 8192
-constexpr int kHistogramCopies = 32;
+constexpr int kHeldPieces = 4;  // 16-byte pieces (eight keys) a thread keeps in registers
+constexpr int kSelectThreads = 1024, kSelectCopies = 32;  // long contexts
+constexpr int kShortThreads = 512, kShortCopies = 8, kShortKeys = 8192;  // contexts up to 8192 tokens
 typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 
 // Inclusive prefix sum over the 64 lanes with data-parallel-primitive moves (no LDS crossbar, no
@@ -294,17 +292,24 @@ __device__ __forceinline__ int WaveInclusiveScan(int v) {
 }
 
 // Adds up the copies of the histogram and finds the byte value that holds the `wanted`-th largest
-// entry and the number of entries above it. Thread t owns counters 8 t .. 8 t + 7, a quarter of bin
-// t / 4, and leaves them cleared; behind the barrier every wavefront looks for the bin itself (four
+// entry and the number of entries above it. Each thread owns the copies of a bin, or an equal share
+// of them, and leaves them cleared; behind the barrier every wavefront looks for the bin itself (four
 // bins per lane, a prefix sum over the lanes), so the answer needs no second one.
+template <int THREADS, int COPIES>
 __device__ __forceinline__ void FindBin(int* counters, int* totals, int wanted, int tid, int* bin, int* entries_above) {
-  u32x4* own = reinterpret_cast<u32x4*>(counters + 8 * tid);
-  const u32x4 lo = own[0], hi = own[1];
-  own[0] = own[1] = u32x4{0u, 0u, 0u, 0u};
-  int sum = static_cast<int>(((lo.x + lo.y) + (lo.z + lo.w)) + ((hi.x + hi.y) + (hi.z + hi.w)));
-  sum += __builtin_amdgcn_update_dpp(0, sum, 0xb1, 0xf, 0xf, false);  // quad_perm:[1,0,3,2]
-  sum += __builtin_amdgcn_update_dpp(0, sum, 0x4e, 0xf, 0xf, false);  // quad_perm:[2,3,0,1]
-  if ((tid & 3) == 0) totals[tid >> 2] = sum;
+  constexpr int kPerBin = THREADS / 256, kOwn = COPIES / kPerBin / 4;  // threads of a bin, 16-byte groups of counters of a thread
+  static_assert(kPerBin == 1 || kPerBin == 2 || kPerBin == 4, "a quad of lanes at most adds up a bin");
+  u32x4* own = reinterpret_cast<u32x4*>(counters) + kOwn * tid;
+  u32x4 counted = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int i = 0; i < kOwn; ++i) {
+    counted += own[i];
+    own[i] = u32x4{0u, 0u, 0u, 0u};
+  }
+  int sum = static_cast<int>((counted.x + counted.y) + (counted.z + counted.w));
+  if constexpr (kPerBin > 1) sum += __builtin_amdgcn_update_dpp(0, sum, 0xb1, 0xf, 0xf, false);  // quad_perm:[1,0,3,2]
+  if constexpr (kPerBin > 2) sum += __builtin_amdgcn_update_dpp(0, sum, 0x4e, 0xf, 0xf, false);  // quad_perm:[2,3,0,1]
+  if (tid % kPerBin == 0) totals[tid / kPerBin] = sum;
   __syncthreads();
   const int lane = tid & 63;
   const u32x4 four = *reinterpret_cast<const u32x4*>(totals + 4 * lane);
@@ -330,25 +335,31 @@ __device__ __forceinline__ void FindBin(int* counters, int* totals, int wanted, 
 // One workgroup per sequence. The k-th largest key is found by its high and then its low byte (two
 // 256-bin histograms); then an ordered compaction writes the positions above it and the first ones
 // equal to it. Thread t holds `pieces` consecutive groups of eight keys, as many as the sequence
-// needs for all threads together (1 up to 8192 keys, 4 up to 32768), so thread order is position
-// order and the keys are read once; longer sequences go in sweeps of 32768 that are read again, from
-// the L2, for each of the three steps.
+// needs for all threads together (with 1024 threads 1 up to 8192 keys, 4 up to 32768), so thread order
+// is position order and the keys are read once; longer sequences go in sweeps of 32768 that are read
+// again, from the L2, for each of the three steps.
 // What bounds it is one CU's time for a sequence: the chain of its steps and the counting. Scores
 // crowd into a few exponents, so one histogram is a handful of hot counters: with 32 copies, lane L
 // counting in copy L % 32, the 64 lanes of an addition meet at most in pairs and never in a bank.
+// Up to 8192 keys the copies cost more than the counters they relieve, and half of the threads is
+// enough. Index key append, indexer and attention (16 heads) of a layer, 32 sequences, 1024 threads with 32 copies /
+// with 8 copies / 512 with 8 / 256 with 8, us: 500 tokens 22.5 / 22.0 / 20.7 / 20.5; 2000: 24.4 / 24.1 / 22.6 /
+// 22.3; 4000: 26.8 / 26.3 / 25.1 / 25.5; 8192: 27.8 / 27.7 / 26.8 / -.
 // Measured, top 512 of 8192 keys (32 sequences) and top 2048 of up to 32768 (9 sequences):
 // 5.8 -> 5.7 us and 18.7 -> 10.3 us against one histogram and passes of 8192 keys that re-read the later
 // ones in every step. (A separate path without the per-key end tests measured the same.)
-__global__ __launch_bounds__(kSelectThreads) void IndexerSelectKernel(IndexerArgs a) {
-  __shared__ __attribute__((aligned(16))) int counters[256 * kHistogramCopies];  // copy c of bin b at 32 b + c
+template <int THREADS, int COPIES>
+__global__ __launch_bounds__(THREADS) void IndexerSelectKernel(IndexerArgs a) {
+  constexpr int kWaves = THREADS / 64, kKeysPerPiece = THREADS * 8;
+  __shared__ __attribute__((aligned(16))) int counters[256 * COPIES];  // copy c of bin b at COPIES b + c
   __shared__ __attribute__((aligned(16))) int totals[2][256];  // one per byte, so that no barrier separates the rounds
-  __shared__ unsigned wave_counts[kSelectWaves];
+  __shared__ unsigned wave_counts[kWaves];
   const int seq = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = max(min(a.seq_lens[seq], a.max_seq_len), 0);
   const int k = a.sparse_count;
   int32_t* out = a.indices_out + seq * a.indices_seq_stride;
   if (n <= k) {
-    for (int i = tid; i < k; i += kSelectThreads) out[i] = i < n ? i : -1;
+    for (int i = tid; i < k; i += THREADS) out[i] = i < n ? i : -1;
     return;
   }
   const unsigned short* keys = a.keys + seq * a.keys_stride;
@@ -368,12 +379,13 @@ __global__ __launch_bounds__(kSelectThreads) void IndexerSelectKernel(IndexerArg
   };
   int first = load(0);
   {
-    u32x4* own = reinterpret_cast<u32x4*>(counters + 8 * tid);
-    own[0] = own[1] = u32x4{0u, 0u, 0u, 0u};
+    u32x4* all = reinterpret_cast<u32x4*>(counters);
+#pragma unroll
+    for (int i = tid; i < 64 * COPIES; i += THREADS) all[i] = u32x4{0u, 0u, 0u, 0u};
   }
   __syncthreads();
 
-  int* const copy = counters + (lane & (kHistogramCopies - 1));
+  int* const copy = counters + (lane & (COPIES - 1));
   int high = 0, low = 0, above_high = 0, above_low = 0;
   for (int sweep = 0; sweep < sweeps; ++sweep) {
     if (sweep > 0) first = load(sweep);
@@ -383,12 +395,12 @@ __global__ __launch_bounds__(kSelectThreads) void IndexerSelectKernel(IndexerArg
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const unsigned byte = (held[p][i >> 1] >> (i & 1 ? 24 : 8)) & 255u;
-        if (first + 8 * p + i < n) atomicAdd(copy + byte * kHistogramCopies, 1);
+        if (first + 8 * p + i < n) atomicAdd(copy + byte * COPIES, 1);
       }
     }
   }
   __syncthreads();
-  FindBin(counters, totals[0], k, tid, &high, &above_high);
+  FindBin<THREADS, COPIES>(counters, totals[0], k, tid, &high, &above_high);
   if (sweeps > 1) first = load(0);
   for (int sweep = 0; sweep < sweeps; ++sweep) {
     if (sweep > 0) first = load(sweep);
@@ -398,12 +410,12 @@ __global__ __launch_bounds__(kSelectThreads) void IndexerSelectKernel(IndexerArg
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const unsigned key = (held[p][i >> 1] >> (i & 1 ? 16 : 0)) & 0xffffu;
-        if ((key >> 8) == static_cast<unsigned>(high) && first + 8 * p + i < n) atomicAdd(copy + (key & 255u) * kHistogramCopies, 1);
+        if ((key >> 8) == static_cast<unsigned>(high) && first + 8 * p + i < n) atomicAdd(copy + (key & 255u) * COPIES, 1);
       }
     }
   }
   __syncthreads();
-  FindBin(counters, totals[1], k - above_high, tid, &low, &above_low);
+  FindBin<THREADS, COPIES>(counters, totals[1], k - above_high, tid, &low, &above_low);
   const unsigned short threshold = static_cast<unsigned short>((high << 8) | low);
   const int greater_total = above_high + above_low, equal_wanted = k - greater_total;
 
@@ -440,7 +452,7 @@ __global__ __launch_bounds__(kSelectThreads) void IndexerSelectKernel(IndexerArg
     __syncthreads();
     unsigned before = inclusive - packed, all = 0u;
 #pragma unroll
-    for (int v = 0; v < kSelectWaves; ++v) {
+    for (int v = 0; v < kWaves; ++v) {
       const unsigned c = wave_counts[v];
       if (v < wave) before += c;
       all += c;
@@ -529,7 +541,8 @@ hipError_t PrepareIndexerKernels() {
   for (const hipError_t e : results) {
     if (e != hipSuccess) return e;
   }
-  for (const void* kernel : {reinterpret_cast<const void*>(&IndexerSelectKernel), reinterpret_cast<const void*>(&IndexKeyAppendKernel)}) {
+  for (const void* kernel : {reinterpret_cast<const void*>(&IndexerSelectKernel<kShortThreads, kShortCopies>), reinterpret_cast<const void*>(&IndexerSelectKernel<kSelectThreads, kSelectCopies>),
+                             reinterpret_cast<const void*>(&IndexKeyAppendKernel)}) {
     hipFuncAttributes attributes;
     if (hipError_t e = hipFuncGetAttributes(&attributes, kernel); e != hipSuccess) return e;
   }
@@ -559,7 +572,11 @@ hipError_t LaunchIndexer(const IndexerArgs& args, hipStream_t stream) {
     }
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(IndexerSelectKernel, dim3(args.batch), dim3(kSelectThreads), 0, stream, args);
+  if (args.max_seq_len <= kShortKeys) {
+    hipLaunchKernelGGL((IndexerSelectKernel<kShortThreads, kShortCopies>), dim3(args.batch), dim3(kShortThreads), 0, stream, args);
+  } else {
+    hipLaunchKernelGGL((IndexerSelectKernel<kSelectThreads, kSelectCopies>), dim3(args.batch), dim3(kSelectThreads), 0, stream, args);
+  }
   return hipGetLastError();
 }
 
