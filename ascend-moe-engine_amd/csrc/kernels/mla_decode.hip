@@ -2149,7 +2149,7 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
       if (lane == 0) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       // Whichever part arrives last, the result is the same: every partial enters as the bf16 rows
       // that were stored, in the order of the parts (this wave's own among them, read back as well;
-      // a part that does not exist repeats the last one with weight 0).
+      // a part that does not exist repeats the last one and is not added).
       float lses2[PARTS], top = lse2;
       u32x4 slice[PARTS][4];
 #pragma unroll
@@ -2173,6 +2173,7 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
       const float inv_w = 1.0f / total;
 #pragma unroll
       for (int p = 0; p < PARTS; ++p) {
+        if (p >= parts) break;  // no such part: its weight is 0, but 0 x infinity would be NaN
 #pragma unroll
         for (int it = 0; it < 4; ++it) *reinterpret_cast<u32x4*>(stage + (4 * it + sub) * kStageRow + piece * 16) = slice[p][it];
         const float c = weight[p] * inv_w;

@@ -88,3 +88,20 @@ def test_merge_keeps_a_nan(ctxs):
     others = [s for s in range(len(ctxs)) if s != 1]
     assert kt.torch.isnan(out[1].float()).all() and kt.torch.isnan(lse[1]).all()
     assert kt.torch.equal(out[others], clean[others])
+
+
+# A launch of four workgroups per unit holds sequences of two and three tiles too, whose last workgroups do not
+# exist. With q = 0 every row has the same weight, and 32 rows of 3e38 add up to an infinity in fp32:
+# infinite in the output whatever the number of workgroups, never 0 x infinity.
+@pytest.mark.parametrize("tokens", [64, 96])
+def test_workgroups_without_a_tile_leave_infinities_alone(tokens):
+    ctxs = [300, tokens]
+    cache, table = _cache(ctxs, 64, seed=931)
+    last = (tokens - 32) // 64, (tokens - 32) % 64
+    cache.latent[0, int(table[1, last[0]]), last[1]:last[1] + 32, 7] = 3e38
+    q = kt.torch.zeros(2, 64, LATENT + ROPE, dtype=kt.torch.bfloat16, device="cuda")
+    for options in ({}, {"selection_units": kt.ffi.ATTN_UNITS_HEAD_BLOCK_HALVES}):
+        out, lse, _ = kt.attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE, **options)
+        assert kt.torch.isposinf(out[1, :, 7].float()).all(), options
+        rest = [c for c in range(LATENT) if c != 7]
+        assert kt.torch.isfinite(out[1][:, rest].float()).all() and kt.torch.isfinite(lse).all()
