@@ -344,10 +344,10 @@ int64_t CapUnitTiles(int32_t block_size, bool sparse) {
   return cap < 1 ? 1 : cap;
 }
 
-// What the workgroups that share a unit of 16 heads leave in the workspace: `parts` partials of 16
-// rows per (sequence, 16 heads) and, behind the rows of all of them, their LSEs (4 x 16 floats each).
+// What the workgroups that share a unit of 16 heads leave in the workspace: `parts` partials per
+// (sequence, 16 heads) and, behind all of them, their LSEs (4 x 16 floats each).
 uint64_t HeadBlockPartialBytes(int32_t batch, int32_t heads, int32_t parts) {
-  return static_cast<uint64_t>(batch) * (heads / 16) * parts * (16 * mlakv::kLatentDim * 2 + 4 * 16 * sizeof(float));
+  return static_cast<uint64_t>(batch) * (heads / 16) * parts * (mlakv::HeadBlockPartBytes(parts) + 4 * 16 * sizeof(float));
 }
 
 struct PlanShape {

@@ -176,6 +176,9 @@ constexpr int kRopeDim = 64;
 constexpr int kTileTokens = 32;
 constexpr int kAttnSelectionMax = 2048;    // selected tokens of a sequence, at most
 constexpr int kAttnTableEntries = 512;     // block-table entries (or selected tokens) of one segment staged in LDS
+// What one of the workgroups that share a unit of 16 heads leaves in the workspace besides its LSEs: two parts
+// 16 bf16 rows each, four parts the fp32 accumulators.
+constexpr int HeadBlockPartBytes(int parts) { return 16 * kLatentDim * (parts > 2 ? 4 : 2); }
 constexpr int kAttnBoundaryTiles = 4;      // what entering a sequence inside a work unit costs, in tiles (see MakeCut)
 constexpr int kAttnSyncSequences = 4096;   // (head group, sequence) pairs a launch can merge in place
 constexpr int kAttnHeadBlockTokens = 1024; // selected tokens a whole-sequence unit of 16 heads stages in LDS

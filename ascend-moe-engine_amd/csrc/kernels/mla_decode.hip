@@ -635,6 +635,7 @@ __device__ __forceinline__ void WaitAgentLoads(u32x4 (&v)[8]) {
                :
                : "memory");
 }
+constexpr int kAgentScope = 16;  // sc1, as a buffer load's cache policy
 __device__ __forceinline__ void StoreAgentF32(float* p, float v) {
   __hip_atomic_store(reinterpret_cast<unsigned*>(p), __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1654,9 +1655,9 @@ hipError_t LaunchMerge(const AttnArgs& args, int head_groups, hipStream_t stream
 // PARTS: two or four workgroups per (sequence, 16 heads), neighbours on one XCD, each with an equal
 // share of the selection's tiles, so that more CUs (and more rows in flight) work on a launch that
 // has fewer units than the chip has CUs. The exchange is a matter between the output waves that hold
-// the same 128 columns, one in each workgroup: each leaves its normalised slice (bf16 rows and a
-// log2-domain LSE per head, agent-scope stores) in the workspace and counts itself on the word of
-// (unit, slice); the one that finds every other count there reads the slices back, combines them and
+// the same 128 columns, one in each workgroup: each leaves its normalised slice (bf16 rows with two
+// parts, fp32 accumulators with four, and a log2-domain LSE per head, agent-scope stores) in the
+// workspace and counts itself on the word of (unit, slice); the one that finds every other count there reads the slices back, combines them and
 // writes the output. Nobody waits, no barrier is involved: those that arrive earlier leave. The words
 // are zero between launches (the last to arrive clears its word). A selection of fewer tiles than
 // parts is taken by the first of them, one tile each.
@@ -2130,16 +2131,29 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
     };
     u32x4 v[4];
     if (shared) {
-      // This part's partial at (unit, part) of the workspace: 16 rows of 1 KB, and behind the rows
-      // of all units the 16 LSEs once per slice, so that each wave's count covers what its partners read.
+      // This part's partial in the workspace: its slice at (unit, part), and behind the slices of all
+      // units the 16 LSEs once per slice, so that each wave's count covers what its partners read.
+      constexpr int kPartBytes = HeadBlockPartBytes(PARTS);
       const int pair = seq * head_blocks + hb;
-      const int64_t unit_row0 = static_cast<int64_t>(pair) * (PARTS * 16);
-      float* lses = reinterpret_cast<float*>(a.partial_out + static_cast<int64_t>(a.batch) * head_blocks * (PARTS * 16) * (kLatentDim * 2)) +
-                    unit_row0 * 4 + 16 * hw + i16;                                      // + part * 64
-      char* slices = a.partial_out + unit_row0 * (kLatentDim * 2) + kSliceBytes * hw + piece * 16;  // + (16 part + row) KB
-      rows_of_o(v);
+      char* unit_parts = a.partial_out + static_cast<int64_t>(pair) * (PARTS * kPartBytes);
+      float* lses = reinterpret_cast<float*>(a.partial_out + static_cast<int64_t>(a.batch) * head_blocks * (PARTS * kPartBytes)) +
+                    static_cast<int64_t>(pair) * (PARTS * 64) + 16 * hw + i16;  // + part * 64
+      // Two parts: 16 rows of bf16, a slice = 256 bytes of each.
+      char* slices = unit_parts + kSliceBytes * hw + piece * 16;  // + (16 part + row) KB
+      // Four: the accumulators as they are, a slice = 8 KB, 16 bytes per lane and column tile. Slices of bf16
+      // cost precision where the parts' weights differ (rows that grow by 40 x along 257 to 768 tokens:
+      // 2.26e-3 against float64, two parts 2.06e-3); these give 1.74e-3 (one workgroup 1.79e-3) and the same
+      // time: twice the bytes, but no way through the staging rows. 8 x 64 heads, 512 tokens: 11.6 us
+      // with slices of bf16, 11.7 so; 768: 13.0 / 13.1.
+      char* tiles = unit_parts + hw * (kPartBytes / kScoreWaves) + lane * 16;  // + part * kPartBytes + n KB
+      if constexpr (PARTS == 2) {
+        rows_of_o(v);
 #pragma unroll
-      for (int it = 0; it < 4; ++it) StoreAgent16(slices + (16 * part + 4 * it + sub) * (kLatentDim * 2), v[it]);
+        for (int it = 0; it < 4; ++it) StoreAgent16(slices + (16 * part + 4 * it + sub) * (kLatentDim * 2), v[it]);
+      } else {
+#pragma unroll
+        for (int n = 0; n < kDvPerWave; ++n) StoreAgent16(tiles + part * kPartBytes + n * 1024, __builtin_bit_cast(u32x4, o[n]));
+      }
       if (g == 0) StoreAgentF32(lses + part * 64, lse2);
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partial stores are complete
       unsigned* word = a.sync + 4 * pair + hw;
@@ -2147,44 +2161,82 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
       if (lane == 0) arrived = __hip_atomic_fetch_add(word, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (Uniform(arrived) != static_cast<unsigned>(parts - 1)) return;  // the last part's wave will find this slice
       if (lane == 0) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      // Whichever part arrives last, the result is the same: every partial enters as the bf16 rows
-      // that were stored, in the order of the parts (this wave's own among them, read back as well;
-      // a part that does not exist repeats the last one and is not added).
-      float lses2[PARTS], top = lse2;
-      u32x4 slice[PARTS][4];
+      asm volatile("" ::: "memory");  // (no load below moves in front of the count)
+      // Whichever part arrives last, the result is the same: every partial enters as it was stored, in
+      // the order of the parts (parts that do not exist are left out).
+      float lses2[PARTS], top = lse2, weight[PARTS], total = 0.0f;
+      const auto weigh = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int p = 0; p < PARTS; ++p) {
-        const int from = min(p, parts - 1);
-        lses2[p] = LoadAgentF32(lses + from * 64);
-#pragma unroll
-        for (int it = 0; it < 4; ++it) slice[p][it] = LoadAgent16(slices + (16 * from + 4 * it + sub) * (kLatentDim * 2));
-      }
-#pragma unroll
-      for (int p = 0; p < PARTS; ++p) {
-        asm volatile("s_waitcnt vmcnt(0)" : "+v"(slice[p][0]), "+v"(slice[p][1]), "+v"(slice[p][2]), "+v"(slice[p][3]) : : "memory");
-        top = fmaxf(top, lses2[p]);
-      }
-      float weight[PARTS], total = 0.0f;
-#pragma unroll
-      for (int p = 0; p < PARTS; ++p) {
-        weight[p] = p < parts ? __builtin_amdgcn_exp2f(lses2[p] - top) : 0.0f;
-        total += weight[p];
-      }
-      const float inv_w = 1.0f / total;
-#pragma unroll
-      for (int p = 0; p < PARTS; ++p) {
-        if (p >= parts) break;  // no such part: its weight is 0, but 0 x infinity would be NaN
-#pragma unroll
-        for (int it = 0; it < 4; ++it) *reinterpret_cast<u32x4*>(stage + (4 * it + sub) * kStageRow + piece * 16) = slice[p][it];
-        const float c = weight[p] * inv_w;
-#pragma unroll
-        for (int n = 0; n < kDvPerWave; ++n) {
-          const u32x2 packed = *reinterpret_cast<const u32x2*>(stage + i16 * kStageRow + (16 * n + 4 * g) * 2);
-          const float values[4] = {__builtin_bit_cast(float, packed.x << 16), __builtin_bit_cast(float, packed.x & 0xffff0000u),
-                                   __builtin_bit_cast(float, packed.y << 16), __builtin_bit_cast(float, packed.y & 0xffff0000u)};
-#pragma unroll
-          for (int j = 0; j < 4; ++j) o[n][j] = p == 0 ? values[j] * c : o[n][j] + values[j] * c;
+        for (int p = 0; p < PARTS; ++p) {
+          if (p < parts) top = fmaxf(top, lses2[p]);
         }
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+          weight[p] = p < parts ? __builtin_amdgcn_exp2f(lses2[p] - top) : 0.0f;
+          total += weight[p];
+        }
+      };
+      if constexpr (PARTS == 2) {
+        u32x4 slice[PARTS][4];
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+          lses2[p] = LoadAgentF32(lses + p * 64);
+#pragma unroll
+          for (int it = 0; it < 4; ++it) slice[p][it] = LoadAgent16(slices + (16 * p + 4 * it + sub) * (kLatentDim * 2));
+        }
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+          asm volatile("s_waitcnt vmcnt(0)" : "+v"(slice[p][0]), "+v"(slice[p][1]), "+v"(slice[p][2]), "+v"(slice[p][3]) : : "memory");
+        }
+        weigh();
+        const float inv_w = 1.0f / total;
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+#pragma unroll
+          for (int it = 0; it < 4; ++it) *reinterpret_cast<u32x4*>(stage + (4 * it + sub) * kStageRow + piece * 16) = slice[p][it];
+          const float c = weight[p] * inv_w;
+#pragma unroll
+          for (int n = 0; n < kDvPerWave; ++n) {
+            const u32x2 packed = *reinterpret_cast<const u32x2*>(stage + i16 * kStageRow + (16 * n + 4 * g) * 2);
+            const float values[4] = {__builtin_bit_cast(float, packed.x << 16), __builtin_bit_cast(float, packed.x & 0xffff0000u),
+                                     __builtin_bit_cast(float, packed.y << 16), __builtin_bit_cast(float, packed.y & 0xffff0000u)};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[n][j] = p == 0 ? values[j] * c : o[n][j] + values[j] * c;
+          }
+        }
+      } else {
+        // (this part's own slice is still in the registers)
+        const __amdgpu_buffer_rsrc_t memory = __builtin_amdgcn_make_buffer_rsrc(unit_parts, 0, PARTS * kPartBytes, 0x00020000);
+        const int at = hw * (kPartBytes / kScoreWaves) + lane * 16;
+        f32x4 theirs[PARTS][kDvPerWave];
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+          lses2[p] = lse2;
+          if (p < parts && p != part) {
+            lses2[p] = LoadAgentF32(lses + p * 64);
+#pragma unroll
+            for (int n = 0; n < kDvPerWave; ++n) {
+              theirs[p][n] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(memory, at + n * 1024, p * kPartBytes, kAgentScope));
+            }
+          }
+        }
+        weigh();
+        const float inv_w = 1.0f / total;
+        f32x4 sum[kDvPerWave];
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+          if (p >= parts) break;
+          const float c = weight[p] * inv_w;
+          if (p == part) {
+#pragma unroll
+            for (int n = 0; n < kDvPerWave; ++n) sum[n] = p == 0 ? o[n] * c : sum[n] + o[n] * c;
+          } else {
+#pragma unroll
+            for (int n = 0; n < kDvPerWave; ++n) sum[n] = p == 0 ? theirs[p][n] * c : sum[n] + theirs[p][n] * c;
+          }
+        }
+#pragma unroll
+        for (int n = 0; n < kDvPerWave; ++n) o[n] = sum[n];
       }
       lse2 = top + __builtin_amdgcn_logf(total);
     }

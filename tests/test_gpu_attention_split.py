@@ -105,3 +105,22 @@ def test_workgroups_without_a_tile_leave_infinities_alone(tokens):
         assert kt.torch.isposinf(out[1, :, 7].float()).all(), options
         rest = [c for c in range(LATENT) if c != 7]
         assert kt.torch.isfinite(out[1][:, rest].float()).all() and kt.torch.isfinite(lse).all()
+
+
+# Sharing a unit between four workgroups must not cost precision against two: error (2-norm, against the
+# oracle's float64 sums) over rows that grow or fall along the context, where the parts' weights differ and
+# every rounding of a part's rows shows (with bf16 slices it was 1.10 to 1.15 x that of two), and over equal
+# ones. No margin: four parts of fp32 round once less than two of bf16.
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("shape", ["grow", "fall", "equal"])
+def test_four_workgroups_are_as_precise_as_two(shape, fp8):
+    ctxs, heads = [768, 500, 300, 257, 90], 64
+    factor = {"grow": lambda at: 0.1 + at / 180.0, "fall": lambda at: 4.5 - at / 180.0, "equal": None}[shape]
+    cache, table = _cache(ctxs, 64, seed=941, fp8=fp8, grow=factor)
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=945).cuda()
+    expected, _ = kt.oracle_attention(cache, 0, q, table, ctxs, SCALE)
+    errors = []
+    for units in (kt.ffi.ATTN_UNITS_AUTO, kt.ffi.ATTN_UNITS_HEAD_BLOCK_HALVES):
+        out, _, _ = kt.attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE, selection_units=units)
+        errors.append(np.linalg.norm(out.double().cpu().numpy() - expected) / np.linalg.norm(expected))
+    assert errors[0] <= errors[1], errors
