@@ -678,9 +678,9 @@ struct MergeState {
 // loads: 0.3 to 0.5 us less per launch).
 // AGENT: the partials were written by other CUs of this launch (agent-scope loads); otherwise by
 // an earlier launch (plain streaming loads).
-// SHARED: other waves hold partials of the same head. A wave whose partials are all NaN then says so
-// with its denominator: beside finite partials of the others the row is NaN.
-template <bool AGENT, bool SHARED>
+// A NaN LSE spoils the row as it does in a sequence that is not split: where no maximum shows it (every
+// partial so far empty or NaN) the denominator carries it on.
+template <bool AGENT>
 __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_in_group, int first_slot, int u0, int first, int step,
                                              int n, int lane, MergeState& s) {
 #pragma unroll
@@ -706,12 +706,10 @@ __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_
     float group_max = s.m;
 #pragma unroll
     for (int u = 0; u < 8; ++u) group_max = fmaxf(group_max, l[u]);
-    if (group_max == -__builtin_inff()) {  // nothing but empty partials so far, or NaN ones, which no maximum shows
-      if constexpr (SHARED) {
+    if (group_max == -__builtin_inff()) {  // nothing but empty partials so far, or NaN ones
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          if (l[u] != l[u]) s.denom = l[u];
-        }
+      for (int u = 0; u < 8; ++u) {
+        if (l[u] != l[u]) s.denom = l[u];
       }
       continue;
     }
@@ -897,7 +895,7 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
           const int h = u * kMergeHeads + wave0;
           if (h < heads_here) {
             MergeState state;
-            TakePartials<true, false>(a, z, h, a.max_units + seq, u0, 0, 1, n, lane0, state);
+            TakePartials<true>(a, z, h, a.max_units + seq, u0, 0, 1, n, lane0, state);
             FinishHead<MXQ>(a, z, seq, h, lane0, state);
           }
         }
@@ -1577,7 +1575,7 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
   const int partials = (seq_end - 1) / cut.tiles_per_unit - first_unit + 1;
   if (partials == 1) return;  // written by the workgroup that held the whole sequence
   MergeState state;
-  if (has_head) TakePartials<false, (WAYS > 1)>(a, z, h, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
+  if (has_head) TakePartials<false>(a, z, h, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
   if constexpr (WAYS > 1) {
     if (way != 0 && has_head) {
 #pragma unroll
@@ -1605,8 +1603,9 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) state.acc[j] += weight * shared_acc[wave + w][j][lane];
       }
-    } else {
-      state.denom = 0.0f;  // no finite partial at all: zeros, as from one wave
+    } else {  // no finite partial at all: 0 from every wave, or NaN
+#pragma unroll
+      for (int w = 1; w < WAYS; ++w) state.denom += shared_ends[wave + w][1];
     }
   }
   FinishHead<MXQ>(a, z, seq, h, lane, state);

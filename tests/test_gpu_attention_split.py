@@ -124,3 +124,40 @@ def test_four_workgroups_are_as_precise_as_two(shape, fp8):
         out, _, _ = kt.attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE, selection_units=units)
         errors.append(np.linalg.norm(out.double().cpu().numpy() - expected) / np.linalg.norm(expected))
     assert errors[0] <= errors[1], errors
+
+
+# A NaN query row gives a NaN output row and LSE, whatever merges it: one, four or eight waves per head (10, 16
+# and 85 partials per sequence on average), the merge inside the launch, and a sequence that is not split.
+@pytest.mark.parametrize("ctxs,options", [([900] * 24, {"selection_units": 1}), ([2000] * 16, {"selection_units": 1}),
+                                          ([3000, 2000, 1000], {"selection_units": 1}),
+                                          ([900, 400, 700], {"chunk_tiles": 2, "merge_mode": 1}), ([900, 400, 30], {"chunk_tiles": 100})])
+def test_a_nan_query_head_gives_a_nan_row(ctxs, options):
+    cache, table = _cache(ctxs, 64, seed=951)
+    q = kt.randn_bf16((len(ctxs), 64, LATENT + ROPE), seed=955).cuda()
+    arguments = (kt.dev_i32(table), kt.dev_i32(ctxs), SCALE)
+    clean, clean_lse, _ = kt.attention(cache, 0, q, *arguments, **options)
+    spoiled = q.clone()
+    spoiled[1, 5] = float("nan")
+    out, lse, _ = kt.attention(cache, 0, spoiled, *arguments, **options)
+    assert kt.torch.isnan(out[1, 5].float()).all() and kt.torch.isnan(lse[1, 5])
+    out[1, 5], lse[1, 5] = clean[1, 5], clean_lse[1, 5]
+    assert kt.torch.equal(out, clean) and kt.torch.equal(lse, clean_lse)
+
+
+# NaN rows that fill exactly the first group of eight partials of a sequence, with finite partials behind them:
+# NaN from one wave per head (24 sequences; units of four tiles, the first of the long one with two of its
+# own), from eight, and from the merge inside the launch.
+@pytest.mark.parametrize("ctxs,options", [([40] * 23 + [20000], {"selection_units": 1}), ([600], {"chunk_tiles": 1}),
+                                          ([600, 64], {"chunk_tiles": 1, "merge_mode": 1})])
+def test_leading_nan_partials_spoil_the_row(ctxs, options):
+    cache, table = _cache(ctxs, 64, seed=961)
+    at = max(range(len(ctxs)), key=lambda s: ctxs[s])
+    spoiled = 32 * (2 + 7 * 4) if ctxs[at] > 600 else 32 * 8
+    for position in range(0, spoiled, 64):
+        rows = min(64, spoiled - position)
+        cache.latent[0, int(table[at, position // 64]), :rows] = float("nan")
+    q = kt.randn_bf16((len(ctxs), 64, LATENT + ROPE), seed=965).cuda()
+    out, lse, _ = kt.attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE, **options)
+    assert kt.torch.isnan(out[at].float()).all() and kt.torch.isnan(lse[at]).all()
+    others = [s for s in range(len(ctxs)) if s != at]
+    assert kt.torch.isfinite(out[others].float()).all()
