@@ -334,6 +334,8 @@ mlakvStatus mlakvCopyBlocks(const mlakvCacheView* cache, int32_t layer_begin, in
 namespace {
 
 constexpr int32_t kDefaultMergeSpinUs = 50;
+// mlakvAttnPlan::reserved: whole contexts, a selection, a selection whose halved units four workgroups share.
+constexpr int32_t kPlanContext = 0, kPlanSelection = 1, kPlanSelectionQuarters = 3;
 static_assert(MLAKV_ATTN_HEAD_BLOCK_TOKENS == mlakv::kAttnHeadBlockTokens, "the header states the kernel's staging size");
 
 // The largest unit (in tiles) whose block-table entries fit the kernel's LDS staging whatever
@@ -452,7 +454,7 @@ mlakvStatus AttnPlanImpl(const char* who, int32_t batch, int32_t heads, int32_t 
   // launch, which needs no counters, is the default.
   plan->merge_mode = chosen.merge_mode == MLAKV_ATTN_MERGE_IN_LAUNCH && fits ? MLAKV_ATTN_MERGE_IN_LAUNCH : MLAKV_ATTN_MERGE_SECOND_LAUNCH;
   plan->merge_spin_us = chosen.merge_spin_us == 0 ? kDefaultMergeSpinUs : (chosen.merge_spin_us < 0 ? -1 : chosen.merge_spin_us);
-  plan->reserved = sparse ? 1 : 0;
+  plan->reserved = sparse ? kPlanSelection : kPlanContext;
   // Whole-selection units of 16 heads where they apply, unless the caller asked for properties of
   // the split (a unit size, a workgroup count, a merge).
   const bool head_block_fits = sparse && max_seq_len <= MLAKV_ATTN_HEAD_BLOCK_TOKENS;
@@ -503,6 +505,12 @@ mlakvStatus AttnPlanImpl(const char* who, int32_t batch, int32_t heads, int32_t 
     plan->selection_units = chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && split_asked ? MLAKV_ATTN_UNITS_SPLIT : chosen.selection_units;
   }
   if (halves) shape = ShapeOf(batch, heads, max_seq_len, block_size, sparse, chunk_tiles, work_groups, true);
+  // A caller that asks for halves gets two workgroups per unit and their footprint in the workspace; only
+  // the plan's own choice may share a unit between four.
+  if (halves && chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && SharedUnitParts(pairs) == 4 &&
+      HeadBlockPartialBytes(batch, heads, 4) <= shape.workspace) {
+    plan->reserved = kPlanSelectionQuarters;
+  }
   plan->workspace_bytes = shape.workspace;
   return MLAKV_SUCCESS;
 }
@@ -583,8 +591,10 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
   {
     const bool fields = plan->batch > 0 && plan->batch <= 65535 && plan->heads > 0 && plan->heads % 16 == 0 && plan->heads <= 128 &&
                         plan->max_seq_len > 0 && plan->block_size > 0 && plan->chunk_tiles >= 0 && plan->work_groups >= 1 &&
-                        plan->work_groups <= 65535 && (plan->reserved == 0 || plan->reserved == 1) &&
-                        (plan->reserved == 0 ? (plan->selection_units == MLAKV_ATTN_UNITS_AUTO || plan->selection_units == MLAKV_ATTN_UNITS_SPLIT ||
+                        plan->work_groups <= 65535 &&
+                        (plan->reserved == kPlanContext || plan->reserved == kPlanSelection ||
+                         (plan->reserved == kPlanSelectionQuarters && plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES)) &&
+                        (plan->reserved == kPlanContext ? (plan->selection_units == MLAKV_ATTN_UNITS_AUTO || plan->selection_units == MLAKV_ATTN_UNITS_SPLIT ||
                                                 ((plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK ||
                                                   plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) &&
                                                  plan->max_seq_len <= MLAKV_ATTN_HEAD_BLOCK_TOKENS))
@@ -592,14 +602,14 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
                                                 ((plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK ||
                                                   plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) &&
                                                  plan->max_seq_len <= MLAKV_ATTN_HEAD_BLOCK_TOKENS))) &&
-                        (plan->reserved == 0 || plan->max_seq_len <= 2048) &&
+                        (plan->reserved == kPlanContext || plan->max_seq_len <= 2048) &&
                         (plan->merge_mode == MLAKV_ATTN_MERGE_IN_LAUNCH || plan->merge_mode == MLAKV_ATTN_MERGE_SECOND_LAUNCH) &&
                         (plan->merge_spin_us == -1 || (plan->merge_spin_us > 0 && plan->merge_spin_us <= 1000000));
     bool sane = fields;
     if (fields) {
-      const PlanShape shape = ShapeOf(plan->batch, plan->heads, plan->max_seq_len, plan->block_size, plan->reserved == 1,
+      const PlanShape shape = ShapeOf(plan->batch, plan->heads, plan->max_seq_len, plan->block_size, plan->reserved != kPlanContext,
                                       plan->chunk_tiles, plan->work_groups,
-                                      plan->reserved == 1 && plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES);
+                                      plan->reserved != kPlanContext && plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES);
       sane = plan->chunk_tiles <= shape.cap && plan->max_units == shape.units && plan->workspace_bytes == shape.workspace &&
              (plan->merge_mode != MLAKV_ATTN_MERGE_IN_LAUNCH ||
               (static_cast<int64_t>(plan->batch) * shape.head_groups <= mlakv::kAttnSyncSequences && shape.units < 65535));
@@ -609,9 +619,9 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
     }
   }
   const bool sparse = sparse_indices != nullptr;
-  if (sparse != (plan->reserved == 1)) {
+  if (sparse != (plan->reserved != kPlanContext)) {
     return Fail(MLAKV_ERR_PARAM_INVALID, "%s: the plan was made by %s", who,
-                plan->reserved == 1 ? "mlakvAttnSparsePlanInit (selected-token attention)" : "mlakvAttnPlanInit (whole-context attention)");
+                plan->reserved != kPlanContext ? "mlakvAttnSparsePlanInit (selected-token attention)" : "mlakvAttnPlanInit (whole-context attention)");
   }
   if (sparse && (sparse_indices_seq_stride < plan->max_seq_len || reinterpret_cast<uintptr_t>(sparse_indices) % 4 != 0)) {
     return Fail(MLAKV_ERR_PARAM_INVALID, "%s: a row of the selection holds %d int32 entries", who, plan->max_seq_len);
@@ -696,15 +706,14 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
   args.merge_in_launch = plan->merge_mode == MLAKV_ATTN_MERGE_IN_LAUNCH;
   args.fp8 = cache->dtype == MLAKV_DTYPE_FP8_E4M3;
   args.head_block_units = plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK ? 1 : (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES ? 2 : 0);
-  const int64_t pairs = static_cast<int64_t>(plan->batch) * (plan->heads / 16);
   // (the parts' partials must fit the plan's workspace, which is sized for the split and, with a
   // selection, for two parts)
   const auto partial_bytes = [&]() { return HeadBlockPartialBytes(plan->batch, plan->heads, args.head_block_units); };
   const auto shrink_to_workspace = [&]() {
     while (args.head_block_units > 1 && partial_bytes() > plan->workspace_bytes) args.head_block_units /= 2;
   };
-  if (sparse && args.head_block_units == 2 && args.sparse_count > 256) {
-    args.head_block_units = SharedUnitParts(pairs);
+  if (plan->reserved == kPlanSelectionQuarters) {
+    args.head_block_units = 4;
     shrink_to_workspace();
   }
   if (!sparse) {

@@ -185,7 +185,8 @@ typedef struct mlakvAttnPlan {
   int32_t max_units;       /* bound on the work units of one launch (sizes the workspace) */
   int32_t merge_mode;      /* MLAKV_ATTN_MERGE_IN_LAUNCH or _SECOND_LAUNCH */
   int32_t merge_spin_us;   /* bound of the in-launch merge's wait for a sequence's other partials */
-  int32_t reserved;        /* 1: made by mlakvAttnSparsePlanInit (max_seq_len holds sparse_count) */
+  int32_t reserved;        /* 1 or 3: made by mlakvAttnSparsePlanInit (max_seq_len holds sparse_count); 3: its halved units are
+                            * shared by four workgroups each */
   int32_t selection_units; /* selected-token plans: MLAKV_ATTN_UNITS_SPLIT, _HEAD_BLOCK or _HEAD_BLOCK_HALVES, fixed by the plan;
                             * whole-context plans: what the options asked for, MLAKV_ATTN_UNITS_AUTO = every launch chooses */
   uint64_t workspace_bytes;
@@ -202,12 +203,12 @@ mlakvStatus mlakvAttnPlanInit(int32_t batch, int32_t heads, int32_t max_seq_len,
  *   unit; units that hold part of a selection leave partials that a merge puts together.
  * HEAD_BLOCK: one unit = the whole selection of one sequence for 16 heads; nothing to merge and the
  *   workspace stays untouched. sparse_count up to MLAKV_ATTN_HEAD_BLOCK_TOKENS.
- * HEAD_BLOCK_HALVES: the same unit shared by two workgroups, half of the selection's tiles each (or by
- *   four, a quarter each, above 256 selected tokens while four per unit fit the CUs once); each
- *   leaves a partial (16 rows) in the workspace and counts itself on a word of the library's
- *   counters (those of MLAKV_ATTN_MERGE_IN_LAUNCH, with their limit on launches in flight); the
- *   last to finish combines them inside the launch, nobody waits. Up to 2048 (sequence, 16
- *   heads) pairs.
+ * HEAD_BLOCK_HALVES: the same unit shared by two workgroups, half of the selection's tiles each (a
+ *   plan in which AUTO chose it shares a unit between four, a quarter each, while four per unit fit the
+ *   CUs once: its `reserved` is 3); each leaves a partial (16 rows) in the workspace and counts
+ *   itself on a word of the library's counters (those of MLAKV_ATTN_MERGE_IN_LAUNCH, with their
+ *   limit on launches in flight); the last to finish combines them inside the launch, nobody
+ *   waits. Up to 2048 (sequence, 16 heads) pairs.
  * AUTO, unless chunk_tiles, work_groups or merge_mode ask for properties of the split, takes what
  * was measured ahead. bf16 caches: HEAD_BLOCK_HALVES from 257 to 768 selected tokens while two
  * workgroups per unit fit the CUs once; else HEAD_BLOCK up to 512 selected tokens while batch x
@@ -349,7 +350,8 @@ mlakvStatus mlakvAttnDecodeMxQuant(const mlakvAttnPlan* plan, const mlakvCacheVi
  * The plan comes from mlakvAttnSparsePlanInit (sparse_count takes the place of max_seq_len); how
  * it cuts the work (plan->selection_units) is described with MLAKV_ATTN_UNITS_* above. The
  * workspace is required either way; whole-selection units leave it untouched, halved ones use
- * its first 2112 bytes x batch x heads. */
+ * its first 2112 bytes x batch x heads, those that four workgroups share (plan->reserved is 3; never
+ * where the options ask for HEAD_BLOCK_HALVES) its first 8256 bytes x batch x heads. */
 mlakvStatus mlakvAttnSparsePlanInit(int32_t batch, int32_t heads, int32_t sparse_count, int32_t block_size, int32_t dtype,
                                     mlakvAttnPlan* plan);
 mlakvStatus mlakvAttnDecodeSparse(const mlakvAttnPlan* plan, const mlakvCacheView* cache, int32_t layer,

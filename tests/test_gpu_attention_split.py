@@ -1,6 +1,7 @@
 """GPU parity of the variants of the split-KV decode attention, at the sizes where the choice between
 them changes, against the CPU oracle (float64 accumulation) with the tolerances of
 test_gpu_attention.py: 2e-2 of the peak for bf16 KV, 6e-2 for FP8 KV."""
+import ctypes as C
 import math
 
 import numpy as np
@@ -161,3 +162,42 @@ def test_leading_nan_partials_spoil_the_row(ctxs, options):
     assert kt.torch.isnan(out[at].float()).all() and kt.torch.isnan(lse[at]).all()
     others = [s for s in range(len(ctxs)) if s != at]
     assert kt.torch.isfinite(out[others].float()).all()
+
+
+SENTINEL = 0xA5
+
+
+def _workspace_after(cache, table, ctxs, heads, sparse=None, selection_units=0):
+    """The plan, and its workspace (filled with SENTINEL before) after one launch."""
+    lib, batch, row = kt.ffi.load(), len(ctxs), 2 * (LATENT + ROPE)
+    plan = kt.make_plan(batch, heads, max(ctxs) if sparse is None else sparse.shape[1], cache.block_size, cache.fp8,
+                        selection=sparse is not None, selection_units=selection_units)
+    workspace = kt.torch.full((int(plan.workspace_bytes),), SENTINEL, dtype=kt.torch.uint8, device="cuda")
+    q = kt.randn_bf16((batch, heads, LATENT + ROPE), seed=975).cuda()
+    out = kt.torch.zeros(batch, heads, LATENT, dtype=kt.torch.bfloat16, device="cuda")
+    table_d, lens_d = kt.dev_i32(table), kt.dev_i32(ctxs)
+    before = (C.byref(plan), C.byref(cache.view), 0, q.data_ptr(), heads * row, row, q.data_ptr() + 2 * LATENT, heads * row, row,
+              table_d.data_ptr(), table_d.shape[1], lens_d.data_ptr())
+    after = (SCALE, out.data_ptr(), 2 * heads * LATENT, 2 * LATENT, None, workspace.data_ptr(), int(plan.workspace_bytes), kt.stream_ptr())
+    if sparse is None:
+        kt.ffi.check(lib.mlakvAttnDecode(*before, *after))
+    else:
+        selection = kt.dev_i32(sparse)
+        kt.ffi.check(lib.mlakvAttnDecodeSparse(*before, selection.data_ptr(), sparse.shape[1], *after))
+    kt.torch.cuda.synchronize()
+    return plan, workspace
+
+
+# What halved units write: two workgroups per unit (asked for by the options) the first 2112 bytes x batch x heads
+# that the header gives them, four (the plan's own choice) 8256 and more than 2112, where four per unit fit.
+@pytest.mark.parametrize("k", [257, 512, 768])
+def test_halved_units_keep_to_their_part_of_the_workspace(k):
+    ctxs, heads = [k + 100, 900, k], 64
+    cache, table = _cache(ctxs, 64, seed=971)
+    sparse = np.stack([np.random.default_rng(973).permutation(n)[:k] for n in ctxs]).astype(np.int32)
+    plan, workspace = _workspace_after(cache, table, ctxs, heads, sparse, kt.ffi.ATTN_UNITS_HEAD_BLOCK_HALVES)
+    assert plan.reserved == 1 and (workspace[:1024 * heads] != SENTINEL).any()
+    assert (workspace[2112 * len(ctxs) * heads:] == SENTINEL).all()
+    plan, workspace = _workspace_after(cache, table, ctxs, heads, sparse)
+    assert plan.reserved == 3 and (workspace[2112 * len(ctxs) * heads:] != SENTINEL).any()
+    assert (workspace[8256 * len(ctxs) * heads:] == SENTINEL).all()
