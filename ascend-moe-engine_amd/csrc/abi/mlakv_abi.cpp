@@ -382,10 +382,16 @@ PlanShape ShapeOf(int32_t batch, int32_t heads, int32_t max_seq_len, int32_t blo
 }
 
 // Workgroups of a unit of 16 heads that is shared: four while four per unit fit the CUs once, else
-// two. Measured, append + attention of a layer, whole contexts (us, one / two / four workgroups): batch 8,
-// 64 heads, bf16, 256 tokens 13.1 / 13.3 / 13.3; 384: 16.5 / 14.9 / 14.5; 512: 19.3 / 16.5 / 15.4; 768: 24.6 /
-// 19.2 / 16.9; batch 16, 600: 21.5 / 18.3 / 16.5; 7 x 128 heads, 600: 21.3 / 18.0 / 16.5; FP8 alike.
-int32_t SharedUnitParts(int64_t pairs) { return 4 * pairs <= ComputeUnits() ? 4 : 2; }
+// two. A sequence's units all sit on one XCD (sequence s on XCD s % 8), so it is the CUs of the XCD
+// with the most sequences that have to hold them; where they need a second round there, four lose. Measured,
+// attention launch alone (us, two / four workgroups): 8 x 64 heads, bf16, 384 tokens 11.4 / 11.0; 512:
+// 12.7 / 11.7; 768: 15.5 / 13.1; 16 x 64, 600: 14.1 / 12.6; 8 x 128, 600: 14.2 / 12.9; FP8 alike. In two
+// rounds: 17 x 48, 288: 10.7 / 18.3; 768: 15.8 / 20.7; 12 x 80, 600: 14.2 / 20.1; 9 x 112, 768: 16.0 / 23.8.
+int32_t SharedUnitParts(int32_t batch, int32_t heads) {
+  constexpr int32_t kXcds = 8;
+  const int64_t fullest = static_cast<int64_t>((batch + kXcds - 1) / kXcds) * (heads / 16);
+  return 4 * fullest <= ComputeUnits() / kXcds ? 4 : 2;
+}
 
 // How a whole-context launch whose longest context is `bound` tokens cuts its work: 0 = the
 // 64-head kernel's flat cut, 1 = one workgroup per (sequence, 16 heads), 2 or 4 = that many. Measured on
@@ -401,7 +407,7 @@ int32_t ShortContextUnits(const mlakvAttnPlan* plan, int32_t bound) {
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK) return 1;
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) return 2;
   const int64_t pairs = static_cast<int64_t>(plan->batch) * (plan->heads / 16);
-  if (2 * pairs <= ComputeUnits()) return bound <= 256 ? 1 : (bound <= 768 ? SharedUnitParts(pairs) : 0);
+  if (2 * pairs <= ComputeUnits()) return bound <= 256 ? 1 : (bound <= 768 ? SharedUnitParts(plan->batch, plan->heads) : 0);
   if (pairs <= ComputeUnits()) return bound <= 512 ? 1 : 0;
   if (pairs <= 2 * ComputeUnits()) return bound <= 256 ? 1 : 0;
   return 0;
@@ -507,7 +513,7 @@ mlakvStatus AttnPlanImpl(const char* who, int32_t batch, int32_t heads, int32_t 
   if (halves) shape = ShapeOf(batch, heads, max_seq_len, block_size, sparse, chunk_tiles, work_groups, true);
   // A caller that asks for halves gets two workgroups per unit and their footprint in the workspace; only
   // the plan's own choice may share a unit between four.
-  if (halves && chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && SharedUnitParts(pairs) == 4 &&
+  if (halves && chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && SharedUnitParts(batch, heads) == 4 &&
       HeadBlockPartialBytes(batch, heads, 4) <= shape.workspace) {
     plan->reserved = kPlanSelectionQuarters;
   }

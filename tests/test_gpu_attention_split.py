@@ -201,3 +201,20 @@ def test_halved_units_keep_to_their_part_of_the_workspace(k):
     plan, workspace = _workspace_after(cache, table, ctxs, heads, sparse)
     assert plan.reserved == 3 and (workspace[2112 * len(ctxs) * heads:] != SENTINEL).any()
     assert (workspace[8256 * len(ctxs) * heads:] == SENTINEL).all()
+
+
+# Four workgroups per unit only where the XCD with the most sequences holds them all at once (32 CUs, sequence s on
+# XCD s % 8): seen in the workspace, where four write beyond the 2080 bytes x batch x heads of two.
+@pytest.mark.skipif(not kt.torch.cuda.is_available() or kt.torch.cuda.get_device_properties(0).multi_processor_count != 256,
+                    reason="the sizes are those of 256 CUs")
+@pytest.mark.parametrize("batch,heads,parts", [(16, 64, 4), (17, 64, 2), (8, 128, 4), (9, 128, 2), (16, 48, 4), (17, 48, 2), (21, 48, 2),
+                                               (8, 80, 4), (12, 80, 2), (8, 112, 4), (9, 112, 2), (64, 16, 4)])
+def test_four_workgroups_only_where_an_xcd_holds_them(batch, heads, parts):
+    ctxs = [400 + i for i in range(batch)]
+    cache, table = _cache(ctxs, 64, seed=981)
+    _, workspace = _workspace_after(cache, table, ctxs, heads)
+    assert bool((workspace[2112 * batch * heads:] != SENTINEL).any()) == (parts == 4)
+    sparse = np.stack([np.arange(400) for _ in ctxs]).astype(np.int32)
+    plan, workspace = _workspace_after(cache, table, ctxs, heads, sparse)
+    assert plan.reserved == (3 if parts == 4 else 1)
+    assert bool((workspace[2112 * batch * heads:] != SENTINEL).any()) == (parts == 4)
