@@ -2161,8 +2161,8 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
       if (Uniform(arrived) != static_cast<unsigned>(parts - 1)) return;  // the last part's wave will find this slice
       if (lane == 0) __hip_atomic_store(word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       asm volatile("" ::: "memory");  // (no load below moves in front of the count)
-      // Whichever part arrives last, the result is the same: every partial enters as it was stored, in
-      // the order of the parts (parts that do not exist are left out).
+      // Whichever part arrives last, the result is the same: every partial enters as it was stored, this
+      // wave's own from its registers, in the order of the parts (those that do not exist are left out).
       float lses2[PARTS], top = lse2, weight[PARTS], total = 0.0f;
       const auto weigh = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -2176,35 +2176,30 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
         }
       };
       if constexpr (PARTS == 2) {
-        u32x4 slice[PARTS][4];
+        const int other = part ^ 1;
+        const float lse2_other = LoadAgentF32(lses + other * 64);
 #pragma unroll
-        for (int p = 0; p < PARTS; ++p) {
-          lses2[p] = LoadAgentF32(lses + p * 64);
+        for (int it = 0; it < 4; ++it) v[it] = LoadAgent16(slices + (16 * other + 4 * it + sub) * (kLatentDim * 2));
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) : : "memory");
 #pragma unroll
-          for (int it = 0; it < 4; ++it) slice[p][it] = LoadAgent16(slices + (16 * p + 4 * it + sub) * (kLatentDim * 2));
-        }
-#pragma unroll
-        for (int p = 0; p < PARTS; ++p) {
-          asm volatile("s_waitcnt vmcnt(0)" : "+v"(slice[p][0]), "+v"(slice[p][1]), "+v"(slice[p][2]), "+v"(slice[p][3]) : : "memory");
-        }
+        for (int it = 0; it < 4; ++it) *reinterpret_cast<u32x4*>(stage + (4 * it + sub) * kStageRow + piece * 16) = v[it];
+        const bool second = part != 0;
+        lses2[0] = second ? lse2_other : lse2;
+        lses2[1] = second ? lse2 : lse2_other;
         weigh();
-        const float inv_w = 1.0f / total;
+        const float inv_w = 1.0f / total, c_first = weight[0] * inv_w, c_second = weight[1] * inv_w;
 #pragma unroll
-        for (int p = 0; p < PARTS; ++p) {
+        for (int n = 0; n < kDvPerWave; ++n) {
+          const u32x2 packed = *reinterpret_cast<const u32x2*>(stage + i16 * kStageRow + (16 * n + 4 * g) * 2);
+          const float theirs[4] = {__builtin_bit_cast(float, packed.x << 16), __builtin_bit_cast(float, packed.x & 0xffff0000u),
+                                   __builtin_bit_cast(float, packed.y << 16), __builtin_bit_cast(float, packed.y & 0xffff0000u)};
 #pragma unroll
-          for (int it = 0; it < 4; ++it) *reinterpret_cast<u32x4*>(stage + (4 * it + sub) * kStageRow + piece * 16) = slice[p][it];
-          const float c = weight[p] * inv_w;
-#pragma unroll
-          for (int n = 0; n < kDvPerWave; ++n) {
-            const u32x2 packed = *reinterpret_cast<const u32x2*>(stage + i16 * kStageRow + (16 * n + 4 * g) * 2);
-            const float values[4] = {__builtin_bit_cast(float, packed.x << 16), __builtin_bit_cast(float, packed.x & 0xffff0000u),
-                                     __builtin_bit_cast(float, packed.y << 16), __builtin_bit_cast(float, packed.y & 0xffff0000u)};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) o[n][j] = p == 0 ? values[j] * c : o[n][j] + values[j] * c;
+          for (int j = 0; j < 4; ++j) {
+            const float mine = static_cast<float>(static_cast<__bf16>(o[n][j]));
+            o[n][j] = (second ? theirs[j] : mine) * c_first + (second ? mine : theirs[j]) * c_second;
           }
         }
       } else {
-        // (this part's own slice is still in the registers)
         const __amdgpu_buffer_rsrc_t memory = __builtin_amdgcn_make_buffer_rsrc(unit_parts, 0, PARTS * kPartBytes, 0x00020000);
         const int at = hw * (kPartBytes / kScoreWaves) + lane * 16;
         f32x4 theirs[PARTS][kDvPerWave];
