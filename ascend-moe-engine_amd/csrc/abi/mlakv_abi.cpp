@@ -387,8 +387,12 @@ PlanShape ShapeOf(int32_t batch, int32_t heads, int32_t max_seq_len, int32_t blo
 // attention launch alone (us, two / four workgroups): 8 x 64 heads, bf16, 384 tokens 11.4 / 11.0; 512:
 // 12.7 / 11.7; 768: 15.5 / 13.1; 16 x 64, 600: 14.1 / 12.6; 8 x 128, 600: 14.2 / 12.9; FP8 alike. In two
 // rounds: 17 x 48, 288: 10.7 / 18.3; 768: 15.8 / 20.7; 12 x 80, 600: 14.2 / 20.1; 9 x 112, 768: 16.0 / 23.8.
-int32_t SharedUnitParts(int32_t batch, int32_t heads) {
+// Nine tiles in quarters are level with halves (8 x 64, 288: 10.5 / 10.5), and behind where a sequence has more
+// than four units, which all fetch the same rows: 8 x 128, bf16, 257: 10.8 / 11.3; 320: 11.1 / 11.4; 384:
+// 11.9 / 12.1; 416: 12.1 / 12.0; FP8, 288: 11.2 / 11.4; 320: 11.7 / 11.5.
+int32_t SharedUnitParts(int32_t batch, int32_t heads, int32_t tokens, int32_t dtype) {
   constexpr int32_t kXcds = 8;
+  if (heads > 64 && tokens <= (dtype == MLAKV_DTYPE_BF16 ? 384 : 288)) return 2;
   const int64_t fullest = static_cast<int64_t>((batch + kXcds - 1) / kXcds) * (heads / 16);
   return 4 * fullest <= ComputeUnits() / kXcds ? 4 : 2;
 }
@@ -407,7 +411,7 @@ int32_t ShortContextUnits(const mlakvAttnPlan* plan, int32_t bound) {
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK) return 1;
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) return 2;
   const int64_t pairs = static_cast<int64_t>(plan->batch) * (plan->heads / 16);
-  if (2 * pairs <= ComputeUnits()) return bound <= 256 ? 1 : (bound <= 768 ? SharedUnitParts(plan->batch, plan->heads) : 0);
+  if (2 * pairs <= ComputeUnits()) return bound <= 256 ? 1 : (bound <= 768 ? SharedUnitParts(plan->batch, plan->heads, bound, plan->dtype) : 0);
   if (pairs <= ComputeUnits()) return bound <= 512 ? 1 : 0;
   if (pairs <= 2 * ComputeUnits()) return bound <= 256 ? 1 : 0;
   return 0;
@@ -513,7 +517,7 @@ mlakvStatus AttnPlanImpl(const char* who, int32_t batch, int32_t heads, int32_t 
   if (halves) shape = ShapeOf(batch, heads, max_seq_len, block_size, sparse, chunk_tiles, work_groups, true);
   // A caller that asks for halves gets two workgroups per unit and their footprint in the workspace; only
   // the plan's own choice may share a unit between four.
-  if (halves && chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && SharedUnitParts(batch, heads) == 4 &&
+  if (halves && chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && SharedUnitParts(batch, heads, max_seq_len, dtype) == 4 &&
       HeadBlockPartialBytes(batch, heads, 4) <= shape.workspace) {
     plan->reserved = kPlanSelectionQuarters;
   }

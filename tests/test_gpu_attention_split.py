@@ -204,17 +204,21 @@ def test_halved_units_keep_to_their_part_of_the_workspace(k):
 
 
 # Four workgroups per unit only where the XCD with the most sequences holds them all at once (32 CUs, sequence s on
-# XCD s % 8): seen in the workspace, where four write beyond the 2080 bytes x batch x heads of two.
+# XCD s % 8), with more than 64 heads from 385 tokens on (FP8 289): seen in the workspace, where four write beyond
+# the 2080 bytes x batch x heads of two.
 @pytest.mark.skipif(not kt.torch.cuda.is_available() or kt.torch.cuda.get_device_properties(0).multi_processor_count != 256,
                     reason="the sizes are those of 256 CUs")
-@pytest.mark.parametrize("batch,heads,parts", [(16, 64, 4), (17, 64, 2), (8, 128, 4), (9, 128, 2), (16, 48, 4), (17, 48, 2), (21, 48, 2),
-                                               (8, 80, 4), (12, 80, 2), (8, 112, 4), (9, 112, 2), (64, 16, 4)])
-def test_four_workgroups_only_where_an_xcd_holds_them(batch, heads, parts):
-    ctxs = [400 + i for i in range(batch)]
-    cache, table = _cache(ctxs, 64, seed=981)
+@pytest.mark.parametrize("batch,heads,most,fp8,parts", [
+    (16, 64, 415, False, 4), (17, 64, 416, False, 2), (8, 128, 407, False, 4), (9, 128, 408, False, 2), (16, 48, 415, False, 4),
+    (17, 48, 416, False, 2), (21, 48, 420, False, 2), (8, 80, 407, False, 4), (12, 80, 411, False, 2), (8, 112, 407, False, 4),
+    (9, 112, 408, False, 2), (64, 16, 463, False, 4), (2, 128, 384, False, 2), (2, 128, 385, False, 4), (2, 80, 288, True, 2),
+    (2, 80, 289, True, 4), (2, 64, 257, False, 4), (2, 64, 256, False, 1)])
+def test_four_workgroups_only_where_an_xcd_holds_them(batch, heads, most, fp8, parts):
+    ctxs = [most - i for i in range(batch)]
+    cache, table = _cache(ctxs, 64, seed=981, fp8=fp8)
     _, workspace = _workspace_after(cache, table, ctxs, heads)
     assert bool((workspace[2112 * batch * heads:] != SENTINEL).any()) == (parts == 4)
-    sparse = np.stack([np.arange(400) for _ in ctxs]).astype(np.int32)
+    sparse = np.stack([np.r_[:n, [-1] * (most - n)] for n in ctxs]).astype(np.int32)
     plan, workspace = _workspace_after(cache, table, ctxs, heads, sparse)
     assert plan.reserved == (3 if parts == 4 else 1)
     assert bool((workspace[2112 * batch * heads:] != SENTINEL).any()) == (parts == 4)
