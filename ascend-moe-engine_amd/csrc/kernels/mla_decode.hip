@@ -678,8 +678,7 @@ struct MergeState {
 // loads: 0.3 to 0.5 us less per launch).
 // AGENT: the partials were written by other CUs of this launch (agent-scope loads); otherwise by
 // an earlier launch (plain streaming loads).
-// A NaN LSE spoils the row as it does in a sequence that is not split: where no maximum shows it (every
-// partial so far empty or NaN) the denominator carries it on.
+// A NaN LSE spoils the row as it does in a sequence that is not split: the maximum carries it on.
 template <bool AGENT>
 __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_in_group, int first_slot, int u0, int first, int step,
                                              int n, int lane, MergeState& s) {
@@ -705,14 +704,8 @@ __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_
     if constexpr (AGENT) WaitAgentLoads(v);
     float group_max = s.m;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) group_max = fmaxf(group_max, l[u]);
-    if (group_max == -__builtin_inff()) {  // nothing but empty partials so far, or NaN ones
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        if (l[u] != l[u]) s.denom = l[u];
-      }
-      continue;
-    }
+    for (int u = 0; u < 8; ++u) group_max = __builtin_elementwise_maximum(group_max, l[u]);
+    if (group_max == -__builtin_inff()) continue;  // nothing but empty partials so far
     const float rescale = __builtin_amdgcn_exp2f(s.m - group_max);  // 0 on the first group
     s.m = group_max;
     s.denom *= rescale;
@@ -1589,7 +1582,7 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
     if (way != 0 || !has_head) return;
     float top = state.m;
 #pragma unroll
-    for (int w = 1; w < WAYS; ++w) top = fmaxf(top, shared_ends[wave + w][0]);
+    for (int w = 1; w < WAYS; ++w) top = __builtin_elementwise_maximum(top, shared_ends[wave + w][0]);
     if (top != -__builtin_inff()) {
       const float own = __builtin_amdgcn_exp2f(state.m - top);
       state.m = top;
@@ -1603,9 +1596,6 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) state.acc[j] += weight * shared_acc[wave + w][j][lane];
       }
-    } else {  // no finite partial at all: 0 from every wave, or NaN
-#pragma unroll
-      for (int w = 1; w < WAYS; ++w) state.denom += shared_ends[wave + w][1];
     }
   }
   FinishHead<MXQ>(a, z, seq, h, lane, state);
