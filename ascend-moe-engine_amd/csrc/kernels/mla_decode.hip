@@ -1522,54 +1522,85 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
 }
 
 // The merge as a launch of its own, for launches that have no counters to meet on: block =
-// (8 / WAYS heads, sequence, head group); every wave repeats the cut of the flat tile axis. WAYS
-// waves share a head, wave w of them takes partials w, w + WAYS, ..., and the first adds up what
-// they hold through LDS. What bounds it is the chain of memory trips (lengths, then a group of eight
-// rows at a time) and how many rows are on their way at once: one wave per head leaves a launch of
-// few sequences with few waves and many partials each. Measured (64 heads, FP8, 3 sequences of 15k
-// to 33k tokens, about 85 partials per head): 18.6 us with one wave per head, 6.9 us with eight.
+// (8 / WAYS heads, sequence, head group). WAYS waves share a head, wave w of them takes partials w,
+// w + WAYS, ..., and the first adds up what they hold through LDS. What bounds it is the chain of
+// memory trips (lengths, then a group of eight rows at a time) and how many rows are on their way at once:
+// one wave per head leaves a launch of few sequences with few waves and many partials each. Measured (64
+// heads, FP8, 3 sequences of 15k to 33k tokens, about 85 partials per head): 18.6 us with one wave per
+// head, 6.9 us with eight.
+// The launch is made for the partials that the plan allows. A sequence that has fewer is merged by one wave per
+// head in the first workgroups, and the others leave: up to eight partials are one group of loads
+// for a wave, and more waves would only load the same rows. Measured, attention + merge of a layer in a
+// plan of 32768 tokens, one wave / all: eight waves per head, 1 x 1000 tokens (8 partials) 16.6 / 17.0 us, 1 x
+// 1100 (9) 17.4 / 16.6, 4 x 1200 (10) 18.8 / 17.9; four, where the chip is fuller, 20 x 4000 (12) 29.8 / 31.2, 16
+// x 2000 (14) 22.2 / 22.6, 12 x 2000 (17) 20.8 / 21.1, 12 x 3000 (25) 23.7 / 22.7.
+// So that the surplus costs little, one wave repeats the cut of the flat tile axis for its workgroup
+// (20 x 32 tokens, nothing to merge: 12.5 us with every wave, 11.4 so), and where waves share heads
+// all first workgroups of the sequences come before any second (with a sequence's workgroups side by
+// side those with work sat on an eighth or a quarter of the CUs: 20 x 200 tokens 19.5 us, 17.8 so).
 template <bool MXQ, bool SPARSE, int WAYS>
 __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
   __shared__ float shared_acc[WAYS > 1 ? kMergeHeads : 1][8][64];
   __shared__ float shared_ends[WAYS > 1 ? kMergeHeads : 1][2];  // reference maximum and denominator
+  __shared__ int cut_lds[2];
   const int lane = threadIdx.x & 63, wave = Uniform(threadIdx.x >> 6);
   // Workgroups go to the XCDs round-robin by linear id. The main launch put the units of XCD x's
   // share of the flat tile axis on XCD x; with equal lengths that is the x-th eighth of the
   // sequences, whose partials are most likely still in that L2.
-  int seq = blockIdx.y, group = blockIdx.x;
-  const int z = blockIdx.z;
-  if ((gridDim.y & (kXcds - 1)) == 0) {
-    const int linear = blockIdx.y * gridDim.x + blockIdx.x;
-    const int within = linear / kXcds;
-    seq = (linear & (kXcds - 1)) * (gridDim.y / kXcds) + within / static_cast<int>(gridDim.x);
-    group = within % static_cast<int>(gridDim.x);
+  const int groups = WAYS == 1 ? gridDim.x : gridDim.y, batch = WAYS == 1 ? gridDim.y : gridDim.x;
+  const int linear = blockIdx.y * gridDim.x + blockIdx.x, z = blockIdx.z;
+  int seq = WAYS == 1 ? blockIdx.y : blockIdx.x, group = WAYS == 1 ? blockIdx.x : blockIdx.y;
+  if ((batch & (kXcds - 1)) == 0) {
+    const int within = linear / kXcds, share = batch / kXcds;
+    seq = (linear & (kXcds - 1)) * share + (WAYS == 1 ? within / groups : within % share);
+    group = WAYS == 1 ? within % groups : within / share;
   }
-  const int h = group * (kMergeHeads / WAYS) + wave / WAYS, way = wave % WAYS;
-  const bool has_head = h < min(64, a.heads - 64 * z);
-  if (WAYS == 1 && !has_head) return;
-  SeqWindow<SPARSE> win;
-  win.Load(a, lane, 0, 0, 0);
-  int end_tiles = 0, end_live = 0, seq_tiles = 0, common_tiles = 0;
-  for (;;) {
-    if (seq >= win.base && seq < win.base + 64) {
-      end_tiles = win.End(seq, 0);
-      end_live = win.End(seq, 1) - end_tiles;
-      seq_tiles = win.Tiles(seq);
+  const int heads_here = min(64, a.heads - 64 * z);
+  if (WAYS == 1 && group * kMergeHeads + wave >= heads_here) return;
+  int first_unit = 0, partials = 0;
+  if (WAYS == 1 || wave == 0) {
+    SeqWindow<SPARSE> win;
+    win.Load(a, lane, 0, 0, 0);
+    int end_tiles = 0, end_live = 0, seq_tiles = 0, common_tiles = 0;
+    for (;;) {
+      if (seq >= win.base && seq < win.base + 64) {
+        end_tiles = win.End(seq, 0);
+        end_live = win.End(seq, 1) - end_tiles;
+        seq_tiles = win.Tiles(seq);
+      }
+      const int here = win.CommonTiles();
+      if (here != 0) common_tiles = common_tiles == 0 || common_tiles == here ? here : -1;
+      if (win.base + 64 >= a.batch) break;
+      win.Next(a, lane);
     }
-    const int here = win.CommonTiles();
-    if (here != 0) common_tiles = common_tiles == 0 || common_tiles == here ? here : -1;
-    if (win.base + 64 >= a.batch) break;
-    win.Next(a, lane);
+    if (seq_tiles != 0) {
+      const Cut cut = MakeCut(a, win.EndTiles(), win.EndLive(), common_tiles, a.work_groups);
+      const int seq_end = end_tiles + cut.pad * end_live;
+      first_unit = (seq_end - seq_tiles) / cut.tiles_per_unit;
+      partials = (seq_end - 1) / cut.tiles_per_unit - first_unit + 1;
+    }
   }
-  if (seq_tiles == 0) return;  // (as is all below, the same for the whole workgroup)
-  const Cut cut = MakeCut(a, win.EndTiles(), win.EndLive(), common_tiles, a.work_groups);
-  const int seq_end = end_tiles + cut.pad * end_live;
-  const int first_unit = (seq_end - seq_tiles) / cut.tiles_per_unit;
-  const int partials = (seq_end - 1) / cut.tiles_per_unit - first_unit + 1;
-  if (partials == 1) return;  // written by the workgroup that held the whole sequence
-  MergeState state;
-  if (has_head) TakePartials<false>(a, z, h, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
   if constexpr (WAYS > 1) {
+    if (wave == 0 && lane == 0) {
+      cut_lds[0] = first_unit;
+      cut_lds[1] = partials;
+    }
+    __syncthreads();
+    first_unit = Uniform(cut_lds[0]);
+    partials = Uniform(cut_lds[1]);
+  }
+  if (partials <= 1) return;  // empty, or written by the workgroup that held the whole sequence
+  constexpr int kSharedPartials = WAYS == 8 ? 9 : 17;  // from here on all waves of a head have work worth sharing
+  int h = group * kMergeHeads + wave;
+  MergeState state;
+  if (WAYS == 1 || partials < kSharedPartials) {
+    if (h >= heads_here) return;
+    TakePartials<false>(a, z, h, a.max_units + seq, first_unit, 0, 1, partials, lane, state);
+  } else if constexpr (WAYS > 1) {
+    h = group * (kMergeHeads / WAYS) + wave / WAYS;
+    const int way = wave % WAYS;
+    const bool has_head = h < heads_here;
+    if (has_head) TakePartials<false>(a, z, h, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
     if (way != 0 && has_head) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) shared_acc[wave][j][lane] = state.acc[j];
@@ -1601,11 +1632,11 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
   FinishHead<MXQ>(a, z, seq, h, lane, state);
 }
 
-// Waves per head of the second-launch merge, from the partials a sequence has on average. Measured,
-// append + attention + merge of a layer at 64 heads with one wave per head / with the choice below:
-// 256 partials per sequence (1 x 32000 tokens) 59.5 / 28.0 us, 64 (4 x 8000) 32.5 / 26.0, 32 (8 x 4000)
-// 28.1 / 25.3, 21 (12 x 3000) 27.5 / 26.3, 16 (16 x 4096) 32.5 / 32.0, 12 (20 x 4000) 38.1 / 37.7. At 8
-// (32 x 2048) two waves per head took 6.2 us where one takes 5.9: a head's rows fit one group of loads.
+// Waves per head of the second-launch merge, from the partials a sequence may have on average (those that it has
+// decide in the kernel). Measured, append + attention + merge of a layer at 64 heads with one wave per head / with
+// the choice below: 256 partials per sequence (1 x 32000 tokens) 59.5 / 28.0 us, 64 (4 x 8000) 32.5 / 26.0,
+// 32 (8 x 4000) 28.1 / 25.3, 21 (12 x 3000) 27.5 / 26.3. At 8 (32 x 2048) two waves per head took 6.2 us where
+// one takes 5.9: a head's rows fit one group of loads.
 int MergeWays(const AttnArgs& a) {
   const int partials = a.max_units / std::max(a.batch, 1);
   return partials >= 32 ? 8 : (partials >= 12 ? 4 : 1);
@@ -1614,7 +1645,8 @@ int MergeWays(const AttnArgs& a) {
 template <bool MXQ, bool SPARSE>
 hipError_t LaunchMerge(const AttnArgs& args, int head_groups, hipStream_t stream) {
   const int ways = MergeWays(args), heads_per_block = kMergeHeads / ways;
-  const dim3 grid((std::min(64, args.heads) + heads_per_block - 1) / heads_per_block, args.batch, head_groups), block(kMergeHeads * 64);
+  const unsigned groups = (std::min(64, args.heads) + heads_per_block - 1) / heads_per_block, batch = args.batch;
+  const dim3 grid(ways == 1 ? groups : batch, ways == 1 ? batch : groups, head_groups), block(kMergeHeads * 64);
   switch (ways) {
     case 8: hipLaunchKernelGGL((MlaMergeKernel<MXQ, SPARSE, 8>), grid, block, 0, stream, args); break;
     case 4: hipLaunchKernelGGL((MlaMergeKernel<MXQ, SPARSE, 4>), grid, block, 0, stream, args); break;

@@ -57,6 +57,21 @@ def test_merge_with_several_waves_per_head(ctxs, heads, fp8):
         _check(cache, table, ctxs, heads, seed=905, fp8=fp8, **options)
 
 
+# The same merge in plans made for longer contexts, as a server's are: how many waves share a head goes by the
+# partials that a sequence has. Up to eight waves from 9 partials on (1000 and 1100 tokens in units of 128: 8 and 9),
+# up to four from 17 (2000 and 2100 tokens of twelve sequences: 16 and 17), sequences with nothing to merge, second
+# head groups that leave waves without a head (80 and 112 heads).
+@pytest.mark.parametrize("ctxs,heads,fp8,capacity", [([1000, 1100, 90], 64, False, 32768), ([896, 900, 1152, 1160], 112, True, 16384),
+                                                     ([2000, 2100] * 6, 64, False, 8192), ([30, 0, 600], 48, True, 4096),
+                                                     ([700, 2300, 33] * 4, 80, True, 8192)])
+def test_merge_in_plans_of_longer_contexts(ctxs, heads, fp8, capacity):
+    cache, table = _cache(ctxs, 64, seed=991, fp8=fp8)
+    wide = np.zeros((len(ctxs), capacity // 64), dtype=table.dtype)
+    wide[:, :table.shape[1]] = table
+    for options in ({"selection_units": 1}, {"chunk_tiles": 2}, {"chunk_tiles": 4}):
+        _check(cache, wide, ctxs, heads, seed=995, fp8=fp8, max_seq_len=capacity, **options)
+
+
 # Units of 16 heads shared by four workgroups (whole contexts and selections of 257 tokens and more while four
 # per unit fit the 256 CUs): fewer tiles than workgroups, shares of different sizes, the last batch
 # that fits (16 x 64 heads) and the first that is shared by two (17).
