@@ -342,20 +342,19 @@ __device__ __forceinline__ void FindBin(int* counters, int* totals, int wanted, 
 // crowd into a few exponents, so one histogram is a handful of hot counters: with 32 copies, lane L
 // counting in copy L % 32, the 64 lanes of an addition meet at most in pairs and never in a bank.
 // Up to 8192 keys the copies cost more than the counters they relieve, and half of the threads is
-// enough. Index key append, indexer and attention (16 heads) of a layer, 32 sequences, 1024 threads with 32 copies /
+// enough: those sequences are done so whatever the launch is made for, by the first half of the
+// workgroup where it is a large one (32 sequences of 2000 tokens in a launch made for 32768: indexer
+// 21.9 us with 1024 threads and 32 copies, 20.2 so, 21.1 with one histogram). Index key append, indexer and attention (16 heads) of a layer, 32 sequences, 1024 threads with 32 copies /
 // with 8 copies / 512 with 8 / 256 with 8, us: 500 tokens 22.5 / 22.0 / 20.7 / 20.5; 2000: 24.4 / 24.1 / 22.6 /
 // 22.3; 4000: 26.8 / 26.3 / 25.1 / 25.5; 8192: 27.8 / 27.7 / 26.8 / -.
 // Measured, top 512 of 8192 keys (32 sequences) and top 2048 of up to 32768 (9 sequences):
 // 5.8 -> 5.7 us and 18.7 -> 10.3 us against one histogram and passes of 8192 keys that re-read the later
 // ones in every step. (A separate path without the per-key end tests measured the same.)
+// counters: copy c of bin b at COPIES b + c; totals: one per byte, so that no barrier separates the rounds.
 template <int THREADS, int COPIES>
-__global__ __launch_bounds__(THREADS) void IndexerSelectKernel(IndexerArgs a) {
+__device__ __forceinline__ void SelectSequence(const IndexerArgs& a, int n, int* counters, int (*totals)[256], unsigned* wave_counts) {
   constexpr int kWaves = THREADS / 64, kKeysPerPiece = THREADS * 8;
-  __shared__ __attribute__((aligned(16))) int counters[256 * COPIES];  // copy c of bin b at COPIES b + c
-  __shared__ __attribute__((aligned(16))) int totals[2][256];  // one per byte, so that no barrier separates the rounds
-  __shared__ unsigned wave_counts[kWaves];
   const int seq = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n = max(min(a.seq_lens[seq], a.max_seq_len), 0);
   const int k = a.sparse_count;
   int32_t* out = a.indices_out + seq * a.indices_seq_stride;
   if (n <= k) {
@@ -472,6 +471,22 @@ __global__ __launch_bounds__(THREADS) void IndexerSelectKernel(IndexerArgs a) {
   }
 }
 
+// LONG: made for more than 8192 tokens.
+template <bool LONG>
+__global__ __launch_bounds__(LONG ? kSelectThreads : kShortThreads) void IndexerSelectKernel(IndexerArgs a) {
+  constexpr int kCounters = 256 * (LONG ? kSelectCopies : kShortCopies), kWaves = (LONG ? kSelectThreads : kShortThreads) / 64;
+  __shared__ __attribute__((aligned(16))) int counters[kCounters];
+  __shared__ __attribute__((aligned(16))) int totals[2][256];
+  __shared__ unsigned wave_counts[kWaves];
+  const int n = max(min(a.seq_lens[blockIdx.x], a.max_seq_len), 0);
+  if (!LONG || n <= kShortKeys) {
+    if (LONG && threadIdx.x >= kShortThreads) return;  // whole waves: the barriers wait for those that are left
+    SelectSequence<kShortThreads, kShortCopies>(a, n, counters, totals, wave_counts);
+  } else if constexpr (LONG) {
+    SelectSequence<kSelectThreads, kSelectCopies>(a, n, counters, totals, wave_counts);
+  }
+}
+
 // Index-key append: sixteen lanes per token (eight bf16 values each), four tokens per wavefront.
 // The row's absmax by four lane exchanges, scale = absmax / 448, codes from the correctly rounded
 // quotient (the E4M3 conversion saturates behind a clamp to +-448).
@@ -541,7 +556,7 @@ hipError_t PrepareIndexerKernels() {
   for (const hipError_t e : results) {
     if (e != hipSuccess) return e;
   }
-  for (const void* kernel : {reinterpret_cast<const void*>(&IndexerSelectKernel<kShortThreads, kShortCopies>), reinterpret_cast<const void*>(&IndexerSelectKernel<kSelectThreads, kSelectCopies>),
+  for (const void* kernel : {reinterpret_cast<const void*>(&IndexerSelectKernel<false>), reinterpret_cast<const void*>(&IndexerSelectKernel<true>),
                              reinterpret_cast<const void*>(&IndexKeyAppendKernel)}) {
     hipFuncAttributes attributes;
     if (hipError_t e = hipFuncGetAttributes(&attributes, kernel); e != hipSuccess) return e;
@@ -573,9 +588,9 @@ hipError_t LaunchIndexer(const IndexerArgs& args, hipStream_t stream) {
     if (e != hipSuccess) return e;
   }
   if (args.max_seq_len <= kShortKeys) {
-    hipLaunchKernelGGL((IndexerSelectKernel<kShortThreads, kShortCopies>), dim3(args.batch), dim3(kShortThreads), 0, stream, args);
+    hipLaunchKernelGGL(IndexerSelectKernel<false>, dim3(args.batch), dim3(kShortThreads), 0, stream, args);
   } else {
-    hipLaunchKernelGGL((IndexerSelectKernel<kSelectThreads, kSelectCopies>), dim3(args.batch), dim3(kSelectThreads), 0, stream, args);
+    hipLaunchKernelGGL(IndexerSelectKernel<true>, dim3(args.batch), dim3(kSelectThreads), 0, stream, args);
   }
   return hipGetLastError();
 }

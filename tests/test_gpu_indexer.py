@@ -148,10 +148,10 @@ def test_index_key_append_matches_the_oracle_quantiser(bs):
     assert lib.mlakvIndexKeyAppend(C.byref(view), rows_d.data_ptr(), D * 2, slots_d.data_ptr(), 0, kt.stream_ptr()) == 0
 
 
-# Launches up to 8192 keys: 512 threads with one piece of eight keys up to 4096 keys, two beyond. Longer
-# ones: 1024 threads, one piece up to 8192 keys, four up to 32768, sweeps of 32768 beyond. The
-# edges of each, a last piece that is not full, selections that end inside a run of equal keys.
-@pytest.mark.parametrize("seq_lens,k", [([4095, 4096, 4097, 8192], 700), ([513, 64, 7], 7), ([8191, 8192, 8193], 2048), ([16384, 16385, 24577], 700), ([32761, 32768, 32769], 2048),
+# Sequences up to 8192 keys: 512 threads with one piece of eight keys up to 4096 keys, two beyond, in launches made for
+# more than 8192 tokens as well. Longer ones: 1024 threads, two to four pieces up to 32768 keys, sweeps of 32768
+# beyond. The edges of each, a last piece that is not full, selections that end inside a run of equal keys.
+@pytest.mark.parametrize("seq_lens,k", [([4095, 4096, 4097, 8192], 700), ([513, 64, 7], 7), ([8191, 8192, 8193], 2048), ([600, 20000, 2000, 513, 8192, 4097, 8193], 512), ([16384, 16385, 24577], 700), ([32761, 32768, 32769], 2048),
                                         ([2, 70001], 1)])
 def test_selection_at_the_edges_of_pieces_and_sweeps(seq_lens, k):
     _run(seq_lens, 64, 16, k, seed=140)
