@@ -754,16 +754,22 @@ hipError_t LaunchNormRopeAppendAs(const NormRopeAppendArgs& args, hipStream_t st
 }  // namespace
 
 // Without query heads two rows per wavefront. With them a wavefront of its own for every eight heads
-// while those are few (up to two per SIMD): the launch is one chain of loads and arithmetic then, and
-// 32 heads in a wavefront make it longer (200 tokens of 64 heads, FP8 cache: 3.57
-// against 3.75 us; 700 tokens of 32 heads 4.32 against 3.95).
+// where there are no more, or while the wavefronts are few: the launch is one chain of loads and
+// arithmetic then, and 32 heads in a wavefront make it longer. Few are 2048 beside the quantising append of an
+// FP8 cache, itself a long chain, and where two groups of heads are all there is; beside the copy of a bf16 row
+// the heads are the longest chain, and a wavefront for eight of them is ahead up to 3840, or 5120 where the
+// last of 32 would hold eight. Measured, eight / 32 heads per wavefront, us (waves at eight): FP8, 200 tokens
+// of 64 heads (1800) 3.40 / 3.36, 700 of 32 (3500) 4.24 / 3.87, 400 of 64 (3600) 4.05 / 3.85, 4096 of 8 5.89 / 6.21;
+// bf16, 700 of 16 (2100) 3.16 / 2.93, 400 of 48 (2800) 3.18 / 3.46, 400 of 64 (3600) 3.43 / 3.56, 1000 of 24 (4000)
+// 3.53 / 3.28, 700 of 40 (4200) 3.63 / 3.79, 850 of 40 (5100) 3.86 / 4.10, 600 of 64 (5400) 4.09 / 3.83.
 hipError_t LaunchNormRopeAppend(const NormRopeAppendArgs& args, hipStream_t stream) {
   if (args.append.num_tokens <= 0) return hipSuccess;
   constexpr int kRowsAlone = 2;
   if (args.q_rope == nullptr || args.num_heads <= 0) return LaunchNormRopeAppendAs<kRowsAlone, 1>(args, stream);
-  constexpr int64_t kFewWaves = 2048;
-  const int64_t waves = static_cast<int64_t>(args.append.num_tokens) * (1 + DivUp(args.num_heads, kQueryHeadsPerGroup));
-  return waves <= kFewWaves ? LaunchNormRopeAppendAs<1, 1>(args, stream) : LaunchNormRopeAppendAs<1, kQueryGroups>(args, stream);
+  const int groups = DivUp(args.num_heads, kQueryHeadsPerGroup);
+  const int64_t few = args.append.fp8 || groups <= 2 ? 2048 : (groups % kQueryGroups == 1 ? 5120 : 3840);
+  const int64_t waves = static_cast<int64_t>(args.append.num_tokens) * (1 + groups);
+  return groups == 1 || waves <= few ? LaunchNormRopeAppendAs<1, 1>(args, stream) : LaunchNormRopeAppendAs<1, kQueryGroups>(args, stream);
 }
 
 namespace {

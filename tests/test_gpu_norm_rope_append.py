@@ -169,13 +169,16 @@ def test_query_rope_slices_rotate_in_place_with_the_key(heads):
     assert np.array_equal(cache.rope_np(0), rope_plane.reshape(-1))
 
 
-# 2048 wavefronts with eight heads each at most, 32 heads each beyond: both sides of the line, head
-# counts that leave a wavefront part of its heads, values so small that the products are subnormal
-# (bf16 keeps 7 bits of them: the bound is one bf16 step or one step of the subnormal grid).
-@pytest.mark.parametrize("tokens,heads", [(1024, 1), (1025, 1), (409, 32), (410, 32), (410, 33), (700, 9), (300, 100), (1, 128)])
-def test_query_heads_on_both_sides_of_the_split(tokens, heads):
+# 3840 wavefronts with eight heads each at most (5120 where 32 each would leave eight for the last, 2048 for an FP8
+# cache and for up to 16 heads), 32 heads each beyond, eight where there are no more: both sides of each line, head counts that leave a wavefront
+# part of its heads, values so small that the products are subnormal (bf16 keeps 7 bits of them: the
+# bound is one bf16 step or one step of the subnormal grid).
+@pytest.mark.parametrize("tokens,heads,fp8", [(1024, 1, False), (1025, 1, False), (4000, 8, True), (409, 32, True), (410, 32, True),
+                                              (410, 33, True), (700, 9, False), (682, 16, False), (683, 16, False), (768, 32, False),
+                                              (769, 32, False), (300, 100, True), (853, 40, False), (854, 40, False), (1, 128, False)])
+def test_query_heads_on_both_sides_of_the_split(tokens, heads, fp8):
     bs, max_pos = 64, 128
-    cache = kt.PagedCache(1, -(-tokens // bs), bs)
+    cache = kt.PagedCache(1, -(-tokens // bs), bs, fp8=fp8)
     lib = ffi.load()
     kv_d = kt.randn_bf16((tokens, LATENT + ROPE), seed=41).cuda()
     q = kt.randn_bf16((tokens, heads, ROPE), seed=42)
