@@ -743,12 +743,9 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
       // The units have no quantising epilogue: they write bf16 rows (the caller's, or rows of the
       // workspace behind the parts' partials) and the standalone quantiser follows in the same
       // stream; its codes are those of the fused epilogue, by construction of both from the bf16 rows.
-      const auto partials_end = [&]() { return args.head_block_units > 1 ? ((partial_bytes() + 255) & ~255ull) : 0; };
+      const uint64_t rows_offset = args.head_block_units > 1 ? ((partial_bytes() + 255) & ~255ull) : 0;
       const uint64_t rows_bytes = static_cast<uint64_t>(plan->batch) * plan->heads * mlakv::kLatentDim * 2;
       const bool own_rows = out == nullptr;
-      // (four parts only where the rows fit behind their partials as well)
-      if (own_rows && args.head_block_units == 4 && partials_end() + rows_bytes > plan->workspace_bytes) args.head_block_units = 2;
-      const uint64_t rows_offset = partials_end();
       const bool uniform = (own_rows || out_seq_stride == plan->heads * out_head_stride) &&
                            quant->codes_seq_stride == plan->heads * quant->codes_head_stride &&
                            quant->scales_seq_stride == plan->heads * quant->scales_head_stride;
