@@ -1522,22 +1522,26 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
 }
 
 // The merge as a launch of its own, for launches that have no counters to meet on: block =
-// (8 / WAYS heads, sequence, head group). WAYS waves share a head, wave w of them takes partials w,
-// w + WAYS, ..., and the first adds up what they hold through LDS. What bounds it is the chain of
-// memory trips (lengths, then a group of eight rows at a time) and how many rows are on their way at once:
-// one wave per head leaves a launch of few sequences with few waves and many partials each. Measured (64
-// heads, FP8, 3 sequences of 15k to 33k tokens, about 85 partials per head): 18.6 us with one wave per
-// head, 6.9 us with eight.
-// The launch is made for the partials that the plan allows. A sequence that has fewer is merged by one wave per
-// head in the first workgroups, and the others leave: up to eight partials are one group of loads
-// for a wave, and more waves would only load the same rows. Measured, attention + merge of a layer in a
-// plan of 32768 tokens, one wave / all: eight waves per head, 1 x 1000 tokens (8 partials) 16.6 / 17.0 us, 1 x
-// 1100 (9) 17.4 / 16.6, 4 x 1200 (10) 18.8 / 17.9; four, where the chip is fuller, 20 x 4000 (12) 29.8 / 31.2, 16
-// x 2000 (14) 22.2 / 22.6, 12 x 2000 (17) 20.8 / 21.1, 12 x 3000 (25) 23.7 / 22.7.
+// (8 / WAYS heads, sequence). WAYS waves share a head, wave w of them takes partials w, w + WAYS, ...,
+// and the first adds up what they hold through LDS. What bounds it is the chain of memory trips
+// (lengths, then a group of eight rows at a time) and how many rows are on their way at once: one wave
+// per head leaves a launch of few sequences with few waves and many partials each. Measured (64 heads,
+// FP8, 3 sequences of 15k to 33k tokens, about 85 partials per head): 18.6 us with one wave per head,
+// 6.9 us with eight.
+// The launch is made for the partials that the plan allows. A sequence that has fewer is merged by one
+// wave per head in the first workgroups, and the others leave: up to eight partials are one group
+// of loads for a wave, and more waves would only load the same rows. Where one wave per head is already
+// more than a wave for every SIMD (1024), more of them pay only from the fourth group on. Measured,
+// append, attention and merge of a layer, us (partials of a sequence), up to 8 / 16 / 24 of them by one wave: 6
+// x 900..2600 tokens of 128 heads (6 to 17) 24.0 / 25.1 / -, 10 x 700..2500 of 48 (6 to 21) 22.9 / 23.4 / -, 14 x
+// 2000 of 64 (17) 25.4 / 26.2 / -, 9 x 1400 of 64 (12) 25.0 / 24.3 / -, 16 x 2000 of 64 (14) 26.3 / 26.0 / -; 20 x
+// 2000..5000 of 64 (7 to 19) 34.8 / 35.6 / 34.5, 20 x 4000 of 64 (12) 38.9 / 37.6 / 37.5, 18 x 1000..6000 of 96,
+// FP8 (4 to 25), - / 44.1 / 41.9. (With up to 24 by one wave 9 x 800..3000 of 64 take 26.5, up to 8 25.4.)
 // So that the surplus costs little, one wave repeats the cut of the flat tile axis for its workgroup
 // (20 x 32 tokens, nothing to merge: 12.5 us with every wave, 11.4 so), and where waves share heads
-// all first workgroups of the sequences come before any second (with a sequence's workgroups side by
-// side those with work sat on an eighth or a quarter of the CUs: 20 x 200 tokens 19.5 us, 17.8 so).
+// all first workgroups of the sequences come before any second, those of all heads: with a sequence's
+// workgroups side by side those with work sat on an eighth or a quarter of the CUs (20 x 200 tokens
+// 19.5 us, 17.8 so), with those of heads 64 to 127 at the end they began late (9 x 800..3000 of 128 28.1 / 26.1).
 template <bool MXQ, bool SPARSE, int WAYS>
 __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
   __shared__ float shared_acc[WAYS > 1 ? kMergeHeads : 1][8][64];
@@ -1547,16 +1551,18 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
   // Workgroups go to the XCDs round-robin by linear id. The main launch put the units of XCD x's
   // share of the flat tile axis on XCD x; with equal lengths that is the x-th eighth of the
   // sequences, whose partials are most likely still in that L2.
-  const int groups = WAYS == 1 ? gridDim.x : gridDim.y, batch = WAYS == 1 ? gridDim.y : gridDim.x;
-  const int linear = blockIdx.y * gridDim.x + blockIdx.x, z = blockIdx.z;
-  int seq = WAYS == 1 ? blockIdx.y : blockIdx.x, group = WAYS == 1 ? blockIdx.x : blockIdx.y;
-  if ((batch & (kXcds - 1)) == 0) {
-    const int within = linear / kXcds, share = batch / kXcds;
-    seq = (linear & (kXcds - 1)) * share + (WAYS == 1 ? within / groups : within % share);
-    group = WAYS == 1 ? within % groups : within / share;
+  int seq, group;
+  if constexpr (WAYS == 1) {
+    seq = blockIdx.y, group = blockIdx.x;
+    if ((gridDim.y & (kXcds - 1)) == 0) {
+      const int linear = blockIdx.y * gridDim.x + blockIdx.x, within = linear / kXcds;
+      seq = (linear & (kXcds - 1)) * (gridDim.y / kXcds) + within / static_cast<int>(gridDim.x);
+      group = within % static_cast<int>(gridDim.x);
+    }
+  } else {
+    seq = blockIdx.x, group = blockIdx.y;
+    if ((gridDim.x & (kXcds - 1)) == 0) seq = (blockIdx.x & (kXcds - 1)) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
   }
-  const int heads_here = min(64, a.heads - 64 * z);
-  if (WAYS == 1 && group * kMergeHeads + wave >= heads_here) return;
   int first_unit = 0, partials = 0;
   if (WAYS == 1 || wave == 0) {
     SeqWindow<SPARSE> win;
@@ -1590,18 +1596,17 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
     partials = Uniform(cut_lds[1]);
   }
   if (partials <= 1) return;  // empty, or written by the workgroup that held the whole sequence
-  constexpr int kSharedPartials = WAYS == 8 ? 9 : 17;  // from here on all waves of a head have work worth sharing
+  const int shared_from = a.batch * a.heads <= 1024 ? 9 : 25;  // partials
   int h = group * kMergeHeads + wave;
   MergeState state;
-  if (WAYS == 1 || partials < kSharedPartials) {
-    if (h >= heads_here) return;
-    TakePartials<false>(a, z, h, a.max_units + seq, first_unit, 0, 1, partials, lane, state);
+  if (WAYS == 1 || partials < shared_from) {
+    if (h >= a.heads) return;
+    TakePartials<false>(a, h >> 6, h & 63, a.max_units + seq, first_unit, 0, 1, partials, lane, state);
   } else if constexpr (WAYS > 1) {
     h = group * (kMergeHeads / WAYS) + wave / WAYS;
     const int way = wave % WAYS;
-    const bool has_head = h < heads_here;
-    if (has_head) TakePartials<false>(a, z, h, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
-    if (way != 0 && has_head) {
+    TakePartials<false>(a, h >> 6, h & 63, a.max_units + seq, first_unit, way, WAYS, partials, lane, state);
+    if (way != 0) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) shared_acc[wave][j][lane] = state.acc[j];
       if (lane == 0) {
@@ -1610,7 +1615,7 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
       }
     }
     __syncthreads();
-    if (way != 0 || !has_head) return;
+    if (way != 0) return;
     float top = state.m;
 #pragma unroll
     for (int w = 1; w < WAYS; ++w) top = __builtin_elementwise_maximum(top, shared_ends[wave + w][0]);
@@ -1629,7 +1634,7 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
       }
     }
   }
-  FinishHead<MXQ>(a, z, seq, h, lane, state);
+  FinishHead<MXQ>(a, h >> 6, seq, h & 63, lane, state);
 }
 
 // Waves per head of the second-launch merge, from the partials a sequence may have on average (those that it has
@@ -1643,10 +1648,10 @@ int MergeWays(const AttnArgs& a) {
 }
 
 template <bool MXQ, bool SPARSE>
-hipError_t LaunchMerge(const AttnArgs& args, int head_groups, hipStream_t stream) {
-  const int ways = MergeWays(args), heads_per_block = kMergeHeads / ways;
-  const unsigned groups = (std::min(64, args.heads) + heads_per_block - 1) / heads_per_block, batch = args.batch;
-  const dim3 grid(ways == 1 ? groups : batch, ways == 1 ? batch : groups, head_groups), block(kMergeHeads * 64);
+hipError_t LaunchMerge(const AttnArgs& args, hipStream_t stream) {
+  const int ways = MergeWays(args);
+  const unsigned groups = args.heads * ways / kMergeHeads, batch = args.batch;  // (heads come in sixteens)
+  const dim3 grid = ways == 1 ? dim3(groups, batch) : dim3(batch, groups), block(kMergeHeads * 64);
   switch (ways) {
     case 8: hipLaunchKernelGGL((MlaMergeKernel<MXQ, SPARSE, 8>), grid, block, 0, stream, args); break;
     case 4: hipLaunchKernelGGL((MlaMergeKernel<MXQ, SPARSE, 4>), grid, block, 0, stream, args); break;
@@ -2445,8 +2450,8 @@ hipError_t LaunchAttnDecode(const AttnArgs& args_in, hipStream_t stream) {
   }
   if (e != hipSuccess || merge_in_launch) return e;
   if (!AnySequenceSplit(args)) return hipSuccess;  // every sequence is written by the one unit that holds it
-  if (sparse) return LaunchMerge<false, true>(args, head_groups, stream);
-  return quantise ? LaunchMerge<true, false>(args, head_groups, stream) : LaunchMerge<false, false>(args, head_groups, stream);
+  if (sparse) return LaunchMerge<false, true>(args, stream);
+  return quantise ? LaunchMerge<true, false>(args, stream) : LaunchMerge<false, false>(args, stream);
 }
 
 // Split-KV partials for callers that cannot allocate: one array per GPU, held from module load to

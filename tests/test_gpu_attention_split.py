@@ -47,7 +47,7 @@ def _check(cache, table, ctxs, heads, seed, fp8=False, sparse=None, **options):
 
 # Partials per sequence on average (256 units on a full chip): 85 (eight waves per head in the merge),
 # 36 with 128 heads in two groups, 19 and 12 (four), 10 (one); empty sequences and sequences of one
-# unit among them, head counts that leave waves of the merge without a head.
+# unit among them.
 @pytest.mark.parametrize("ctxs,heads,fp8", [([3000, 1, 1900], 64, True), ([900, 2100, 40], 128, False), ([4096], 16, False),
                                             ([300] * 12 + [0], 48, False), ([130] * 21, 64, True), ([200] * 24 + [1700], 32, False)])
 def test_merge_with_several_waves_per_head(ctxs, heads, fp8):
@@ -58,18 +58,30 @@ def test_merge_with_several_waves_per_head(ctxs, heads, fp8):
 
 
 # The same merge in plans made for longer contexts, as a server's are: how many waves share a head goes by the
-# partials that a sequence has. Up to eight waves from 9 partials on (1000 and 1100 tokens in units of 128: 8 and 9),
-# up to four from 17 (2000 and 2100 tokens of twelve sequences: 16 and 17), sequences with nothing to merge, second
-# head groups that leave waves without a head (80 and 112 heads).
+# partials that a sequence has, several from 9 partials on (1000 and 1100 tokens in units of 128: 8 and 9), with more
+# than 1024 heads in the batch from 25 (1500 and 1620 tokens in units of 64: 24 and 26). Sequences with nothing to
+# merge among them, and second head groups of 16 and 48 heads (80 and 112 in all).
 @pytest.mark.parametrize("ctxs,heads,fp8,capacity", [([1000, 1100, 90], 64, False, 32768), ([896, 900, 1152, 1160], 112, True, 16384),
                                                      ([2000, 2100] * 6, 64, False, 8192), ([30, 0, 600], 48, True, 4096),
-                                                     ([700, 2300, 33] * 4, 80, True, 8192)])
+                                                     ([700, 2300, 33] * 4, 80, True, 8192),
+                                                     ([1500, 1620, 300, 2600] * 5, 64, False, 8192)])
 def test_merge_in_plans_of_longer_contexts(ctxs, heads, fp8, capacity):
     cache, table = _cache(ctxs, 64, seed=991, fp8=fp8)
     wide = np.zeros((len(ctxs), capacity // 64), dtype=table.dtype)
     wide[:, :table.shape[1]] = table
     for options in ({"selection_units": 1}, {"chunk_tiles": 2}, {"chunk_tiles": 4}):
         _check(cache, wide, ctxs, heads, seed=995, fp8=fp8, max_seq_len=capacity, **options)
+
+
+# Rows that grow or fall along the context: the reference maxima of a head's waves lie far apart, and the weights of
+# whole partials vanish beside those of others. Eight, four and one wave per head.
+@pytest.mark.parametrize("rising", [True, False])
+@pytest.mark.parametrize("ctxs,heads,fp8", [([3000, 5000], 64, False), ([2000, 600] * 6, 64, True), ([1500] * 24, 16, False)])
+def test_merge_of_partials_with_unequal_weights(ctxs, heads, fp8, rising):
+    longest = max(ctxs)
+    cache, table = _cache(ctxs, 64, seed=985, fp8=fp8, grow=lambda at: 0.1 + 4.0 * (at if rising else longest - at) / longest)
+    for options in ({"selection_units": 1}, {"chunk_tiles": 2}):
+        _check(cache, table, ctxs, heads, seed=987, fp8=fp8, **options)
 
 
 # Units of 16 heads shared by four workgroups (whole contexts and selections of 257 tokens and more while four
