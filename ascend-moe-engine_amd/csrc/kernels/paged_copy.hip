@@ -362,7 +362,7 @@ __global__ __launch_bounds__(kThreads) void AppendFp8Kernel(AppendArgs a, WORDS 
 // wavefront share one pair of table loads (a memory latency behind the position's) and its
 // conversions. Measured, 2029 tokens of 64 heads with an FP8 cache: 10.4 us with a
 // wavefront, and table loads, per eight heads and shuffles for the partner, 8.0 us with 32 heads.
-constexpr int kQueryHeadsPerGroup = 8, kQueryGroups = 4;
+constexpr int kQueryHeadsPerGroup = 8, kQueryGroups = 4, kQueryGroupsApart = 2;
 
 __device__ __forceinline__ unsigned FourLanesAway(unsigned x) {  // lane ^ 7, then lane ^ 3
   const int mirrored = __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x141, 0xf, 0xf, false);     // row_half_mirror
@@ -375,6 +375,8 @@ __device__ __forceinline__ void RotateQueryHeads(const NormRopeAppendArgs& n, in
   const int head = head0 + (lane >> 3);
   const int part = lane & 7;
   const int position = Uniform(n.positions[token]);
+  // (launches of 16 heads per wavefront: nothing is asked for before the position is there, see LaunchNormRopeAppend)
+  if constexpr (GROUPS == kQueryGroupsApart) asm volatile("" : : "s"(position) : "memory");
   char* q = n.q_rope + token * n.q_rope_token_stride + head * n.q_rope_head_stride + part * 16;
   u32x4 qv[GROUPS];
 #pragma unroll
@@ -398,7 +400,7 @@ __device__ __forceinline__ void RotateQueryHeads(const NormRopeAppendArgs& n, in
     u32x4 out;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const unsigned pv = FourLanesAway(qv[k][i]);
+      const unsigned pv = GROUPS == kQueryGroupsApart ? __shfl_xor(qv[k][i], 4) : FourLanesAway(qv[k][i]);
       const float x0 = Bf16ToF32(qv[k][i] & 0xffffu), x1 = __builtin_bit_cast(float, qv[k][i] & 0xffff0000u);
       const float p0 = Bf16ToF32(pv & 0xffffu), p1 = __builtin_bit_cast(float, pv & 0xffff0000u);
       out[i] = PackBf16Pair(x0 * c[2 * i] + p0 * s[2 * i], x1 * c[2 * i + 1] + p1 * s[2 * i + 1]);
@@ -762,6 +764,12 @@ hipError_t LaunchNormRopeAppendAs(const NormRopeAppendArgs& args, hipStream_t st
 // of 64 heads (1800) 3.40 / 3.36, 700 of 32 (3500) 4.24 / 3.87, 400 of 64 (3600) 4.05 / 3.85, 4096 of 8 5.89 / 6.21;
 // bf16, 700 of 16 (2100) 3.16 / 2.93, 400 of 48 (2800) 3.18 / 3.46, 400 of 64 (3600) 3.43 / 3.56, 1000 of 24 (4000)
 // 3.53 / 3.28, 700 of 40 (4200) 3.63 / 3.79, 850 of 40 (5100) 3.86 / 4.10, 600 of 64 (5400) 4.09 / 3.83.
+// Slices that lie apart (the rope part of whole query heads, 128 of 1152 bytes) are one line each wherever they are,
+// and memory serves many of them faster the less a wavefront asks for at once: beyond 32768 wavefronts 16 heads
+// each, loaded after the position and exchanged through the LDS unit. Eight (as a launch of their own once was) / 32 /
+// 16 heads so, us: bf16, 3700 tokens of 64 heads (33300) 16.8 / 16.9 / 16.1, 8192 33.1 / 34.0 / 32.7, 32768 120.8 /
+// 125.8 / 122.7, 8192 of 128 58.7 / 60.4 / 57.6; FP8, 16384 of 64 61.4 / 63.2 / 61.2; 2000 of 64 (18000) 11.0 / 8.6 /
+// 10.2, slices next to each other, 8192 of 64 30.4 / 28.2 / 28.7 (both exchanged by lane moves).
 hipError_t LaunchNormRopeAppend(const NormRopeAppendArgs& args, hipStream_t stream) {
   if (args.append.num_tokens <= 0) return hipSuccess;
   constexpr int kRowsAlone = 2;
@@ -769,7 +777,10 @@ hipError_t LaunchNormRopeAppend(const NormRopeAppendArgs& args, hipStream_t stre
   const int groups = DivUp(args.num_heads, kQueryHeadsPerGroup);
   const int64_t few = args.append.fp8 || groups <= 2 ? 2048 : (groups % kQueryGroups == 1 ? 5120 : 3840);
   const int64_t waves = static_cast<int64_t>(args.append.num_tokens) * (1 + groups);
-  return groups == 1 || waves <= few ? LaunchNormRopeAppendAs<1, 1>(args, stream) : LaunchNormRopeAppendAs<1, kQueryGroups>(args, stream);
+  if (groups == 1 || waves <= few) return LaunchNormRopeAppendAs<1, 1>(args, stream);
+  constexpr int64_t kManyWaves = 32768;
+  if (waves > kManyWaves && args.q_rope_head_stride > kRopeDim * 2) return LaunchNormRopeAppendAs<1, kQueryGroupsApart>(args, stream);
+  return LaunchNormRopeAppendAs<1, kQueryGroups>(args, stream);
 }
 
 namespace {

@@ -200,3 +200,30 @@ def test_query_heads_on_both_sides_of_the_split(tokens, heads, fp8):
     # half a bf16 step of the result, and the fp32 rounding of two products that may cancel
     bound = 2.0 ** -8 * np.abs(want) + 2.0 ** -23 * (np.abs(x) + np.abs(np.roll(x, half, axis=-1))) + 2.0 ** -133
     assert (np.abs(q_d.double().cpu().numpy() - want) <= bound).all()
+
+
+# Slices at the end of wider heads: 32768 wavefronts with eight heads each at most (32 in each then), and beyond, 16 in
+# each; head counts that leave a wavefront part of its heads. What lies between the slices stays. Same bound as above.
+@pytest.mark.parametrize("tokens,heads,fp8", [(3640, 64, False), (3641, 64, True), (5462, 33, False), (8193, 24, False), (10923, 9, True)])
+def test_query_slices_of_wider_heads(tokens, heads, fp8):
+    bs, max_pos, wide = 64, 128, 192
+    cache = kt.PagedCache(1, -(-tokens // bs), bs, fp8=fp8)
+    kv_d = kt.randn_bf16((tokens, LATENT + ROPE), seed=51).cuda()
+    q = kt.randn_bf16((tokens, heads, wide), seed=52)
+    q_d, gamma_d = q.cuda(), torch.ones(LATENT, dtype=torch.bfloat16, device="cuda")
+    cos, sin = _tables(max_pos)
+    cos_d, sin_d = cos.cuda(), sin.cuda()
+    positions = np.random.default_rng(53).integers(0, max_pos, tokens).astype(np.int32)
+    positions_d, slots_d = kt.dev_i32(positions), kt.dev_i32(np.arange(tokens, dtype=np.int32))
+    row = (LATENT + ROPE) * 2
+    ffi.check(ffi.load().mlakvNormRopeAppend(C.byref(cache.view), 0, kv_d.data_ptr(), row, gamma_d.data_ptr(), EPS, cos_d.data_ptr(),
+                                             sin_d.data_ptr(), ROPE * 2, positions_d.data_ptr(), slots_d.data_ptr(), tokens, None, 0,
+                                             None, 0, q_d.data_ptr() + 2 * (wide - ROPE), heads * wide * 2, wide * 2, heads, kt.stream_ptr()))
+    got = q_d.cpu()
+    assert torch.equal(got[..., :wide - ROPE], q[..., :wide - ROPE])
+    x = q[..., wide - ROPE:].double().numpy()
+    c, s = (table.double().numpy()[positions][:, None] for table in (cos, sin))
+    half = ROPE // 2
+    want = x * c + np.concatenate([-x[..., half:], x[..., :half]], axis=-1) * s
+    bound = 2.0 ** -8 * np.abs(want) + 2.0 ** -23 * (np.abs(x) + np.abs(np.roll(x, half, axis=-1))) + 2.0 ** -133
+    assert (np.abs(got[..., wide - ROPE:].double().numpy() - want) <= bound).all()
