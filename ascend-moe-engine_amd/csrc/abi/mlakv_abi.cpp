@@ -405,7 +405,8 @@ int32_t SharedUnitParts(int32_t batch, int32_t heads, int32_t tokens, int32_t dt
 // 20.8-24.0 / 15.5-18.7; 1024: 16.7-25.6 / 26.1-29.6 / 18.3-22.9. Batch 48, 64 (32 x 128): 256:
 // 21.1-22.9 / 12.0-12.8; 512: 21.3-23.9 / 17.9-20.3; 768: 23.7-26.8 / 24.4-37.5. Batch 96, 128
 // (64 x 128), two rounds of units: 256: 24.8-27.6 / 21.1-24.6; 384: 27.5-30.4 / 27.2-32.1. Batch 256:
-// 128: 29.0 / 31.8.
+// 128: 29.0 / 31.8. (The line at 768 is that of two workgroups per unit; where four fit they are ahead to 1024, append
+// included: 8 x 800 21.3 / 17.7 for the 64-head kernel / four, 8 x 1024 22.3 / 18.8, FP8 22.6 / 18.7, 16 x 1024 24.5 / 20.5.)
 int32_t ShortContextUnits(const mlakvAttnPlan* plan, int32_t bound) {
   if (plan->selection_units == MLAKV_ATTN_UNITS_SPLIT || bound > MLAKV_ATTN_HEAD_BLOCK_TOKENS) return 0;
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK) return 1;

@@ -35,7 +35,7 @@ __global__ __launch_bounds__(kThreads) void MxQuantKernel(MxQuantArgs q) {
 #pragma unroll
   for (int u = 0; u < LOADS; ++u) {
     const unsigned at = col0 + threadIdx.x + kThreads * u;
-    // rows of at least 1024 items: the workgroup's items end in the row behind the first at the latest
+    // rows of at least kItemsPerGroup items: the workgroup's items end in the row behind the first at the latest
     const unsigned ahead = items_per_row >= kItemsPerGroup ? (at >= items_per_row ? 1u : 0u) : at / items_per_row;
     row[u] = row0 + ahead;
     col[u] = at - ahead * items_per_row;

@@ -56,7 +56,7 @@ ATTENTION_TRAFFIC = {
     "attention_sparse": {"ratio": 1.320, "source": _TRAFFIC_SOURCE}, # 30.90 MB against 23.41 MB (one dispatch: halved whole-selection units)
     "attention_short": {"ratio": 1.018, "source": _TRAFFIC_SOURCE},  # 14.14 MB against 13.89 MB (one dispatch, no partials)
     "attention_sparse_fp8": {"ratio": 1.613, "source": _TRAFFIC_SOURCE}, # 22.65 MB against 14.04 MB
-    "indexer": {"ratio": 1.094, "source": _TRAFFIC_SOURCE},          # 38.24 MB against 34.96 MB
+    "indexer": {"ratio": 1.096, "source": _TRAFFIC_SOURCE},          # 38.30 MB against 34.96 MB
 }
 # Host orchestration of the reference's own 43-layer decode step (its mock build: every operator
 # launch is a no-op), measured in the build container on 8 cores: 128 steps, 132,480 launches,
