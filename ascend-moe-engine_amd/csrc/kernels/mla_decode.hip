@@ -55,6 +55,7 @@
 #include <mutex>
 #include <utility>
 
+#include "kernel_arguments.h"
 #include "kernels.h"
 
 #include <cstddef>
@@ -528,22 +529,6 @@ __device__ __forceinline__ int LiveLength(const AttnArgs& a, int seq) {
     lengths = reinterpret_cast<const int32_t*>(segment + offsetof(AttnArgs, inline_lens));
   }
   return lengths[seq];
-}
-
-// Asks for every cache line of the argument block (its inline lengths apart) and waits for them once. Read where
-// they are used, the arguments come in as many trips as there are lines met in a row, each a miss of the scalar
-// cache at the start of a launch. In the units of 16 heads, whose workgroups are one chain of latencies: 1 x 129
-// tokens of 64 heads 10.4 -> 9.9 us a layer with its append, 7 x 40..600 of 128 recorded 15.8 -> 15.2, 32 x 512
-// selected of 8192 36.3 -> 35.3. Not in the split units (32 x 2048 tokens with it 32.9, without 32.2) nor their merge
-// (32.8): they get by with fewer lines, and every line more delays them all.
-__device__ __forceinline__ void TouchArguments() {
-  const __attribute__((address_space(4))) unsigned* words = (const __attribute__((address_space(4))) unsigned*)__builtin_amdgcn_kernarg_segment_ptr();
-  constexpr int kLines = (offsetof(AttnArgs, inline_lens) + 63) / 64;
-  unsigned seen[kLines];
-#pragma unroll
-  for (int i = 0; i < kLines; ++i) seen[i] = words[16 * i];
-#pragma unroll
-  for (int i = 0; i < kLines; ++i) asm volatile("" ::"s"(seen[i]));
 }
 
 template <bool SPARSE>
@@ -1738,7 +1723,10 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
   using G = GeomHeadBlock<FP8>;
   using T = Geom<FP8>;
   constexpr int kQSteps = kHeadBlockKSteps<FP8>;
-  TouchArguments();
+  // (without the inline lengths.) 1 x 129 tokens of 64 heads 10.4 -> 9.9 us a layer with its append, 7 x 40..600 of 128
+  // recorded 15.8 -> 15.2, 32 x 512 selected of 8192 36.3 -> 35.3. Not in the split units (32 x 2048 tokens with it
+  // 32.9, without 32.2) nor their merge (32.8).
+  TouchArguments<(offsetof(AttnArgs, inline_lens) + 63) / 64>();
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const unsigned lds_base = Uniform(static_cast<unsigned>(reinterpret_cast<size_t>((__attribute__((address_space(3))) unsigned char*)lds)));
   const int tid = threadIdx.x;

@@ -9,6 +9,7 @@
 // wave-uniform, so the address arithmetic stays in scalar registers.
 #include <mutex>
 
+#include "kernel_arguments.h"
 #include "kernels.h"
 
 #include <hip/hip_ext.h>
@@ -154,6 +155,8 @@ constexpr int kAppendRowsBf16 = 1;  // bf16: a pure copy ran fastest with one ro
 
 template <typename WORDS>
 __global__ __launch_bounds__(kThreads) void AppendBf16Kernel(AppendArgs a, WORDS w) {
+  // (32 x 2048 tokens, append, attention and merge of a layer 32.3 -> 31.9 us)
+  TouchArguments<(sizeof(AppendArgs) + 63) / 64>();
   StoreStepWords(w);
   const int lane = threadIdx.x & (kWave - 1);
   const int token0 = Uniform((blockIdx.x * kWavesPerGroup + (threadIdx.x >> 6)) * kAppendRowsBf16);
@@ -314,6 +317,7 @@ __device__ __forceinline__ void QuantizeRowAndStore(const AppendArgs& a, int lay
 // values it loaded (8-byte store) and one of the 64 rope values (1-byte store).
 template <int ROWS, typename WORDS>
 __global__ __launch_bounds__(kThreads) void AppendFp8Kernel(AppendArgs a, WORDS w) {
+  TouchArguments<(sizeof(AppendArgs) + 63) / 64>();
   static_assert(kRopeDim == kWave, "one rope element per lane");
   StoreStepWords(w);
   const int lane = threadIdx.x & (kWave - 1);
@@ -414,6 +418,8 @@ __device__ __forceinline__ void RotateQueryHeads(const NormRopeAppendArgs& n, in
 // GROUPS: see RotateQueryHeads.
 template <bool FP8, int R, int GROUPS>
 __global__ __launch_bounds__(kThreads) void NormRopeAppendKernel(NormRopeAppendArgs n) {
+  // (2029 tokens into an FP8 cache, 64 query heads rotated along: 8.1 -> 7.8 us)
+  TouchArguments<(sizeof(NormRopeAppendArgs) + 63) / 64>();
   static_assert(kRopeDim == kWave && kLatentDim == 8 * kWave, "lane = 8 latent + 1 rope element");
   const AppendArgs& a = n.append;
   const int lane = threadIdx.x & (kWave - 1);
