@@ -458,7 +458,7 @@ __device__ __forceinline__ bool IssueTileFp8(const AttnArgs& a, TileMap<ALIGNED>
     u32x4 codes = GlobalLoad16(a.rope.base + block * a.rope.block_stride + slot * a.rope.row_stride + (lane & 3) * 16);
     if (!real) codes = u32x4{0u, 0u, 0u, 0u};
     *reinterpret_cast<u32x4*>(buf_ptr + G::kLatRegion + row * G::kRopeRow + (((lane & 3) ^ SwizzleRope8(row)) << 4)) = codes;
-  } else if (wave >= 6 && lane < kTileTokens) {
+  } else if (wave == 6 && lane < kTileTokens) {  // (one wave does: there is no count to keep here)
     int block, slot;
     const bool real = map.Row(tile, lane, &block, &slot);
     const float scale = reinterpret_cast<const float*>(a.scale.base + block * a.scale.block_stride)[slot];
@@ -1102,8 +1102,12 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
           // `loads_c` is the role's loads per tile: in the steady state, kRing - 3 newer tiles on their way, the
           // count to wait for is an immediate. The switch of WaitLoads is some ten taken branches between two
           // barriers; with it for every tile 64 x 512..8192 tokens over an FP8 cache took 72.5 us a layer, so 70.1.
+          // FP8 tiles taken row by row have no count that is known, so neither test nor switch: with the test that never
+          // holds 64 x 512..8192 tokens in blocks of 16 slots took 124.8 us a layer, with the switch alone 122.8, so 118.6.
           const auto publish = [&](int i, auto loads_c) __attribute__((always_inline)) {
-            if (i + 1 < ntiles) {
+            if constexpr (FP8 && !ALIGNED) {
+              asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            } else if (i + 1 < ntiles) {
               if (last_unknown <= i && issued == i + G::kRing - 1 && i + 2 >= solo_tiles) {
                 asm volatile("s_waitcnt vmcnt(%0)" ::"n"((G::kRing - 3) * decltype(loads_c)::value) : "memory");
               } else {
