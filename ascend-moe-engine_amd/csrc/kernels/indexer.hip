@@ -16,7 +16,6 @@
 // and both forms take 16 cycles for 32 elements.
 #include <mutex>
 
-#include "kernel_arguments.h"
 #include "kernels.h"
 
 // (the direct global -> LDS loads name M0, which they set themselves, in their clobber lists)
@@ -492,7 +491,6 @@ __global__ __launch_bounds__(LONG ? kSelectThreads : kShortThreads) void Indexer
 // The row's absmax by four lane exchanges, scale = absmax / 448, codes from the correctly rounded
 // quotient (the E4M3 conversion saturates behind a clamp to +-448).
 __global__ __launch_bounds__(256) void IndexKeyAppendKernel(IndexKeyAppendArgs a) {
-  TouchArguments<(sizeof(IndexKeyAppendArgs) + 63) / 64>();  // (as in the other appends; the indexer's kernels were level with it)
   const int lane = threadIdx.x & 63;
   const int token = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 4);
   const int piece = lane & 15;
