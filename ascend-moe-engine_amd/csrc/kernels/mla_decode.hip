@@ -116,7 +116,7 @@ struct Geom {
   static_assert(kLdsBytes <= 160 * 1024, "one workgroup owns the LDS of a CU");
   __device__ static __forceinline__ int Slot(int i) { return (kRing == 4 ? (i & 3) : (i % kRing)) * kTileBytes; }
 };
-constexpr int kRowsPerWave = kTileTokens / kWaves;           // bf16: latent rows one wave fetches per tile
+constexpr int kRowsPerWave = kTileTokens / kWaves;           // latent rows one wave fetches per tile
 constexpr float kRescaleThreshold = 8.0f;                    // log2 domain
 constexpr int kKAhead = 8;                                   // bf16 K fragments in flight ahead of their MFMA
 constexpr int kKAhead8 = 4;                                  // FP8 K reads (two fragments each) in flight
@@ -305,10 +305,18 @@ struct IssueLane {
   int rope_chunk;
 };
 
-__device__ __forceinline__ int LoadsPerTile(int wave) { return kRowsPerWave + (wave >= kScoreWaves ? 1 : 0); }
+// Latent loads of a wave per whole tile (FP8: a load takes two rows), and all of them: an output wave has one
+// of rope rows or row scales besides. The waits of MlaDecodeKernel count by these: a wave that issued fewer
+// would publish tiles that have not landed.
+template <bool FP8>
+constexpr int kLatentLoads = FP8 ? kRowsPerWave / 2 : kRowsPerWave;
+template <bool FP8>
+constexpr int LoadsPerTile(bool output_wave) {
+  return kLatentLoads<FP8> + (output_wave ? 1 : 0);
+}
 
 // Issues this wave's loads of one tile into the buffer at LDS address `buf`; rows that are not
-// real are zero-filled instead. Returns true when the wave issues exactly LoadsPerTile(wave)
+// real are zero-filled instead. Returns true when the wave issues exactly LoadsPerTile<false>()
 // loads (a full tile), false when the number is not known.
 // WITH_PARTNER: an output wave also fetches the latent rows of the score wave it is paired with
 // (wave - kScoreWaves), for the tiles that the output waves issue alone.
@@ -328,11 +336,11 @@ __device__ __forceinline__ bool IssueTileBf16(const AttnArgs& a, TileMap<ALIGNED
     const int64_t pitch = kWaves * a.latent.row_stride;
     const char* rope = a.rope.base + block * a.rope.block_stride + (slot0 + 8 * rope_group) * a.rope.row_stride;
 #pragma unroll
-    for (int i = 0; i < kRowsPerWave; ++i) DirectLoad16(latent + i * pitch, il.lat[i & 1], buf + (wave + kWaves * i) * G::kLatRow);
+    for (int i = 0; i < kLatentLoads<false>; ++i) DirectLoad16(latent + i * pitch, il.lat[i & 1], buf + (wave + kWaves * i) * G::kLatRow);
     if (WITH_PARTNER) {
       const char* partner = latent - kScoreWaves * a.latent.row_stride;
 #pragma unroll
-      for (int i = 0; i < kRowsPerWave; ++i) {
+      for (int i = 0; i < kLatentLoads<false>; ++i) {
         DirectLoad16(partner + i * pitch, il.partner_lat[i & 1], buf + (wave - kScoreWaves + kWaves * i) * G::kLatRow);
       }
     }
@@ -411,13 +419,11 @@ __host__ __device__ __forceinline__ bool PlainRowsAddressable(const AttnArgs& a)
 // wave access); waves 4 and 5 also own the rope rows 16(w-4) .. +15 (64 B each), waves 6 and 7 the 32
 // row scales (128 B, eight lanes; both the same bytes, so that a role has one count of loads per tile).
 struct IssueLane8 {
-  int lat[2];  // byte offset of this lane's chunk from the first row of pair i
+  int lat[kLatentLoads<true>];  // byte offset of this lane's chunk from the first row of pair i
   int rope;
 };
 
-__device__ __forceinline__ int LoadsPerTile8(int wave) { return 2 + (wave >= kScoreWaves ? 1 : 0); }
-
-// FP8 counterpart of IssueTileBf16. The rare path stages through registers; rows that are not
+// FP8 counterpart of IssueTileBf16 (true: LoadsPerTile<true>() loads). The rare path stages through registers; rows that are not
 // real get zero codes and a zero scale.
 template <bool ALIGNED>
 __device__ __forceinline__ bool IssueTileFp8(const AttnArgs& a, TileMap<ALIGNED>& map, const IssueLane8& il, int tile,
@@ -431,7 +437,7 @@ __device__ __forceinline__ bool IssueTileFp8(const AttnArgs& a, TileMap<ALIGNED>
     const char* latent = a.latent.base + block * a.latent.block_stride + (slot0 + 2 * wave) * a.latent.row_stride;
     const int64_t pitch = 16 * a.latent.row_stride;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) DirectLoad16(latent + i * pitch, il.lat[i], buf + (2 * wave + 16 * i) * G::kLatRow);
+    for (int i = 0; i < kLatentLoads<true>; ++i) DirectLoad16(latent + i * pitch, il.lat[i], buf + (2 * wave + 16 * i) * G::kLatRow);
     if (wave == 4 || wave == 5) {
       const int h = wave - 4;
       const char* rope = a.rope.base + block * a.rope.block_stride + (slot0 + 16 * h) * a.rope.row_stride;
@@ -940,13 +946,13 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
         const int head_base = z * 64 + hw * 16;
         const bool active = head_base < a.heads;  // wave-uniform
         const int head = head_base + i16;
-        const int per_tile = FP8 ? LoadsPerTile8(wave) : LoadsPerTile(wave);
+        const int per_tile = LoadsPerTile<FP8>(wave >= kScoreWaves);
         // Direct loads: lane L of a latent row fetches chunk L ^ swizzle(row); rows of this wave.
         IssueLane il;
         IssueLane8 il8;
         if (FP8) {
       #pragma unroll
-          for (int j = 0; j < 2; ++j) {
+          for (int j = 0; j < kLatentLoads<true>; ++j) {
             const int row = 2 * wave + 16 * j + (lane >> 5);
             il8.lat[j] = (lane >> 5) * static_cast<int>(a.latent.row_stride) + (((lane & 31) ^ SwizzleLat8(row)) << 4);
           }
@@ -1090,7 +1096,7 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
           // Loads this wave has in flight that are newer than those of tile t: the first `solo_tiles`
           // tiles carry `solo_loads` each, the later ones `per_tile`.
           const int solo_tiles = kSoloPrologue ? min(G::kRing - 1, ntiles) : 0;
-          const int solo_loads = score_wave ? 0 : per_tile + kRowsPerWave;
+          const int solo_loads = score_wave ? 0 : per_tile + kLatentLoads<FP8>;
           const auto newer_than = [&](int t) __attribute__((always_inline)) {
             const int solo = max(0, min(issued, solo_tiles) - (t + 1));
             const int shared = max(0, issued - max(t + 1, solo_tiles));
@@ -1116,8 +1122,8 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
             }
             __syncthreads();
           };
-          constexpr std::integral_constant<int, FP8 ? 2 : kRowsPerWave> kScoreLoads{};
-          constexpr std::integral_constant<int, FP8 ? 3 : kRowsPerWave + 1> kOutputLoads{};
+          constexpr std::integral_constant<int, LoadsPerTile<FP8>(false)> kScoreLoads{};
+          constexpr std::integral_constant<int, LoadsPerTile<FP8>(true)> kOutputLoads{};
           // Issues the next tile of the ring (tile i + kRing - 1 during iteration i).
           const auto issue_next = [&](int i) __attribute__((always_inline)) {
             if (issued < ntiles) {
