@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 import kv_testing as kt
+import mlakv_ffi as ffi
 
 pytestmark = pytest.mark.gpu
 
@@ -249,3 +250,32 @@ def test_four_workgroups_only_where_an_xcd_holds_them(batch, heads, most, fp8, p
     plan, workspace = _workspace_after(cache, table, ctxs, heads, sparse)
     assert plan.reserved == (3 if parts == 4 else 1)
     assert bool((workspace[2112 * batch * heads:] != SENTINEL).any()) == (parts == 4)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("bs", [16, 32, 64])
+def test_rows_of_zeros_inside_long_segments(bs, fp8):
+    """Block-table entries that name no block inside segments of many more tiles than the ring holds:
+    the tiles they reach are staged with an unknown number of loads, full waits until they have landed, and
+    the counted waits of whole tiles resume behind them. Holes in the first tiles, alone, in a row, a ring
+    apart and a few tiles before the end. A table that names a block of zeros instead gives the same bits (blocks
+    of 16 slots: half a tile each; over an FP8 cache every tile is staged row by row there)."""
+    heads, tile = 64, 32
+    ctxs = [1700, 900, 3000, 70, 640, 1311]
+    cache, table = _cache(ctxs, bs, seed=1101, fp8=fp8)
+    spare = sorted(set(range(cache.blocks)) - {int(b) for s, n in enumerate(ctxs) for b in table[s, :-(-n // bs)]})[0]
+    broken, zeroed = table.copy(), table.copy()
+    for s, tiles in enumerate([(9, 20, 21, 35, 39, 43), (0, 27), (2, 8, 9, 10, 11, 40, 88), (1,), (3, 7, 11, 15, 19), (1, 6, 30, 37)]):
+        for n, at in enumerate(tiles):
+            broken[s, at * tile // bs] = (-1, cache.blocks, 2 ** 31 - 1)[n % 3]
+            zeroed[s, at * tile // bs] = spare
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1105).cuda()
+    expected, expected_lse = kt.oracle_attention(cache, 0, q, zeroed, ctxs, SCALE)
+    # units of 100 tiles of the 64-head kernel: a sequence is one or two segments
+    options = {"selection_units": ffi.ATTN_UNITS_SPLIT, "chunk_tiles": 100}
+    out, lse, plan = kt.attention(cache, 0, q, kt.dev_i32(broken), kt.dev_i32(ctxs), SCALE, **options)
+    assert plan.selection_units == ffi.ATTN_UNITS_SPLIT and plan.chunk_tiles == 100
+    assert np.abs(out.float().cpu().numpy() - expected).max() <= (TOL_FP8 if fp8 else TOL_BF16) * np.abs(expected).max()
+    assert np.abs(lse.cpu().numpy() - expected_lse).max() <= 2e-2
+    whole, whole_lse, _ = kt.attention(cache, 0, q, kt.dev_i32(zeroed), kt.dev_i32(ctxs), SCALE, **options)
+    assert kt.torch.equal(out, whole) and kt.torch.equal(lse, whole_lse)
