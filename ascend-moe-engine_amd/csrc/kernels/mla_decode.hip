@@ -311,12 +311,12 @@ struct IssueLane {
 template <bool FP8>
 constexpr int kLatentLoads = FP8 ? kRowsPerWave / 2 : kRowsPerWave;
 template <bool FP8>
-constexpr int LoadsPerTile(bool output_wave) {
-  return kLatentLoads<FP8> + (output_wave ? 1 : 0);
+constexpr int LoadsPerTile(int wave) {
+  return kLatentLoads<FP8> + (wave >= kScoreWaves ? 1 : 0);
 }
 
 // Issues this wave's loads of one tile into the buffer at LDS address `buf`; rows that are not
-// real are zero-filled instead. Returns true when the wave issues exactly LoadsPerTile<false>()
+// real are zero-filled instead. Returns true when the wave issues exactly LoadsPerTile<false>(wave)
 // loads (a full tile), false when the number is not known.
 // WITH_PARTNER: an output wave also fetches the latent rows of the score wave it is paired with
 // (wave - kScoreWaves), for the tiles that the output waves issue alone.
@@ -423,7 +423,7 @@ struct IssueLane8 {
   int rope;
 };
 
-// FP8 counterpart of IssueTileBf16 (true: LoadsPerTile<true>() loads). The rare path stages through registers; rows that are not
+// FP8 counterpart of IssueTileBf16 (true: LoadsPerTile<true>(wave) loads). The rare path stages through registers; rows that are not
 // real get zero codes and a zero scale.
 template <bool ALIGNED>
 __device__ __forceinline__ bool IssueTileFp8(const AttnArgs& a, TileMap<ALIGNED>& map, const IssueLane8& il, int tile,
@@ -946,7 +946,7 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
         const int head_base = z * 64 + hw * 16;
         const bool active = head_base < a.heads;  // wave-uniform
         const int head = head_base + i16;
-        const int per_tile = LoadsPerTile<FP8>(wave >= kScoreWaves);
+        const int per_tile = LoadsPerTile<FP8>(wave);
         // Direct loads: lane L of a latent row fetches chunk L ^ swizzle(row); rows of this wave.
         IssueLane il;
         IssueLane8 il8;
@@ -1122,8 +1122,8 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
             }
             __syncthreads();
           };
-          constexpr std::integral_constant<int, LoadsPerTile<FP8>(false)> kScoreLoads{};
-          constexpr std::integral_constant<int, LoadsPerTile<FP8>(true)> kOutputLoads{};
+          constexpr std::integral_constant<int, LoadsPerTile<FP8>(0)> kScoreLoads{};
+          constexpr std::integral_constant<int, LoadsPerTile<FP8>(kScoreWaves)> kOutputLoads{};
           // Issues the next tile of the ring (tile i + kRing - 1 during iteration i).
           const auto issue_next = [&](int i) __attribute__((always_inline)) {
             if (issued < ntiles) {
