@@ -155,7 +155,7 @@ constexpr int kAppendRowsBf16 = 1;  // bf16: a pure copy ran fastest with one ro
 
 template <typename WORDS>
 __global__ __launch_bounds__(kThreads) void AppendBf16Kernel(AppendArgs a, WORDS w) {
-  // (32 x 2048 tokens, append, attention and merge of a layer 32.3 -> 31.9 us)
+  // (32 x 2048 tokens, append, attention and merge of a layer 32.3 -> 31.9 us; 8192 rows 5.1 -> 5.0, 65536 28.0 -> 27.4)
   TouchArguments<(sizeof(AppendArgs) + 63) / 64>();
   StoreStepWords(w);
   const int lane = threadIdx.x & (kWave - 1);
@@ -317,7 +317,7 @@ __device__ __forceinline__ void QuantizeRowAndStore(const AppendArgs& a, int lay
 // values it loaded (8-byte store) and one of the 64 rope values (1-byte store).
 template <int ROWS, typename WORDS>
 __global__ __launch_bounds__(kThreads) void AppendFp8Kernel(AppendArgs a, WORDS w) {
-  TouchArguments<(sizeof(AppendArgs) + 63) / 64>();
+  TouchArguments<(sizeof(AppendArgs) + 63) / 64>();  // (9216 rows 8.6 -> 8.4 us, 65536 level)
   static_assert(kRopeDim == kWave, "one rope element per lane");
   StoreStepWords(w);
   const int lane = threadIdx.x & (kWave - 1);
@@ -418,7 +418,8 @@ __device__ __forceinline__ void RotateQueryHeads(const NormRopeAppendArgs& n, in
 // GROUPS: see RotateQueryHeads.
 template <bool FP8, int R, int GROUPS>
 __global__ __launch_bounds__(kThreads) void NormRopeAppendKernel(NormRopeAppendArgs n) {
-  // (2029 tokens into an FP8 cache, 64 query heads rotated along: 8.1 -> 7.8 us)
+  // (2029 tokens, 64 query heads rotated along: FP8 cache 8.1 -> 7.8 us, bf16 8.1 -> 7.6; 4096 tokens, bf16, 128 heads
+  // 25.8 -> 25.3, FP8, 64 heads level)
   TouchArguments<(sizeof(NormRopeAppendArgs) + 63) / 64>();
   static_assert(kRopeDim == kWave && kLatentDim == 8 * kWave, "lane = 8 latent + 1 rope element");
   const AppendArgs& a = n.append;

@@ -186,8 +186,8 @@ def test_halved_units_side_by_side_on_two_streams():
 @pytest.mark.parametrize("fp8", [False, True])
 def test_table_entries_that_name_no_block_read_as_rows_of_zeros(fp8):
     """A block-table entry outside [0, num_blocks) is never followed: its tokens count as rows of
-    zeros (score 0, nothing added to the output), in the whole-context kernel and in both kinds of
-    selected-token units. The oracle gets a table that points those entries at a block that was
+    zeros (score 0, nothing added to the output), in the units of 16 heads that whole contexts this short go
+    to and in both kinds of selected-token units. The oracle gets a table that points those entries at a block that was
     never written (the cache starts as zeros)."""
     bs, heads, k = 64, 32, 256
     ctxs = [700, 300, 64]
