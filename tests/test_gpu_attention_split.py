@@ -279,3 +279,43 @@ def test_rows_of_zeros_inside_long_segments(bs, fp8):
     assert np.abs(lse.cpu().numpy() - expected_lse).max() <= 2e-2
     whole, whole_lse, _ = kt.attention(cache, 0, q, kt.dev_i32(zeroed), kt.dev_i32(ctxs), SCALE, **options)
     assert kt.torch.equal(out, whole) and kt.torch.equal(lse, whole_lse)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("bs", [16, 48, 80])
+def test_half_tiles_in_blocks_of_their_own(bs, fp8):
+    """Blocks that hold whole half tiles (multiples of 16 slots that are none of 32): each half is fetched as a run of
+    rows. The same bits as from blocks of 24 slots, where every row is located on its own, for lengths that
+    end on, before and behind a half; with holes in first and second halves the bits of a table that names a
+    block of zeros there. The row scales of a block start off any 16-byte boundary."""
+    heads = 64
+    ctxs = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 700, 1296, 1311, 2000]
+    caches = {}
+    for size in (bs, 24):
+        cache, table = _cache(ctxs, size, seed=1201, fp8=fp8)
+        if fp8:
+            padded = kt.torch.zeros(cache.blocks, size + 1, device="cuda")
+            padded[:, :size] = cache.scale[0]
+            cache.view.scale, cache.view.scale_block_stride = padded.data_ptr(), 4 * (size + 1)
+            cache.padded = padded
+        caches[size] = (cache, table)
+    cache, table = caches[bs]
+    general, general_table = caches[24]
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1205).cuda()
+    expected, _ = kt.oracle_attention(cache, 0, q, table, ctxs, SCALE)
+    lens = kt.dev_i32(ctxs)
+    spare = sorted(set(range(cache.blocks)) - {int(b) for s, n in enumerate(ctxs) for b in table[s, :-(-n // bs)]})[0]
+    broken, zeroed = table.copy(), table.copy()
+    for s, n in enumerate(ctxs):
+        for at in range(s % 2, -(-n // bs), 5 if n > 100 else 2):
+            broken[s, at] = (-1, cache.blocks, 2 ** 31 - 1)[at % 3]
+            zeroed[s, at] = spare
+    for options in ({"selection_units": ffi.ATTN_UNITS_SPLIT}, {"chunk_tiles": 100}, {"chunk_tiles": 3}):
+        out, lse, _ = kt.attention(cache, 0, q, kt.dev_i32(table), lens, SCALE, **options)
+        assert np.abs(out.float().cpu().numpy() - expected).max() <= (TOL_FP8 if fp8 else TOL_BF16) * np.abs(expected).max()
+        if "chunk_tiles" in options:  # (the automatic cap of a unit goes by the block size)
+            same, same_lse, _ = kt.attention(general, 0, q, kt.dev_i32(general_table), lens, SCALE, **options)
+            assert kt.torch.equal(out, same) and kt.torch.equal(lse, same_lse)
+        holes = [kt.attention(cache, 0, q, kt.dev_i32(t), lens, SCALE, quant=True, **options) for t in (broken, zeroed)]
+        for got, want in zip(holes[0], holes[1]):
+            assert not isinstance(got, kt.torch.Tensor) or kt.torch.equal(got, want)
