@@ -452,8 +452,13 @@ struct IssueLane8 {
   int rope;
 };
 
-// FP8 counterpart of IssueTileBf16 (true: LoadsPerTile<true>(wave) loads). The rare path stages through registers; rows that are not
-// real get zero codes and a zero scale.
+// FP8 counterpart of IssueTileBf16 (true: LoadsPerTile<true>(wave) loads). Rows that are not real get zero codes and a zero scale.
+// Rows located on their own (selections, block sizes that are no multiple of 16, a sequence's last tile) are fetched by the
+// same number of direct loads as whole tiles, each lane forming its row's address.
+// (Staged through registers they cost a wave two to three memory trips a tile, one after the other. Append and attention
+// of a layer, us, before / now: 64 x 512..8192 tokens in blocks of 24 slots 119.0 / 84.3, of 8 119.5 / 84.2; index keys, selection and
+// attention over 2048 selected tokens of 100 sequences 135.9 / 102.7, of 9 44.9 / 43.1; 64 x 512..8192 in blocks of 64,
+// where only last tiles go this way, 71.5 / 70.0.)
 template <int GRANULE>
 __device__ __forceinline__ bool IssueTileFp8(const AttnArgs& a, TileMap<GRANULE>& map, const IssueLane8& il, int tile,
                                              unsigned buf, unsigned char* buf_ptr, int tid) {
@@ -487,29 +492,47 @@ __device__ __forceinline__ bool IssueTileFp8(const AttnArgs& a, TileMap<GRANULE>
     }
     return true;
   }
-#pragma nounroll
-  for (int i = 0; i < 2; ++i) {
+  // (all rows are located first: the loads are opaque to the compiler, which would keep each LDS read of a staged
+  // entry behind the load before it)
+  const bool rope_wave = wave == 4 || wave == 5, scale_wave = wave >= 6;
+  const int side_row = rope_wave ? 16 * (wave - 4) + (lane >> 2) : lane & (kTileTokens - 1);
+  int blocks[kLatentLoads<true> + 1], slots[kLatentLoads<true> + 1];
+  bool reals[kLatentLoads<true> + 1];
+#pragma unroll
+  for (int i = 0; i < kLatentLoads<true>; ++i) reals[i] = map.Row(tile, 2 * wave + 16 * i + (lane >> 5), &blocks[i], &slots[i]);
+  constexpr int kSide = kLatentLoads<true>;
+  reals[kSide] = map.Row(tile, side_row, &blocks[kSide], &slots[kSide]);
+  bool all_real = true;
+#pragma unroll
+  for (int i = 0; i < kLatentLoads<true>; ++i) {
     const int row = 2 * wave + 16 * i + (lane >> 5);
-    int block, slot;
-    const bool real = map.Row(tile, row, &block, &slot);
-    u32x4 codes = GlobalLoad16(a.latent.base + block * a.latent.block_stride + slot * a.latent.row_stride + (lane & 31) * 16);
-    if (!real) codes = u32x4{0u, 0u, 0u, 0u};
-    *reinterpret_cast<u32x4*>(buf_ptr + row * G::kLatRow + (((lane & 31) ^ SwizzleLat8(row)) << 4)) = codes;
+    const char* src = a.latent.base + blocks[i] * a.latent.block_stride + slots[i] * a.latent.row_stride + (((lane & 31) ^ SwizzleLat8(row)) << 4);
+    all_real = all_real && __builtin_amdgcn_ballot_w64(!reals[i]) == 0;
+    if (reals[i]) {
+      DirectLoad16PerLane(src, buf + (2 * wave + 16 * i) * G::kLatRow);
+    } else {
+      *reinterpret_cast<u32x4*>(buf_ptr + (2 * wave + 16 * i) * G::kLatRow + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
   }
-  if (wave == 4 || wave == 5) {
-    const int row = 16 * (wave - 4) + (lane >> 2);
-    int block, slot;
-    const bool real = map.Row(tile, row, &block, &slot);
-    u32x4 codes = GlobalLoad16(a.rope.base + block * a.rope.block_stride + slot * a.rope.row_stride + (lane & 3) * 16);
-    if (!real) codes = u32x4{0u, 0u, 0u, 0u};
-    *reinterpret_cast<u32x4*>(buf_ptr + G::kLatRegion + row * G::kRopeRow + (((lane & 3) ^ SwizzleRope8(row)) << 4)) = codes;
-  } else if (wave == 6 && lane < kTileTokens) {  // (one wave does: there is no count to keep here)
-    int block, slot;
-    const bool real = map.Row(tile, lane, &block, &slot);
-    const float scale = reinterpret_cast<const float*>(a.scale.base + block * a.scale.block_stride)[slot];
-    reinterpret_cast<float*>(buf_ptr + G::kScaleOff)[lane] = real ? scale : 0.0f;
+  if (rope_wave) {
+    const char* src = a.rope.base + blocks[kSide] * a.rope.block_stride + slots[kSide] * a.rope.row_stride + (((lane & 3) ^ SwizzleRope8(side_row)) << 4);
+    unsigned char* dst = buf_ptr + G::kLatRegion + 16 * (wave - 4) * G::kRopeRow;
+    all_real = all_real && __builtin_amdgcn_ballot_w64(!reals[kSide]) == 0;
+    if (reals[kSide]) {
+      DirectLoad16PerLane(src, buf + G::kLatRegion + 16 * (wave - 4) * G::kRopeRow);
+    } else {
+      *reinterpret_cast<u32x4*>(dst + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
+  } else if (scale_wave) {
+    const char* src = a.scale.base + blocks[kSide] * a.scale.block_stride + slots[kSide] * 4;
+    all_real = all_real && __builtin_amdgcn_ballot_w64(!reals[kSide]) == 0;
+    if (lane < kTileTokens && reals[kSide]) {
+      DirectLoad4PerLane(src, buf + G::kScaleOff);
+    } else if (lane < kTileTokens) {
+      reinterpret_cast<float*>(buf_ptr + G::kScaleOff)[lane] = 0.0f;
+    }
   }
-  return false;
+  return all_real;
 }
 
 __device__ __forceinline__ unsigned int PackBf16(float lo, float hi) {
@@ -1147,12 +1170,8 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
           // `loads_c` is the role's loads per tile: in the steady state, kRing - 3 newer tiles on their way, the
           // count to wait for is an immediate. The switch of WaitLoads is some ten taken branches between two
           // barriers; with it for every tile 64 x 512..8192 tokens over an FP8 cache took 72.5 us a layer, so 70.1.
-          // FP8 tiles taken row by row have no count that is known, so neither test nor switch: with the test that never
-          // holds 64 x 512..8192 tokens taken so took 124.8 us a layer, with the switch alone 122.8, so 118.6.
           const auto publish = [&](int i, auto loads_c) __attribute__((always_inline)) {
-            if constexpr (FP8 && GRANULE == 0) {
-              asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            } else if (i + 1 < ntiles) {
+            if (i + 1 < ntiles) {
               if (last_unknown <= i && issued == i + G::kRing - 1 && i + 2 >= solo_tiles) {
                 asm volatile("s_waitcnt vmcnt(%0)" ::"n"((G::kRing - 3) * decltype(loads_c)::value) : "memory");
               } else {
@@ -2371,8 +2390,8 @@ hipError_t Launch(const AttnArgs& args, const dim3& grid, hipStream_t stream) {
 template <bool MXQ>
 hipError_t LaunchByCache(const AttnArgs& args, const dim3& grid, hipStream_t stream) {
   // Blocks of whole tiles, of whole half tiles, any others. Half tiles are worth a kernel of their own: blocks of 16 slots are
-  // common, and row by row a wave locates each of its rows by itself and FP8 rows pass through registers. 64 x 512..8192
-  // tokens in blocks of 16, append and attention of a layer: FP8 118.4 us row by row, 74.6 in halves (blocks of 64: 73.8);
+  // common, and row by row a wave locates each of its rows by itself. 64 x 512..8192
+  // tokens in blocks of 16, append and attention of a layer: FP8 84.2 us row by row (in blocks of 8), 74.6 in halves (blocks of 64: 73.8);
   // bf16 95.4 / 83.4 (83.2).
   if (args.block_size % kTileTokens == 0) {
     return args.fp8 ? Launch<true, 32, MXQ, false>(args, grid, stream) : Launch<false, 32, MXQ, false>(args, grid, stream);

@@ -282,11 +282,11 @@ def test_rows_of_zeros_inside_long_segments(bs, fp8):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("bs", [16, 48, 80])
+@pytest.mark.parametrize("bs", [16, 48, 80, 24, 8])
 def test_half_tiles_in_blocks_of_their_own(bs, fp8):
     """Blocks that hold whole half tiles (multiples of 16 slots that are none of 32): each half is fetched as a run of
-    rows. The same bits as from blocks of 24 slots, where every row is located on its own, for lengths that
-    end on, before and behind a half; with holes in first and second halves the bits of a table that names a
+    rows. The same bits as from blocks of 24 slots, where every row is located on its own (as in blocks of 8), for
+    lengths that end on, before and behind a half; with holes in first and second halves the bits of a table that names a
     block of zeros there. The row scales of a block start off any 16-byte boundary."""
     heads = 64
     ctxs = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 700, 1296, 1311, 2000]
