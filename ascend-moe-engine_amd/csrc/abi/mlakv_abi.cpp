@@ -335,7 +335,7 @@ namespace {
 
 constexpr int32_t kDefaultMergeSpinUs = 50;
 // mlakvAttnPlan::reserved: whole contexts, a selection, a selection whose halved units four workgroups share.
-constexpr int32_t kPlanContext = 0, kPlanSelection = 1, kPlanSelectionQuarters = 3;
+constexpr int32_t kPlanContext = 0, kPlanSelection = 1, kPlanSelectionQuarters = 3, kPlanSelectionEighths = 5;
 static_assert(MLAKV_ATTN_HEAD_BLOCK_TOKENS == mlakv::kAttnHeadBlockTokens, "the header states the kernel's staging size");
 
 // The largest unit (in tiles) whose block-table entries fit the kernel's LDS staging whatever
@@ -349,7 +349,8 @@ int64_t CapUnitTiles(int32_t block_size, bool sparse) {
 // What the workgroups that share a unit of 16 heads leave in the workspace: `parts` partials per
 // (sequence, 16 heads) and, behind all of them, their LSEs (4 x 16 floats each).
 uint64_t HeadBlockPartialBytes(int32_t batch, int32_t heads, int32_t parts) {
-  return static_cast<uint64_t>(batch) * (heads / 16) * parts * (mlakv::HeadBlockPartBytes(parts) + 4 * 16 * sizeof(float));
+  const int32_t slots = parts > 4 ? 8 : parts;  // (five to eight lie as eight do)
+  return static_cast<uint64_t>(batch) * (heads / 16) * slots * (mlakv::HeadBlockPartBytes(slots) + 4 * 16 * sizeof(float));
 }
 
 struct PlanShape {
@@ -397,6 +398,24 @@ int32_t SharedUnitParts(int32_t batch, int32_t heads, int32_t tokens, int32_t dt
   return 4 * fullest <= ComputeUnits() / kXcds ? 4 : 2;
 }
 
+// Workgroups of a unit of 16 heads over more tokens than quarters are for: as many as fit the CUs once, five to eight; 0
+// where fewer fit or the split is ahead. The head blocks of a part are on one XCD, the parts go round them.
+// The line is where the tiles of a share outgrow what the split spends on its larger query, its partials and their merge.
+// Measured, append and attention of a layer, us, split / so: whole contexts of 1100, 1600, 2400 tokens: 4 x 64 heads 20.8 / 18.3, 20.8 /
+// 20.2, 21.4 / 22.1; FP8 22.2 / 19.2, 22.1 / 21.6, 23.1 / 23.1; 8 x 64 23.0 / 19.8, 23.5 / 20.6, 24.4 / 23.0; 12 x 64 24.0 / 20.3,
+// 24.7 / 21.2, 24.4 / 25.6; 2 x 128 20.9 / 18.6, 21.2 / 19.9, 21.4 / 21.7; 32 x 16 22.2 / 20.7, 23.4 / 22.9, 31.1 / 29.1.
+// Selections of 1100, 1500, 2048 tokens (with index keys and selection): 1 x 64 29.6 / 27.2, 29.6 / 28.4, 30.4 / 29.6; 9 x 64 32.8 / 30.2,
+// 33.3 / 31.0, 35.7 / 33.7; FP8 32.8 / 31.6, 33.7 / 32.3, 35.2 / 34.3; 32 x 16 FP8 37.8 / 35.2, 41.7 / 37.2, 44.1 / 40.2; 4 x 128, whose
+// eight head blocks all fetch the same rows, 32.7 / 30.4, 32.1 / 31.7, 33.1 / 33.8, FP8 32.9 / 31.6, 32.5 / 32.9, 33.3 / 35.1.
+// (Contexts of up to 1024 tokens that quarters do not take keep to the split, as plans of that length always have.)
+int32_t ManyUnitParts(int32_t batch, int32_t heads, int32_t tokens, bool selection) {
+  constexpr int32_t kXcds = 8;
+  if (tokens > (selection ? (heads > 64 ? 1408 : 2048) : 1984)) return 0;
+  const int64_t groups = static_cast<int64_t>(kXcds) * (ComputeUnits() / kXcds / (heads / 16));
+  const int32_t parts = static_cast<int32_t>(std::min<int64_t>(8, groups / batch));
+  return parts >= 5 ? parts : 0;
+}
+
 // How a whole-context launch whose longest context is `bound` tokens cuts its work: 0 = the
 // 64-head kernel's flat cut, 1 = one workgroup per (sequence, 16 heads), 2 or 4 = that many. Measured on
 // MI355X, bf16 and FP8 caches alike (64 heads unless said; us, 64-head kernel / one workgroup per
@@ -408,7 +427,8 @@ int32_t SharedUnitParts(int32_t batch, int32_t heads, int32_t tokens, int32_t dt
 // 128: 29.0 / 31.8. (The line at 768 is that of two workgroups per unit; where four fit they are ahead to 1024, append
 // included: 8 x 800 21.3 / 17.7 for the 64-head kernel / four, 8 x 1024 22.3 / 18.8, FP8 22.6 / 18.7, 16 x 1024 24.5 / 20.5.)
 int32_t ShortContextUnits(const mlakvAttnPlan* plan, int32_t bound) {
-  if (plan->selection_units == MLAKV_ATTN_UNITS_SPLIT || bound > MLAKV_ATTN_HEAD_BLOCK_TOKENS) return 0;
+  if (plan->selection_units == MLAKV_ATTN_UNITS_SPLIT) return 0;
+  if (bound > MLAKV_ATTN_HEAD_BLOCK_TOKENS) return plan->selection_units == MLAKV_ATTN_UNITS_AUTO ? ManyUnitParts(plan->batch, plan->heads, bound, false) : 0;
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK) return 1;
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) return 2;
   const int64_t pairs = static_cast<int64_t>(plan->batch) * (plan->heads / 16);
@@ -522,6 +542,10 @@ mlakvStatus AttnPlanImpl(const char* who, int32_t batch, int32_t heads, int32_t 
       HeadBlockPartialBytes(batch, heads, 4) <= shape.workspace) {
     plan->reserved = kPlanSelectionQuarters;
   }
+  if (sparse && plan->selection_units == MLAKV_ATTN_UNITS_SPLIT && chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && !split_asked &&
+      ManyUnitParts(batch, heads, max_seq_len, true) != 0 && HeadBlockPartialBytes(batch, heads, 8) <= shape.workspace) {
+    plan->reserved = kPlanSelectionEighths;
+  }
   plan->workspace_bytes = shape.workspace;
   return MLAKV_SUCCESS;
 }
@@ -604,7 +628,8 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
                         plan->max_seq_len > 0 && plan->block_size > 0 && plan->chunk_tiles >= 0 && plan->work_groups >= 1 &&
                         plan->work_groups <= 65535 &&
                         (plan->reserved == kPlanContext || plan->reserved == kPlanSelection ||
-                         (plan->reserved == kPlanSelectionQuarters && plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES)) &&
+                         (plan->reserved == kPlanSelectionQuarters && plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) ||
+                         (plan->reserved == kPlanSelectionEighths && plan->selection_units == MLAKV_ATTN_UNITS_SPLIT)) &&
                         (plan->reserved == kPlanContext ? (plan->selection_units == MLAKV_ATTN_UNITS_AUTO || plan->selection_units == MLAKV_ATTN_UNITS_SPLIT ||
                                                 ((plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK ||
                                                   plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) &&
@@ -721,10 +746,14 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
   // selection, for two parts)
   const auto partial_bytes = [&]() { return HeadBlockPartialBytes(plan->batch, plan->heads, args.head_block_units); };
   const auto shrink_to_workspace = [&]() {
+    if (args.head_block_units > 4 && partial_bytes() > plan->workspace_bytes) args.head_block_units = 0;  // the split
     while (args.head_block_units > 1 && partial_bytes() > plan->workspace_bytes) args.head_block_units /= 2;
   };
   if (plan->reserved == kPlanSelectionQuarters) {
     args.head_block_units = 4;
+    shrink_to_workspace();
+  } else if (plan->reserved == kPlanSelectionEighths) {
+    args.head_block_units = ManyUnitParts(plan->batch, plan->heads, plan->max_seq_len, true);
     shrink_to_workspace();
   }
   if (!sparse) {

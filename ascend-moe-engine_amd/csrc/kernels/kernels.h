@@ -128,8 +128,8 @@ struct AttnArgs {
   bool merge_in_launch;       // false: the merge is a second launch
   bool fp8;
   // Selected-token attention only: a workgroup takes the whole selection of one sequence for one
-  // block of 16 heads (1: no partials, no merge), or two or four workgroups take an equal share of it
-  // each and the last to finish combines them (2, 4); sparse_count <= kAttnHeadBlockTokens. 0: the split units.
+  // block of 16 heads (1: no partials, no merge), or two, four or five to eight workgroups take an equal share of it
+  // each and the last to finish combines them (2, 4, 5 .. 8); sparse_count <= kAttnHeadBlockTokens, from five on the share of it. 0: the split units.
   int32_t head_block_units;
   unsigned* sync;             // set by the launcher: this launch's counters, null for a second-launch merge
   // Host-known lengths of a small batch travel here instead of through device memory: no upload,

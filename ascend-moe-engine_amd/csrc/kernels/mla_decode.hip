@@ -1767,6 +1767,10 @@ hipError_t LaunchMerge(const AttnArgs& args, hipStream_t stream) {
 // writes the output. Nobody waits, no barrier is involved: those that arrive earlier leave. The words
 // are zero between launches (the last to arrive clears its word). A selection of fewer tiles than
 // parts is taken by the first of them, one tile each.
+// PARTS 8 stands for five to eight, as many as fit the CUs once (head_block_units), for more tokens than quarters are
+// ahead with or than a workgroup can stage: it stages its own share only, and the last part's waves take the slices in
+// four at a time. Append and attention of a layer, us, split units and merge / so: 1 x 1100 tokens of 64 heads 19.3 / 15.9,
+// 8 x 1100 23.0 / 19.8, 8 x 1600 23.5 / 20.6 (FP8 24.6 / 23.4), 4 x 1600 20.8 / 20.2, 4 x 2400 21.4 / 22.1.
 constexpr int kHbWaves = kWaves, kHbThreads = kHbWaves * 64;
 constexpr int kHbLoaders = kScoreWaves;  // the waves that fetch the tiles when every row is a plain row
 template <bool FP8>
@@ -1791,6 +1795,7 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
   using G = GeomHeadBlock<FP8>;
   using T = Geom<FP8>;
   constexpr int kQSteps = kHeadBlockKSteps<FP8>;
+  constexpr bool kMany = PARTS == 8;
   // (without the inline lengths.) 1 x 129 tokens of 64 heads 10.4 -> 9.9 us a layer with its append, 7 x 40..600 of 128
   // recorded 15.8 -> 15.2, 32 x 512 selected of 8192 36.3 -> 35.3. Not in the split units (32 x 2048 tokens with it
   // 32.9, without 32.2) nor their merge (32.8).
@@ -1803,10 +1808,13 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
   // the head blocks of a sequence are neighbours among them.
   const int head_blocks = a.heads >> 4;  // heads is a multiple of 16
   const int rest = blockIdx.x >> 3;
-  const int part = rest % PARTS;
-  const int unit = rest / PARTS;
+  // (PARTS 8, of which a unit has `share`: the head blocks of one part of a sequence are, the parts go round the XCDs.)
+  const int share = kMany ? a.head_block_units : PARTS;
+  const int unit = kMany ? rest : rest / PARTS;
   const int hb = unit % head_blocks;
-  const int seq = (unit / head_blocks) * kXcds + (blockIdx.x & (kXcds - 1));
+  const int group = (unit / head_blocks) * kXcds + (blockIdx.x & (kXcds - 1));
+  const int seq = kMany ? group / share : group;
+  const int part = kMany ? group - seq * share : rest % PARTS;
   if (seq >= a.batch) return;
   const bool score_wave = wave < kScoreWaves;
   const int hw = wave & (kScoreWaves - 1);
@@ -1827,12 +1835,14 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
   const int32_t* table_row = a.block_table + static_cast<int64_t>(seq) * a.table_stride;
   const int slot_bits = a.block_size > 1 ? 32 - __builtin_clz(static_cast<unsigned>(a.block_size - 1)) : 0;
   constexpr int kPerThread = (kAttnHeadBlockTokens + kHbThreads - 1) / kHbThreads;
-  int index[kPerThread];
+  constexpr int kListed = kMany ? kAttnSelectionMax / kHbThreads : kPerThread;
+  const bool selected = a.sparse_indices != nullptr;
+  int index[kListed];
 #pragma unroll
-  for (int j = 0; j < kPerThread; ++j) {
+  for (int j = 0; j < kListed; ++j) {
     const int i = tid + kHbThreads * j;
     // (no selection: the sequence's own positions 0 .. context - 1, a whole context of up to sparse_count tokens)
-    index[j] = i < a.sparse_count ? (a.sparse_indices != nullptr ? selection[i] : i) : -1;
+    index[j] = i < a.sparse_count ? (selected ? selection[i] : i) : -1;
   }
   // Q fragments of a score wave: lane (head i16, k-group g) holds Q[head][32 ks + 8 g .. +7] for the
   // nine k-steps ks of its half. FP8: the code reads cover k = 64 kp + 16 g .. + 15 (two k-steps),
@@ -1856,7 +1866,6 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
 #pragma unroll
     for (int c = 0; c < kQSteps; ++c) q[c] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
   }
-  int wave_end = a.sparse_count;
   bool any_outside = false;
   const bool shift = (a.block_size & (a.block_size - 1)) == 0;
   // Row starts in 16-byte units, by 24-bit multiplies (the launcher sends pools that these do not
@@ -1864,44 +1873,89 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
   const unsigned lat_block16 = static_cast<unsigned>(a.latent.block_stride >> 4), lat_row16 = static_cast<unsigned>(a.latent.row_stride >> 4);
   const unsigned rope_block16 = static_cast<unsigned>(a.rope.block_stride >> 4), rope_row16 = static_cast<unsigned>(a.rope.row_stride >> 4);
   const unsigned scale_block4 = FP8 ? static_cast<unsigned>(a.scale.block_stride >> 2) : 0u;
-#pragma unroll
-  for (int j = 0; j < kPerThread; ++j) {
-    const int i = tid + kHbThreads * j;
-    const bool good = index[j] >= 0 && index[j] < context;  // false behind the list's end as well
-    const u64 bad = __builtin_amdgcn_ballot_w64(!good);
-    if (bad != 0) wave_end = min(wave_end, kHbThreads * j + 64 * wave + static_cast<int>(__builtin_ctzll(bad)));
-    if (good && i < kAttnHeadBlockTokens) {
-      const int logical = shift ? index[j] >> slot_bits : index[j] / a.block_size;
-      const int entry = table_row[logical];
-      const bool inside = static_cast<unsigned>(entry) < static_cast<unsigned>(a.num_blocks);
-      const unsigned block = static_cast<unsigned>(entry), in_block = static_cast<unsigned>(index[j] - logical * a.block_size);
-      latent_rows[i] = inside ? __umul24(block, lat_block16) + __umul24(in_block, lat_row16) : kNoRow;
-      rope_rows[i] = inside ? __umul24(block, rope_block16) + __umul24(in_block, rope_row16) : kNoRow;
-      if constexpr (FP8) scale_rows[i] = inside ? block * scale_block4 + in_block : kNoRow;
-      if (!inside) any_outside = true;
-    }
-  }
-  if (lane == 0) {
-    end_lds[wave] = wave_end;
-    end_lds[kHbWaves + wave] = __builtin_amdgcn_ballot_w64(any_outside) != 0 ? 1 : 0;
-  }
-  // Every role passes this statement with the query in hand: a wait of the compiler's for it further
-  // down would not know of the tile loads issued from inline assembly, and would wait for them all.
-#pragma unroll
-  for (int c = 0; c < kQSteps; ++c) asm volatile("" ::"v"(q[c]));
-  __syncthreads();
+  // Staged entry i: where the row at `position` starts.
+  const auto stage = [&](int i, int position) __attribute__((always_inline)) {
+    const int logical = shift ? position >> slot_bits : position / a.block_size;
+    const int entry = table_row[logical];
+    const bool inside = static_cast<unsigned>(entry) < static_cast<unsigned>(a.num_blocks);
+    const unsigned block = static_cast<unsigned>(entry), in_block = static_cast<unsigned>(position - logical * a.block_size);
+    latent_rows[i] = inside ? __umul24(block, lat_block16) + __umul24(in_block, lat_row16) : kNoRow;
+    rope_rows[i] = inside ? __umul24(block, rope_block16) + __umul24(in_block, rope_row16) : kNoRow;
+    if constexpr (FP8) scale_rows[i] = inside ? block * scale_block4 + in_block : kNoRow;
+    if (!inside) any_outside = true;
+  };
   int seq_len = a.sparse_count, outside = 0;
+  int staged_from = 0;  // the position of staged entry 0
+  if constexpr (kMany) {
+    // The selection goes to LDS as it is and its end is found; then this part's share of it, or of the context, is
+    // resolved. The words live in the ring's last slot, which is first filled two barriers further down, the list where
+    // the scores will be.
+    int* listed = reinterpret_cast<int*>(lds + G::kSOff);
+    int* words = reinterpret_cast<int*>(lds + G::Slot(G::kRing - 1));
+    static_assert(kAttnSelectionMax * 4 <= 2 * kScoreWaves * 64 * 16, "the list fits the scores' space");
+    if (selected) {
+      int wave_end = a.sparse_count;
 #pragma unroll
-  for (int w = 0; w < kHbWaves; ++w) {
-    seq_len = min(seq_len, end_lds[w]);
-    outside |= end_lds[kHbWaves + w];
+      for (int j = 0; j < kListed; ++j) {
+        const u64 bad = __builtin_amdgcn_ballot_w64(index[j] < 0 || index[j] >= context);
+        if (bad != 0) wave_end = min(wave_end, kHbThreads * j + 64 * wave + static_cast<int>(__builtin_ctzll(bad)));
+        listed[tid + kHbThreads * j] = index[j];
+      }
+      if (lane == 0) words[wave] = wave_end;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < kHbWaves; ++w) seq_len = min(seq_len, words[w]);
+    } else {
+      seq_len = min(seq_len, context);
+    }
+    seq_len = Uniform(seq_len);
+    const int tiles = (seq_len + kTileTokens - 1) / kTileTokens, sharers = min(share, max(tiles, 1));
+    if (part >= sharers) return;
+    const int from = (part * tiles + sharers - 1) / sharers;
+    staged_from = from * kTileTokens;
+    const int own = min(((part + 1) * tiles + sharers - 1) / sharers * kTileTokens, seq_len) - staged_from;  // <= kAttnHeadBlockTokens, ensured by the caller
+#pragma unroll
+    for (int j = 0; j < kPerThread; ++j) {
+      const int i = tid + kHbThreads * j;
+      if (i < min(own, kAttnHeadBlockTokens)) stage(i, selected ? listed[staged_from + i] : staged_from + i);
+    }
+    if (lane == 0) words[kHbWaves + wave] = __builtin_amdgcn_ballot_w64(any_outside) != 0 ? 1 : 0;
+#pragma unroll
+    for (int c = 0; c < kQSteps; ++c) asm volatile("" ::"v"(q[c]));  // (as below)
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kHbWaves; ++w) outside |= words[kHbWaves + w];
+  } else {
+    int wave_end = a.sparse_count;
+#pragma unroll
+    for (int j = 0; j < kPerThread; ++j) {
+      const int i = tid + kHbThreads * j;
+      const bool good = index[j] >= 0 && index[j] < context;  // false behind the list's end as well
+      const u64 bad = __builtin_amdgcn_ballot_w64(!good);
+      if (bad != 0) wave_end = min(wave_end, kHbThreads * j + 64 * wave + static_cast<int>(__builtin_ctzll(bad)));
+      if (good && i < kAttnHeadBlockTokens) stage(i, index[j]);
+    }
+    if (lane == 0) {
+      end_lds[wave] = wave_end;
+      end_lds[kHbWaves + wave] = __builtin_amdgcn_ballot_w64(any_outside) != 0 ? 1 : 0;
+    }
+    // Every role passes this statement with the query in hand: a wait of the compiler's for it further
+    // down would not know of the tile loads issued from inline assembly, and would wait for them all.
+#pragma unroll
+    for (int c = 0; c < kQSteps; ++c) asm volatile("" ::"v"(q[c]));
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kHbWaves; ++w) {
+      seq_len = min(seq_len, end_lds[w]);
+      outside |= end_lds[kHbWaves + w];
+    }
+    seq_len = Uniform(seq_len);
   }
-  seq_len = Uniform(seq_len);
   // Every row a real row of the pool (the usual case): the tile loads need no case distinction.
   const bool plain_rows = Uniform(outside) == 0;
   const int all_tiles = (seq_len + kTileTokens - 1) / kTileTokens;
   // the workgroups that take part, at most one per tile, share the tiles evenly
-  const int parts = min(PARTS, max(all_tiles, 1));
+  const int parts = min(share, max(all_tiles, 1));
   if (part >= parts) return;
   const bool shared = parts > 1;
   const int first_tile = (part * all_tiles + parts - 1) / parts;
@@ -1958,9 +2012,9 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
         if constexpr (FP8) {
           unsigned starts[4];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) starts[r] = latent_rows[min(first + lat_row[r], last)];
+          for (int r = 0; r < 4; ++r) starts[r] = latent_rows[min(first + lat_row[r], last) - staged_from];
           const bool scale_wave = wave >= 2;
-          const unsigned extra_start = (scale_wave ? scale_rows : rope_rows)[min(first + extra_row, last)];
+          const unsigned extra_start = (scale_wave ? scale_rows : rope_rows)[min(first + extra_row, last) - staged_from];
           const unsigned extra_dst = scale_wave ? buf + T::kScaleOff : buf + T::kLatRegion + wave * 16 * T::kRopeRow;
           const char* extra_src = scale_wave ? a.scale.base + (static_cast<u64>(extra_start) << 2) : rope_lane + (static_cast<u64>(extra_start) << 4);
           if (plain_rows) {
@@ -1998,8 +2052,8 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
         } else {
           unsigned starts[kRowsPerLoader];
 #pragma unroll
-          for (int r = 0; r < kRowsPerLoader; ++r) starts[r] = latent_rows[min(first + wave + kHbLoaders * r, last)];
-          const unsigned rope_start = rope_rows[min(first + extra_row, last)];
+          for (int r = 0; r < kRowsPerLoader; ++r) starts[r] = latent_rows[min(first + wave + kHbLoaders * r, last) - staged_from];
+          const unsigned rope_start = rope_rows[min(first + extra_row, last) - staged_from];
           if (plain_rows) {
 #pragma unroll
             for (int r = 0; r < kRowsPerLoader; ++r) {
@@ -2313,31 +2367,68 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
       } else {
         const __amdgpu_buffer_rsrc_t memory = __builtin_amdgcn_make_buffer_rsrc(unit_parts, 0, PARTS * kPartBytes, 0x00020000);
         const int at = hw * (kPartBytes / kScoreWaves) + lane * 16;
-        f32x4 theirs[PARTS][kDvPerWave];
+        f32x4 sum[kDvPerWave];
+        if constexpr (PARTS == 4) {
+          f32x4 theirs[PARTS][kDvPerWave];
 #pragma unroll
-        for (int p = 0; p < PARTS; ++p) {
-          lses2[p] = lse2;
-          if (p < parts && p != part) {
-            lses2[p] = LoadAgentF32(lses + p * 64);
+          for (int p = 0; p < PARTS; ++p) {
+            lses2[p] = lse2;
+            if (p < parts && p != part) {
+              lses2[p] = LoadAgentF32(lses + p * 64);
 #pragma unroll
-            for (int n = 0; n < kDvPerWave; ++n) {
-              theirs[p][n] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(memory, at + n * 1024, p * kPartBytes, kAgentScope));
+              for (int n = 0; n < kDvPerWave; ++n) {
+                theirs[p][n] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(memory, at + n * 1024, p * kPartBytes, kAgentScope));
+              }
             }
           }
-        }
-        weigh();
-        const float inv_w = 1.0f / total;
-        f32x4 sum[kDvPerWave];
+          weigh();
+          const float inv_w = 1.0f / total;
 #pragma unroll
-        for (int p = 0; p < PARTS; ++p) {
-          if (p >= parts) break;
-          const float c = weight[p] * inv_w;
-          if (p == part) {
+          for (int p = 0; p < PARTS; ++p) {
+            if (p >= parts) break;
+            const float c = weight[p] * inv_w;
+            if (p == part) {
 #pragma unroll
-            for (int n = 0; n < kDvPerWave; ++n) sum[n] = p == 0 ? o[n] * c : sum[n] + o[n] * c;
-          } else {
+              for (int n = 0; n < kDvPerWave; ++n) sum[n] = p == 0 ? o[n] * c : sum[n] + o[n] * c;
+            } else {
 #pragma unroll
-            for (int n = 0; n < kDvPerWave; ++n) sum[n] = p == 0 ? theirs[p][n] * c : sum[n] + theirs[p][n] * c;
+              for (int n = 0; n < kDvPerWave; ++n) sum[n] = p == 0 ? theirs[p][n] * c : sum[n] + theirs[p][n] * c;
+            }
+          }
+        } else {
+#pragma unroll
+          for (int p = 0; p < PARTS; ++p) lses2[p] = p < parts && p != part ? LoadAgentF32(lses + p * 64) : lse2;
+          float inv_w = 0.0f;
+          // (four slices at a time are as many as there are registers for)
+#pragma unroll
+          for (int p0 = 0; p0 < PARTS; p0 += 4) {
+            if (p0 >= parts) break;
+            f32x4 theirs[4][kDvPerWave];
+#pragma unroll
+            for (int p = p0; p < p0 + 4; ++p) {
+              if (p < parts && p != part) {
+#pragma unroll
+                for (int n = 0; n < kDvPerWave; ++n) {
+                  theirs[p - p0][n] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(memory, at + n * 1024, p * kPartBytes, kAgentScope));
+                }
+              }
+            }
+            if (p0 == 0) {
+              weigh();
+              inv_w = 1.0f / total;
+            }
+#pragma unroll
+            for (int p = p0; p < p0 + 4; ++p) {
+              if (p >= parts) break;
+              const float c = weight[p] * inv_w;
+              if (p == part) {
+#pragma unroll
+                for (int n = 0; n < kDvPerWave; ++n) sum[n] = p == 0 ? o[n] * c : sum[n] + o[n] * c;
+              } else {
+#pragma unroll
+                for (int n = 0; n < kDvPerWave; ++n) sum[n] = p == 0 ? theirs[p - p0][n] * c : sum[n] + theirs[p - p0][n] * c;
+              }
+            }
           }
         }
 #pragma unroll
@@ -2445,7 +2536,8 @@ hipError_t PrepareAttnKernels() {
       PrepareDecode<false, 0, false, true>(),   PrepareDecode<true, 0, false, true>(),
       PrepareMerge<false, false>(), PrepareMerge<true, false>(), PrepareMerge<false, true>(),
       PrepareHeadBlock<1, false>(), PrepareHeadBlock<2, false>(), PrepareHeadBlock<4, false>(),
-      PrepareHeadBlock<1, true>(), PrepareHeadBlock<2, true>(), PrepareHeadBlock<4, true>()};
+      PrepareHeadBlock<1, true>(), PrepareHeadBlock<2, true>(), PrepareHeadBlock<4, true>(),
+      PrepareHeadBlock<8, false>(), PrepareHeadBlock<8, true>()};
   for (const hipError_t e : results) {
     if (e != hipSuccess) return e;
   }
@@ -2498,6 +2590,13 @@ static hipError_t LaunchHeadBlockUnits(AttnArgs& args, hipStream_t stream) {
   if (together) {
     if (hipError_t sync_error = SyncRegion(&args.sync); sync_error != hipSuccess) return sync_error;
   }
+  if (args.head_block_units > 4) {
+    // (a share is what a workgroup can stage, and there is nothing to fall back to here)
+    const int tiles = (args.sparse_count + kTileTokens - 1) / kTileTokens;
+    if (parts > 8 || parts <= 1 || (tiles + parts - 1) / parts * kTileTokens > kAttnHeadBlockTokens) return hipErrorInvalidValue;
+    const dim3 shares(kXcds * (args.heads / 16) * ((args.batch * parts + kXcds - 1) / kXcds));
+    return args.fp8 ? LaunchHeadBlock<8, true>(args, shares, stream) : LaunchHeadBlock<8, false>(args, shares, stream);
+  }
   const dim3 units(kXcds * (args.heads / 16) * parts * sequences_per_xcd);
   switch (parts) {
     case 4: return args.fp8 ? LaunchHeadBlock<4, true>(args, units, stream) : LaunchHeadBlock<4, false>(args, units, stream);
@@ -2528,12 +2627,12 @@ hipError_t LaunchAttnDecode(const AttnArgs& args_in, hipStream_t stream) {
     if ((static_cast<int64_t>(args.num_blocks) << slot_bits) > (int64_t{1} << 31)) return hipErrorInvalidValue;
     // (a pool whose rows the 32-bit starts of the whole-selection units cannot address goes to the split units)
     if (args.head_block_units != 0 && PlainRowsAddressable(args)) {
-      if (args.sparse_count > kAttnHeadBlockTokens || args.heads % 16 != 0 || args.out == nullptr) return hipErrorInvalidValue;
+      if ((args.sparse_count > kAttnHeadBlockTokens && args.head_block_units <= 4) || args.heads % 16 != 0 || args.out == nullptr) return hipErrorInvalidValue;
       return LaunchHeadBlockUnits(args, stream);
     }
     e = args.fp8 ? Launch<true, 0, false, true>(args, grid, stream) : Launch<false, 0, false, true>(args, grid, stream);
   } else if (args.head_block_units != 0 && !quantise && args.out != nullptr && args.heads % 16 == 0 && args.sparse_count > 0 &&
-             args.sparse_count <= kAttnHeadBlockTokens && PlainRowsAddressable(args)) {
+             (args.sparse_count <= kAttnHeadBlockTokens || args.head_block_units > 4) && PlainRowsAddressable(args)) {
     // a whole context of up to sparse_count tokens in the units of the selected-token attention: no
     // selection, a sequence attends to its own positions
     return LaunchHeadBlockUnits(args, stream);

@@ -185,8 +185,8 @@ typedef struct mlakvAttnPlan {
   int32_t max_units;       /* bound on the work units of one launch (sizes the workspace) */
   int32_t merge_mode;      /* MLAKV_ATTN_MERGE_IN_LAUNCH or _SECOND_LAUNCH */
   int32_t merge_spin_us;   /* bound of the in-launch merge's wait for a sequence's other partials */
-  int32_t reserved;        /* 1 or 3: made by mlakvAttnSparsePlanInit (max_seq_len holds sparse_count); 3: its halved units are
-                            * shared by four workgroups each */
+  int32_t reserved;        /* 1, 3 or 5: made by mlakvAttnSparsePlanInit (max_seq_len holds sparse_count); 3: its halved units are
+                            * shared by four workgroups each; 5: units of 16 heads shared by five to eight take SPLIT's place */
   int32_t selection_units; /* selected-token plans: MLAKV_ATTN_UNITS_SPLIT, _HEAD_BLOCK or _HEAD_BLOCK_HALVES, fixed by the plan;
                             * whole-context plans: what the options asked for, MLAKV_ATTN_UNITS_AUTO = every launch chooses */
   uint64_t workspace_bytes;
@@ -215,13 +215,15 @@ mlakvStatus mlakvAttnPlanInit(int32_t batch, int32_t heads, int32_t max_seq_len,
  * heads / 16 units fit the CUs once and up to 256 while they fit twice; else SPLIT. FP8 caches:
  * HEAD_BLOCK_HALVES from 257 selected tokens while two workgroups per unit fit the CUs once; else
  * HEAD_BLOCK while the units fit the CUs four times (beyond that up to 256 selected tokens); else
- * SPLIT.
+ * SPLIT. Where that leaves SPLIT and five workgroups or more per unit of 16 heads fit the CUs once, the plan (its
+ * `reserved` is 5) shares the units between as many as fit, eight at most, as HEAD_BLOCK_HALVES does between two: bf16 caches
+ * from 769 selected tokens on, FP8 from 1025, up to 1408 with more than 64 heads.
  * Whole-context plans (mlakvAttnPlanInit[Ex] without `selection`) use the same units for short
  * contexts: a unit then takes every position of its sequence. AUTO decides at every launch from
  * the longest context the launch can see -- the lengths themselves with mlakvAttnDecodeHostLens,
  * the plan's max_seq_len with lengths in device memory: while two workgroups per unit fit the CUs
  * once, HEAD_BLOCK up to 256 tokens and HEAD_BLOCK_HALVES (with four workgroups per unit while those
- * fit) up to 768; while one per unit fits,
+ * fit) up to 768, and from 1025 to 1984 shared by five to eight while those fit; while one per unit fits,
  * HEAD_BLOCK up to 512; while they fit twice, up to 256; the 64-head kernel otherwise and whenever
  * chunk_tiles, work_groups or merge_mode ask for properties of the split. SPLIT keeps the 64-head
  * kernel always; HEAD_BLOCK and HEAD_BLOCK_HALVES ask for the units (max_seq_len up to
@@ -351,7 +353,8 @@ mlakvStatus mlakvAttnDecodeMxQuant(const mlakvAttnPlan* plan, const mlakvCacheVi
  * it cuts the work (plan->selection_units) is described with MLAKV_ATTN_UNITS_* above. The
  * workspace is required either way; whole-selection units leave it untouched, halved ones use
  * its first 2112 bytes x batch x heads, those that four workgroups share (plan->reserved is 3; never
- * where the options ask for HEAD_BLOCK_HALVES) its first 8256 bytes x batch x heads. */
+ * where the options ask for HEAD_BLOCK_HALVES) its first 8256 bytes x batch x heads, those that five to eight share
+ * (plan->reserved is 5) its first 16512. */
 mlakvStatus mlakvAttnSparsePlanInit(int32_t batch, int32_t heads, int32_t sparse_count, int32_t block_size, int32_t dtype,
                                     mlakvAttnPlan* plan);
 mlakvStatus mlakvAttnDecodeSparse(const mlakvAttnPlan* plan, const mlakvCacheView* cache, int32_t layer,

@@ -319,3 +319,48 @@ def test_half_tiles_in_blocks_of_their_own(bs, fp8):
         holes = [kt.attention(cache, 0, q, kt.dev_i32(t), lens, SCALE, quant=True, **options) for t in (broken, zeroed)]
         for got, want in zip(holes[0], holes[1]):
             assert not isinstance(got, kt.torch.Tensor) or kt.torch.equal(got, want)
+
+
+# Units of 16 heads shared by five to eight workgroups (whole contexts of 1025 to 1984 tokens; selections from 769 on, FP8 from 1025;
+# seen in the workspace and the plan): sequences of fewer tiles than workgroups, empty ones, shares of different sizes, the
+# batches with the fewest and the most workgroups per unit (12, 9 and 8 x 64 heads: five, seven, eight) and the first that keeps
+# to the split (13). The rows of the workspace behind those of eight stay as they are.
+@pytest.mark.skipif(not kt.torch.cuda.is_available() or kt.torch.cuda.get_device_properties(0).multi_processor_count != 256,
+                    reason="the sizes are those of 256 CUs")
+@pytest.mark.parametrize("ctxs,heads,bs,fp8,many", [
+    ([1984, 1, 0, 33, 1025, 257, 1500, 31], 64, 64, False, True), ([1025], 16, 48, True, True), ([1100, 40, 224], 128, 16, True, True),
+    ([1300 - 100 * i for i in range(12)], 64, 64, False, True), ([1030 + 31 * i for i in range(9)], 64, 128, True, True),
+    ([1300 - 90 * i for i in range(13)], 64, 64, True, False), ([1985, 5], 64, 64, False, False), ([1024, 700], 64, 64, False, False)])
+def test_units_shared_by_five_to_eight_workgroups(ctxs, heads, bs, fp8, many):
+    cache, table = _cache(ctxs, bs, seed=1301, fp8=fp8)
+    if many:
+        _, workspace = _workspace_after(cache, table, ctxs, heads)
+        used = 16512 * len(ctxs) * heads
+        assert bool((workspace[8256 * len(ctxs) * heads:used] != SENTINEL).any())
+        assert (workspace[used:] == SENTINEL).all()
+    _check(cache, table, ctxs, heads, seed=1305, fp8=fp8)
+    rng = np.random.default_rng(1307)
+    for k in (769, 1025, 1400, 2048):
+        sparse = np.full((len(ctxs), k), -1, dtype=np.int32)
+        for s, n in enumerate(ctxs):
+            sparse[s, :min(n, k)] = rng.permutation(n)[:k]
+        plan = kt.make_plan(len(ctxs), heads, k, bs, fp8, selection=True)
+        fits = len(ctxs) * heads <= 12 * 64 and (heads <= 64 or k <= 1408)
+        assert plan.reserved == (5 if fits and k > (1024 if fp8 else 768) else plan.reserved) and (fits or plan.reserved != 5)
+        _check(cache, table, ctxs, heads, seed=1309, fp8=fp8, sparse=sparse)
+
+
+# The slices of up to eight parts are fp32: no further from float64 than the split units' bf16 partials, over rows that grow
+# along the context (the parts' weights lie far apart).
+@pytest.mark.parametrize("fp8", [False, True])
+def test_many_workgroups_are_as_precise_as_the_split(fp8):
+    ctxs, heads = [1900, 1200, 1025, 300], 64
+    cache, table = _cache(ctxs, 64, seed=1321, fp8=fp8, grow=lambda at: 0.1 + 4.0 * at / 1900)
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1323).cuda()
+    expected, _ = kt.oracle_attention(cache, 0, q, table, ctxs, SCALE)
+    errors = []
+    for options in ({}, {"selection_units": ffi.ATTN_UNITS_SPLIT}):
+        out, _, _ = kt.attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE, **options)
+        errors.append(np.linalg.norm(out.float().cpu().numpy() - expected) / np.linalg.norm(expected))
+    print(errors)
+    assert errors[0] <= 1.02 * errors[1]
