@@ -364,3 +364,26 @@ def test_many_workgroups_are_as_precise_as_the_split(fp8):
         errors.append(np.linalg.norm(out.float().cpu().numpy() - expected) / np.linalg.norm(expected))
     print(errors)
     assert errors[0] <= 1.02 * errors[1]
+
+
+# Batches at the edges of a window of 64 sequences and with a window in the middle, whose lengths a workgroup asks for
+# ahead: units that begin in every window (one workgroup goes through all of them, 300 take a few tiles each), empty
+# sequences at the edges, a window without any tile. The same for selections, whose lengths are all the list's.
+@pytest.mark.parametrize("batch", [64, 65, 128, 129, 192, 200])
+@pytest.mark.parametrize("options", [{"selection_units": 1}, {"chunk_tiles": 3, "work_groups": 1}, {"chunk_tiles": 2, "work_groups": 7},
+                                     {"chunk_tiles": 1, "work_groups": 300}])
+def test_units_that_begin_in_every_window_of_sequences(batch, options):
+    heads, fp8 = 16, batch % 2 == 1
+    rng = np.random.default_rng(1401)
+    ctxs = [int(n) for n in rng.integers(1, 150, batch)]
+    for at in (0, 63, 64, 127, 128, 191):
+        if at < batch - 1:
+            ctxs[at] = 0
+    if batch == 192:
+        ctxs[64:128] = [0] * 64
+    cache, table = _cache(ctxs, 16, seed=1403, fp8=fp8)
+    _check(cache, table, ctxs, heads, seed=1405, fp8=fp8, **options)
+    sparse = np.full((batch, 40), -1, dtype=np.int32)
+    for s, n in enumerate(ctxs):
+        sparse[s, :min(n, 40)] = rng.permutation(n)[:40]
+    _check(cache, table, ctxs, heads, seed=1409, fp8=fp8, sparse=sparse, **options)
