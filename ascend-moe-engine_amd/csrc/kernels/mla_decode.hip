@@ -740,22 +740,22 @@ struct MergeState {
 
 // Takes partials first, first + step, ... < n of (sequence, head), in the order of the sequence's
 // tiles. Partial 0 sits in slot `first_slot`, partial i > 0 in slot `u0 + i`. Every partial carries
-// an LSE (-inf for an empty one, whose O row is not data), so the loads of a group of eight partials
+// an LSE (-inf for an empty one, whose O row is not data), so the loads of a group of partials (eight or GROUP)
 // are issued together; a group that is not full asks for the last one again (no branch between the
 // loads: 0.3 to 0.5 us less per launch).
 // AGENT: the partials were written by other CUs of this launch (agent-scope loads); otherwise by
 // an earlier launch (plain streaming loads).
 // A NaN LSE spoils the row as it does in a sequence that is not split: the maximum carries it on.
-template <bool AGENT>
+template <bool AGENT, int GROUP = 8>
 __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_in_group, int first_slot, int u0, int first, int step,
                                              int n, int lane, MergeState& s) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) s.acc[j] = 0.0f;
-  for (int c0 = first; c0 < n; c0 += 8 * step) {
-    u32x4 v[8];
-    float l[8];
+  for (int c0 = first; c0 < n; c0 += GROUP * step) {
+    u32x4 v[GROUP];
+    float l[GROUP];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < GROUP; ++u) {
       const int c = c0 + u * step;
       if constexpr (AGENT) {
         const int64_t row = PartialRow(a, z, c == 0 || n == 1 ? first_slot : u0 + min(c, n - 1), head_in_group);
@@ -771,7 +771,7 @@ __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_
     if constexpr (AGENT) WaitAgentLoads(v);
     float group_max = s.m;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) group_max = __builtin_elementwise_maximum(group_max, l[u]);
+    for (int u = 0; u < GROUP; ++u) group_max = __builtin_elementwise_maximum(group_max, l[u]);
     if (group_max == -__builtin_inff()) continue;  // nothing but empty partials so far
     const float rescale = __builtin_amdgcn_exp2f(s.m - group_max);  // 0 on the first group
     s.m = group_max;
@@ -779,7 +779,7 @@ __device__ __forceinline__ void TakePartials(const AttnArgs& a, int z, int head_
 #pragma unroll
     for (int j = 0; j < 8; ++j) s.acc[j] *= rescale;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < GROUP; ++u) {
       if (l[u] == -__builtin_inff()) continue;  // empty or padding slot
       const float w = __builtin_amdgcn_exp2f(l[u] - s.m);
       s.denom += w;
@@ -1695,7 +1695,22 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
   MergeState state;
   if (WAYS == 1 || partials < shared_from) {
     if (h >= a.heads) return;
-    TakePartials<false>(a, h >> 6, h & 63, a.max_units + seq, first_unit, 0, 1, partials, lane, state);
+    // One wave per head takes few partials in groups of four or six: a padded group fetches its last row again and
+    // again, 1 KB each from the L1, and with up to 8192 waves that is most of what the launch moves. (Groups of eight / so,
+    // append and attention of a layer, us: 100 x 300..700 tokens 37.9 / 35.9, 128 x 1000..2000 over an FP8 cache 60.9 / 59.2, 70 x
+    // 2000..4000 69.8 / 69.3; with groups of two as well the first two take 35.9 and 59.0. Launches that share heads have
+    // little to pad, and the tests cost them 0.3 %: 20 x 2000..5000 tokens 34.6 / 34.7. Eight is tested first: tested last, 32 x
+    // 2048 tokens, which have eight partials, lost 0.4 %.)
+    const auto take = [&](auto size) __attribute__((always_inline)) {
+      TakePartials<false, decltype(size)::value>(a, h >> 6, h & 63, a.max_units + seq, first_unit, 0, 1, partials, lane, state);
+    };
+    if (WAYS > 1 || partials > 6) {
+      take(std::integral_constant<int, 8>{});
+    } else if (partials > 4) {
+      take(std::integral_constant<int, 6>{});
+    } else {
+      take(std::integral_constant<int, 4>{});
+    }
   } else if constexpr (WAYS > 1) {
     h = group * (kMergeHeads / WAYS) + wave / WAYS;
     const int way = wave % WAYS;

@@ -387,3 +387,18 @@ def test_units_that_begin_in_every_window_of_sequences(batch, options):
     for s, n in enumerate(ctxs):
         sparse[s, :min(n, 40)] = rng.permutation(n)[:40]
     _check(cache, table, ctxs, heads, seed=1409, fp8=fp8, sparse=sparse, **options)
+
+
+# One to ten partials per sequence, around the merge's groups of four, six and eight: the bits of the merge inside the
+# launch, which takes eight at a time, and the oracle's values. (Units of 128 tokens, so few per sequence on average that no
+# waves share a head.)
+@pytest.mark.parametrize("heads,fp8,quant", [(64, False, False), (80, True, False), (16, True, True), (128, False, True)])
+def test_groups_of_four_six_and_eight_partials(heads, fp8, quant):
+    ctxs = [128 * i - i % 3 for i in range(1, 11)] + [0, 512, 513, 768, 769]
+    cache, table = _cache(ctxs, 48, seed=1501, fp8=fp8, grow=lambda at: 0.1 + 3.0 * at / 1280)
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1503).cuda()
+    second, inside = [kt.attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE, quant=quant, chunk_tiles=4, merge_mode=mode)
+                      for mode in (ffi.ATTN_MERGE_SECOND_LAUNCH, ffi.ATTN_MERGE_IN_LAUNCH)]
+    for got, want in zip(second, inside):
+        assert not isinstance(got, kt.torch.Tensor) or kt.torch.equal(got, want)
+    _check(cache, table, ctxs, heads, seed=1503, fp8=fp8, chunk_tiles=4)
