@@ -756,6 +756,7 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
     args.head_block_units = ManyUnitParts(plan->batch, plan->heads, plan->max_seq_len, true);
     shrink_to_workspace();
   }
+  if (!mlakv::HeadBlockUnitsReach(args)) args.head_block_units = 0;
   if (!sparse) {
     // A whole context that is short: the units of the selected-token attention (one workgroup, or
     // two, per sequence and 16 heads; no selection, every position of the context) are ahead of the
@@ -769,6 +770,7 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
     }
     args.head_block_units = ShortContextUnits(plan, bound);
     shrink_to_workspace();
+    if (!mlakv::HeadBlockUnitsReach(args)) args.head_block_units = 0;
     if (quant != nullptr && args.head_block_units != 0) {
       // The units have no quantising epilogue: they write bf16 rows (the caller's, or rows of the
       // workspace behind the parts' partials) and the standalone quantiser follows in the same

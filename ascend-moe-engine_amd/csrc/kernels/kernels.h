@@ -183,6 +183,18 @@ constexpr int kAttnBoundaryTiles = 4;      // what entering a sequence inside a 
 constexpr int kAttnSyncSequences = 4096;   // (head group, sequence) pairs a launch can merge in place
 constexpr int kAttnHeadBlockTokens = 1024; // selected tokens a whole-sequence unit of 16 heads stages in LDS
 
+// Whether the units of 16 heads (head_block_units) reach every row of the pool: they form the start of a row inside its
+// plane in 16-byte units with 24-bit multiplies and hold it in 32 bits. The caller of LaunchAttnDecode chooses them only
+// where this holds: what it lays out in the workspace goes by the units or by the split.
+inline bool HeadBlockUnitsReach(const AttnArgs& a) {
+  const int64_t limit = int64_t{1} << 28;  // strides in 16-byte units below 2^24
+  return a.latent.block_stride < limit && a.rope.block_stride < limit && a.latent.row_stride < limit && a.rope.row_stride < limit &&
+         a.num_blocks <= (1 << 24) && a.num_blocks * a.latent.block_stride < (int64_t{1} << 36) &&
+         a.num_blocks * a.rope.block_stride < (int64_t{1} << 36) &&
+         // (FP8: a row's scale, in 4-byte units from its plane's base)
+         (!a.fp8 || a.num_blocks * a.scale.block_stride < (int64_t{1} << 34));
+}
+
 hipError_t LaunchAppend(const AppendArgs& args, hipStream_t stream);
 hipError_t LaunchNormRopeAppend(const NormRopeAppendArgs& args, hipStream_t stream);
 // With both events the launch records its own start and end in them (the dispatch's timestamps:

@@ -431,17 +431,6 @@ __device__ __forceinline__ bool IssueTileBf16(const AttnArgs& a, TileMap<GRANULE
   return false;
 }
 
-// Whether a row's start inside its plane can be formed in 16-byte units with 24-bit multiplies
-// and held in 32 bits (what the whole-selection units of 16 heads stage per selected token).
-__host__ __device__ __forceinline__ bool PlainRowsAddressable(const AttnArgs& a) {
-  const int64_t limit = int64_t{1} << 28;  // strides in 16-byte units below 2^24
-  return a.latent.block_stride < limit && a.rope.block_stride < limit && a.latent.row_stride < limit && a.rope.row_stride < limit &&
-         a.num_blocks <= (1 << 24) && a.num_blocks * a.latent.block_stride < (int64_t{1} << 36) &&
-         a.num_blocks * a.rope.block_stride < (int64_t{1} << 36) &&
-         // (FP8: a row's scale, in 4-byte units from its plane's base)
-         (!a.fp8 || a.num_blocks * a.scale.block_stride < (int64_t{1} << 34));
-}
-
 // ---- FP8 tiles: direct global -> LDS, codes and row scales as they are in the cache -------------
 
 // Wave w of 8 owns the latent row pairs {2w, 2w+1} and {16+2w, 17+2w} (a 512-byte row is half a
@@ -1897,8 +1886,8 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
   }
   bool any_outside = false;
   const bool shift = (a.block_size & (a.block_size - 1)) == 0;
-  // Row starts in 16-byte units, by 24-bit multiplies (the launcher sends pools that these do not
-  // cover to the split units: PlainRowsAddressable).
+  // Row starts in 16-byte units, by 24-bit multiplies (HeadBlockUnitsReach: the callers keep pools that these do not
+  // cover to the split units).
   const unsigned lat_block16 = static_cast<unsigned>(a.latent.block_stride >> 4), lat_row16 = static_cast<unsigned>(a.latent.row_stride >> 4);
   const unsigned rope_block16 = static_cast<unsigned>(a.rope.block_stride >> 4), rope_row16 = static_cast<unsigned>(a.rope.row_stride >> 4);
   const unsigned scale_block4 = FP8 ? static_cast<unsigned>(a.scale.block_stride >> 2) : 0u;
@@ -2654,16 +2643,18 @@ hipError_t LaunchAttnDecode(const AttnArgs& args_in, hipStream_t stream) {
     int slot_bits = 0;
     while ((int64_t{1} << slot_bits) < args.block_size) ++slot_bits;
     if ((static_cast<int64_t>(args.num_blocks) << slot_bits) > (int64_t{1} << 31)) return hipErrorInvalidValue;
-    // (a pool whose rows the 32-bit starts of the whole-selection units cannot address goes to the split units)
-    if (args.head_block_units != 0 && PlainRowsAddressable(args)) {
-      if ((args.sparse_count > kAttnHeadBlockTokens && args.head_block_units <= 4) || args.heads % 16 != 0 || args.out == nullptr) return hipErrorInvalidValue;
+    if (args.head_block_units != 0) {
+      if (!HeadBlockUnitsReach(args) || (args.sparse_count > kAttnHeadBlockTokens && args.head_block_units <= 4) || args.heads % 16 != 0 || args.out == nullptr) return hipErrorInvalidValue;
       return LaunchHeadBlockUnits(args, stream);
     }
     e = args.fp8 ? Launch<true, 0, false, true>(args, grid, stream) : Launch<false, 0, false, true>(args, grid, stream);
-  } else if (args.head_block_units != 0 && !quantise && args.out != nullptr && args.heads % 16 == 0 && args.sparse_count > 0 &&
-             (args.sparse_count <= kAttnHeadBlockTokens || args.head_block_units > 4) && PlainRowsAddressable(args)) {
+  } else if (args.head_block_units != 0) {
     // a whole context of up to sparse_count tokens in the units of the selected-token attention: no
     // selection, a sequence attends to its own positions
+    if (!HeadBlockUnitsReach(args) || quantise || args.out == nullptr || args.heads % 16 != 0 || args.sparse_count <= 0 ||
+        (args.sparse_count > kAttnHeadBlockTokens && args.head_block_units <= 4)) {
+      return hipErrorInvalidValue;
+    }
     return LaunchHeadBlockUnits(args, stream);
   } else {
     e = quantise ? LaunchByCache<true>(args, grid, stream) : LaunchByCache<false>(args, grid, stream);

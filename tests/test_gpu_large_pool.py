@@ -229,3 +229,47 @@ def test_arena_commit_of_a_pool_above_4_gib_is_zero_filled_and_addressed_in_64_b
     assert int(torch.count_nonzero(out_rope[: bs - 1].view(torch.int16))) == 0
     cache.close()
     arena.close()
+
+
+# Blocks 256 MiB apart: the units of 16 heads, which short contexts and selections go to by default, do not reach such
+# rows, and the split takes the launch, the one whose output is quantised too (its bf16 rows, where the caller wants
+# none, share the workspace with whatever partials the launch leaves there). No tolerance: the bits of the split over the same rows in
+# an ordinary pool, and the codes of its output.
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("ctxs", [[700, 40, 0, 300], [1100, 700, 1030]])
+def test_blocks_that_lie_too_far_apart_for_the_units_of_16_heads(ctxs, fp8):
+    bs, heads, stride = 128, 64, 1 << 28
+    blocks = sum(-(-n // bs) for n in ctxs) + 1
+    table = kt.build_tables(ctxs, bs, blocks, seed=401).table()
+    cache = kt.PagedCache(1, blocks, bs, fp8=fp8)
+    total = sum(ctxs)
+    kt.append(cache, kt.randn_bf16((1, total, LATENT), seed=402).cuda(), kt.randn_bf16((1, total, ROPE), seed=403).cuda(),
+              kt.dev_i32(kt.slots_for(table, ctxs, bs)))
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=404).cuda()
+    table_d, lens_d = kt.dev_i32(table), kt.dev_i32(ctxs)
+    rng = np.random.default_rng(405)
+    selections = []
+    for k in (300, 1100):
+        chosen = np.full((len(ctxs), k), -1, dtype=np.int32)
+        for s, n in enumerate(ctxs):
+            chosen[s, :min(n, k)] = rng.permutation(n)[:k]
+        selections.append(kt.dev_i32(chosen))
+    split = {"selection_units": ffi.ATTN_UNITS_SPLIT}
+    want, want_lse, _ = kt.attention(cache, 0, q, table_d, lens_d, SCALE, **split)
+    want_selected = [kt.sparse_attention(cache, 0, q, table_d, lens_d, chosen, SCALE, **split)[0] for chosen in selections]
+    ordinary = kt.attention(cache, 0, q, table_d, lens_d, SCALE)[0]
+    assert not torch.equal(ordinary, want)  # (the units do take these lengths where they reach)
+    far = torch.empty(blocks * stride, dtype=torch.uint8, device="cuda")
+    rows = far.as_strided((blocks, bs * LATENT * cache.element), (stride, 1))
+    rows.copy_(cache.latent[0].reshape(blocks, -1).view(torch.uint8))
+    cache.view.latent, cache.view.latent_block_stride, cache.view.latent_layer_stride = far.data_ptr(), stride, blocks * stride
+    out, lse, _ = kt.attention(cache, 0, q, table_d, lens_d, SCALE)
+    assert torch.equal(out, want) and torch.equal(lse, want_lse)
+    for chosen, expected in zip(selections, want_selected):
+        assert torch.equal(kt.sparse_attention(cache, 0, q, table_d, lens_d, chosen, SCALE)[0], expected)
+    want_codes, want_scales = orc.mx_quant_rows(kt.bits16(want).reshape(-1, LATENT))
+    for want_out in (False, True):
+        out, _, _, codes, scales = kt.attention(cache, 0, q, table_d, lens_d, SCALE, quant=True, want_out=want_out)
+        assert out is None or torch.equal(out, want)
+        assert np.array_equal(codes.cpu().numpy().reshape(-1, LATENT), want_codes)
+        assert np.array_equal(scales.cpu().numpy().reshape(-1, LATENT // 32), want_scales)
