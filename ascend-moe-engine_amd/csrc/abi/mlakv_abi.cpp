@@ -778,10 +778,7 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
       const uint64_t rows_offset = args.head_block_units > 1 ? ((partial_bytes() + 255) & ~255ull) : 0;
       const uint64_t rows_bytes = static_cast<uint64_t>(plan->batch) * plan->heads * mlakv::kLatentDim * 2;
       const bool own_rows = out == nullptr;
-      const bool uniform = (own_rows || out_seq_stride == plan->heads * out_head_stride) &&
-                           quant->codes_seq_stride == plan->heads * quant->codes_head_stride &&
-                           quant->scales_seq_stride == plan->heads * quant->scales_head_stride;
-      if (!uniform || (own_rows && rows_offset + rows_bytes > plan->workspace_bytes)) {
+      if (own_rows && rows_offset + rows_bytes > plan->workspace_bytes) {
         args.head_block_units = 0;
       } else {
         if (own_rows) {
@@ -803,6 +800,15 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
         quantise.scales_row_stride = quant->scales_head_stride;
         quantise.rows = static_cast<int64_t>(plan->batch) * plan->heads;
         quantise.cols = mlakv::kLatentDim;
+        // (not the fused epilogue of the split where there are gaps between the sequences: its rows are rounded otherwise
+        // than mlakvAttnDecode's, whose output the codes are of)
+        if (args.out_seq_stride != plan->heads * args.out_head_stride || quant->codes_seq_stride != plan->heads * quant->codes_head_stride ||
+            quant->scales_seq_stride != plan->heads * quant->scales_head_stride) {
+          quantise.group_rows = plan->heads;
+          quantise.x_group_stride = args.out_seq_stride;
+          quantise.codes_group_stride = quant->codes_seq_stride;
+          quantise.scales_group_stride = quant->scales_seq_stride;
+        }
         status = mlakv::LaunchMxQuant(quantise, static_cast<hipStream_t>(stream));
         return status == hipSuccess ? MLAKV_SUCCESS : HipFail(status, who);
       }

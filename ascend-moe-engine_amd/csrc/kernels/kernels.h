@@ -147,6 +147,9 @@ struct MxQuantArgs {
   int64_t scales_row_stride;
   int64_t rows;
   int32_t cols;
+  // Rows in groups that do not go on from one to the next at the rows' stride (0: one group).
+  int32_t group_rows;
+  int64_t x_group_stride, codes_group_stride, scales_group_stride;
 };
 
 struct IndexerArgs {

@@ -20,8 +20,14 @@ constexpr int kThreads = 256;
 // each dividing its 64-bit item number by the row length, a large launch was bound by its vector
 // instructions. Measured per launch, rows of 64 x 512 values: 4096 rows 75.9 -> 63.7 us (6.3 TB/s),
 // 300 rows 7.8 -> 7.6 us, 32 rows 2.75 -> 2.56 us.
-template <int LOADS>
+// GROUPED: rows in groups with strides of their own, a division more per item.
+template <int LOADS, bool GROUPED>
 __global__ __launch_bounds__(kThreads) void MxQuantKernel(MxQuantArgs q) {
+  const auto at_row = [&](int64_t row, int64_t row_stride, int64_t group_stride) __attribute__((always_inline)) {
+    if constexpr (!GROUPED) return row * row_stride;
+    const unsigned group = static_cast<unsigned>(row) / static_cast<unsigned>(q.group_rows);  // (fewer than 2^32 rows, ensured by the launcher)
+    return group * group_stride + (row - static_cast<int64_t>(group) * q.group_rows) * row_stride;
+  };
   constexpr int kItemsPerGroup = kThreads * LOADS;
   const unsigned items_per_row = static_cast<unsigned>(q.cols) >> 3;
   // the workgroup's first item: a division on uniform values, in 32 bits wherever they suffice
@@ -41,7 +47,7 @@ __global__ __launch_bounds__(kThreads) void MxQuantKernel(MxQuantArgs q) {
     col[u] = at - ahead * items_per_row;
     live[u] = row[u] < q.rows;
     v[u] = u32x4{0u, 0u, 0u, 0u};
-    if (live[u]) v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(q.x + row[u] * q.x_row_stride + col[u] * 16));
+    if (live[u]) v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(q.x + at_row(row[u], q.x_row_stride, q.x_group_stride) + col[u] * 16));
   }
 #pragma unroll
   for (int u = 0; u < LOADS; ++u) {
@@ -53,18 +59,18 @@ __global__ __launch_bounds__(kThreads) void MxQuantKernel(MxQuantArgs q) {
     if (!live[u]) continue;
     const MxScale s = MxScaleFromMaxBits(magnitude);
     const u32x2 codes = {MxEncodeFour(v[u][0], v[u][1], s), MxEncodeFour(v[u][2], v[u][3], s)};
-    __builtin_nontemporal_store(codes, reinterpret_cast<u32x2*>(q.codes + row[u] * q.codes_row_stride + col[u] * 8));
+    __builtin_nontemporal_store(codes, reinterpret_cast<u32x2*>(q.codes + at_row(row[u], q.codes_row_stride, q.codes_group_stride) + col[u] * 8));
     if ((col[u] & 3u) == 0u) {
-      reinterpret_cast<unsigned char*>(q.scales + row[u] * q.scales_row_stride)[col[u] >> 2] = static_cast<unsigned char>(s.code);
+      reinterpret_cast<unsigned char*>(q.scales + at_row(row[u], q.scales_row_stride, q.scales_group_stride))[col[u] >> 2] = static_cast<unsigned char>(s.code);
     }
   }
 }
 
-template <int LOADS>
+template <int LOADS, bool GROUPED>
 hipError_t Launch(const MxQuantArgs& args, int64_t items, hipStream_t stream) {
   const int64_t groups = (items + kThreads * LOADS - 1) / (kThreads * LOADS);
   if (groups > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(MxQuantKernel<LOADS>, dim3(static_cast<unsigned>(groups)), dim3(kThreads), 0, stream, args);
+  hipLaunchKernelGGL((MxQuantKernel<LOADS, GROUPED>), dim3(static_cast<unsigned>(groups)), dim3(kThreads), 0, stream, args);
   return hipGetLastError();
 }
 
@@ -72,7 +78,8 @@ hipError_t Launch(const MxQuantArgs& args, int64_t items, hipStream_t stream) {
 
 hipError_t PrepareMxQuantKernels() {
   hipFuncAttributes attributes;  // (no attribute to set: the calls only load the kernels onto the current device)
-  const void* kernels[] = {reinterpret_cast<const void*>(&MxQuantKernel<1>), reinterpret_cast<const void*>(&MxQuantKernel<2>)};
+  const void* kernels[] = {reinterpret_cast<const void*>(&MxQuantKernel<1, false>), reinterpret_cast<const void*>(&MxQuantKernel<2, false>),
+                           reinterpret_cast<const void*>(&MxQuantKernel<1, true>), reinterpret_cast<const void*>(&MxQuantKernel<2, true>)};
   for (const void* kernel : kernels) {
     if (hipError_t e = hipFuncGetAttributes(&attributes, kernel); e != hipSuccess) return e;
   }
@@ -87,7 +94,11 @@ hipError_t LaunchMxQuant(const MxQuantArgs& args, hipStream_t stream) {
   // us, 100 rows 3.5 / 3.8 / 5.1, 300 rows 7.7 / 7.6 / 7.4, 1000 rows 20.3 / 18.5 / 18.5, 4096 rows
   // 74.4 / 63.6 / 65.4.
   constexpr int64_t kResidentThreads = 256 * 2048;
-  return items <= kResidentThreads ? Launch<1>(args, items, stream) : Launch<2>(args, items, stream);
+  if (args.group_rows > 0) {
+    if (args.rows > 0xffffffffll) return hipErrorInvalidValue;
+    return items <= kResidentThreads ? Launch<1, true>(args, items, stream) : Launch<2, true>(args, items, stream);
+  }
+  return items <= kResidentThreads ? Launch<1, false>(args, items, stream) : Launch<2, false>(args, items, stream);
 }
 
 }  // namespace mlakv

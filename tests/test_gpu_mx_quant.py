@@ -126,6 +126,39 @@ def test_attention_epilogue_equals_quantising_the_bf16_output(fp8, options):
     assert none_out is None and torch.equal(codes2, codes) and torch.equal(scales2, scales)
 
 
+# Rows, codes and scales that do not go on from sequence to sequence at their heads' stride, for lengths that the units of
+# 16 heads take by default (up to 768 and from 1025 tokens) and that they leave to the 64-head kernel: the codes of mlakvAttnDecode's
+# output whatever the strides, and nothing written between the sequences.
+@pytest.mark.parametrize("ctxs", [[300, 1, 0, 200], [700, 40, 600], [1000, 900], [1100, 0, 1029]])
+@pytest.mark.parametrize("want_out", [False, True])
+def test_attention_with_gaps_between_the_quantised_sequences(ctxs, want_out):
+    lib, bs, heads, batch = ffi.load(), 64, 64, len(ctxs)
+    table = kt.build_tables(ctxs, bs, sum(-(-c // bs) for c in ctxs) + 3, seed=411).table()
+    cache = kt.PagedCache(1, sum(-(-c // bs) for c in ctxs) + 3, bs)
+    kt.append(cache, kt.randn_bf16((1, sum(ctxs), LATENT), seed=412).cuda(), kt.randn_bf16((1, sum(ctxs), ROPE), seed=413).cuda(),
+              kt.dev_i32(kt.slots_for(table, ctxs, bs)))
+    q = kt.randn_bf16((batch, heads, LATENT + ROPE), seed=414).cuda()
+    table_d, lens_d = kt.dev_i32(table), kt.dev_i32(ctxs)
+    plain, _, plan = kt.attention(cache, 0, q, table_d, lens_d, SCALE)
+    want_codes, want_scales = orc.mx_quant_rows(kt.bits16(plain).reshape(-1, LATENT))
+    row, out_row, code_row, scale_row = (LATENT + ROPE) * 2, (heads + 1) * LATENT, (heads + 2) * LATENT, (heads + 3) * 16
+    out = torch.full((batch, out_row), -7.0, dtype=torch.bfloat16, device="cuda")
+    codes = torch.full((batch, code_row), 0xAA, dtype=torch.uint8, device="cuda")
+    scales = torch.full((batch, scale_row), 0xAA, dtype=torch.uint8, device="cuda")
+    workspace = torch.empty(int(plan.workspace_bytes), dtype=torch.uint8, device="cuda")
+    target = ffi.MxQuantOut(codes.data_ptr(), code_row, LATENT, scales.data_ptr(), scale_row, 16)
+    ffi.check(lib.mlakvAttnDecodeMxQuant(C.byref(plan), C.byref(cache.view), 0, q.data_ptr(), heads * row, row, q.data_ptr() + LATENT * 2,
+                                         heads * row, row, table_d.data_ptr(), table_d.shape[1], lens_d.data_ptr(), SCALE,
+                                         out.data_ptr() if want_out else None, out_row * 2, LATENT * 2, C.byref(target), None,
+                                         workspace.data_ptr(), workspace.numel(), kt.stream_ptr()))
+    torch.cuda.synchronize()
+    if want_out:
+        assert torch.equal(out[:, :heads * LATENT].reshape(batch, heads, LATENT), plain) and (out[:, heads * LATENT:] == -7).all()
+    assert np.array_equal(codes[:, :heads * LATENT].cpu().numpy().reshape(-1, LATENT), want_codes)
+    assert np.array_equal(scales[:, :heads * 16].cpu().numpy().reshape(-1, 16), want_scales)
+    assert (codes[:, heads * LATENT:] == 0xAA).all() and (scales[:, heads * 16:] == 0xAA).all()
+
+
 def test_fused_entry_argument_checks():
     bs, heads = 64, 16
     cache = kt.PagedCache(1, 4, bs)
