@@ -14,6 +14,7 @@
 #include <string>
 
 #include "../kernels/kernels.h"
+#include "../kernels/sync_regions.h"
 #include "abi_common.h"
 #include "moe_hip/kv_cache_manager.hpp"
 #include "moe_hip/static_arena.hpp"
@@ -543,7 +544,7 @@ mlakvStatus AttnPlanImpl(const char* who, int32_t batch, int32_t heads, int32_t 
     plan->reserved = kPlanSelectionQuarters;
   }
   if (sparse && plan->selection_units == MLAKV_ATTN_UNITS_SPLIT && chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && !split_asked &&
-      ManyUnitParts(batch, heads, max_seq_len, true) != 0 && HeadBlockPartialBytes(batch, heads, 8) <= shape.workspace) {
+      ManyUnitParts(batch, heads, max_seq_len, true) != 0) {
     plan->reserved = kPlanSelectionEighths;
   }
   plan->workspace_bytes = shape.workspace;
@@ -742,21 +743,26 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
   args.merge_in_launch = plan->merge_mode == MLAKV_ATTN_MERGE_IN_LAUNCH;
   args.fp8 = cache->dtype == MLAKV_DTYPE_FP8_E4M3;
   args.head_block_units = plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK ? 1 : (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES ? 2 : 0);
-  // (the parts' partials must fit the plan's workspace, which is sized for the split and, with a
-  // selection, for two parts)
   const auto partial_bytes = [&]() { return HeadBlockPartialBytes(plan->batch, plan->heads, args.head_block_units); };
-  const auto shrink_to_workspace = [&]() {
-    if (args.head_block_units > 4 && partial_bytes() > plan->workspace_bytes) args.head_block_units = 0;  // the split
-    while (args.head_block_units > 1 && partial_bytes() > plan->workspace_bytes) args.head_block_units /= 2;
+  // What the launch can have of the units that were chosen. The parts' partials must fit the plan's workspace, which is
+  // sized for the split and, with a selection, for two parts; the units must reach the pool's rows; and parts
+  // that share a unit need counters to meet on.
+  const auto settle_units = [&]() {
+    while (args.head_block_units > 1 && partial_bytes() > plan->workspace_bytes) {
+      args.head_block_units = args.head_block_units > 4 ? 0 : args.head_block_units / 2;
+    }
+    if (!mlakv::HeadBlockUnitsReach(args)) args.head_block_units = 0;
+    if (args.head_block_units <= 1) return hipSuccess;
+    const hipError_t status =
+        mlakv::AttnCounters(workspace, plan->workspace_bytes, int64_t{4} * plan->batch * (plan->heads / 16), &args.sync);
+    if (args.sync == nullptr) args.head_block_units = mlakv::PartsWithoutCounters(args.head_block_units);
+    return status;
   };
-  if (plan->reserved == kPlanSelectionQuarters) {
-    args.head_block_units = 4;
-    shrink_to_workspace();
-  } else if (plan->reserved == kPlanSelectionEighths) {
-    args.head_block_units = ManyUnitParts(plan->batch, plan->heads, plan->max_seq_len, true);
-    shrink_to_workspace();
+  if (plan->reserved == kPlanSelectionQuarters) args.head_block_units = 4;
+  if (plan->reserved == kPlanSelectionEighths) args.head_block_units = ManyUnitParts(plan->batch, plan->heads, plan->max_seq_len, true);
+  if (sparse) {
+    if (const hipError_t settled = settle_units(); settled != hipSuccess) return HipFail(settled, who);
   }
-  if (!mlakv::HeadBlockUnitsReach(args)) args.head_block_units = 0;
   if (!sparse) {
     // A whole context that is short: the units of the selected-token attention (one workgroup, or
     // two, per sequence and 16 heads; no selection, every position of the context) are ahead of the
@@ -769,8 +775,7 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
       for (int32_t i = 0; i < plan->batch; ++i) bound = std::max(bound, std::min(std::max(host_lens[i], 0), args.max_tokens));
     }
     args.head_block_units = ShortContextUnits(plan, bound);
-    shrink_to_workspace();
-    if (!mlakv::HeadBlockUnitsReach(args)) args.head_block_units = 0;
+    if (const hipError_t settled = settle_units(); settled != hipSuccess) return HipFail(settled, who);
     if (quant != nullptr && args.head_block_units != 0) {
       // The units have no quantising epilogue: they write bf16 rows (the caller's, or rows of the
       // workspace behind the parts' partials) and the standalone quantiser follows in the same
@@ -814,6 +819,12 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
       }
     }
     args.sparse_count = args.head_block_units != 0 ? std::max(bound, 1) : 0;
+  }
+  if (args.head_block_units == 0) args.sync = nullptr;  // (the split takes counters for a wish to merge in the launch)
+  if (args.head_block_units == 0 && args.merge_in_launch) {
+    const int64_t words = int64_t{2} * plan->batch * ((plan->heads + 63) / 64);
+    if (const hipError_t e = mlakv::AttnCounters(workspace, plan->workspace_bytes, words, &args.sync); e != hipSuccess) return HipFail(e, who);
+    args.merge_in_launch = args.sync != nullptr;
   }
   const hipError_t status = mlakv::LaunchAttnDecode(args, static_cast<hipStream_t>(stream));
   return status == hipSuccess ? MLAKV_SUCCESS : HipFail(status, who);

@@ -131,7 +131,9 @@ struct AttnArgs {
   // block of 16 heads (1: no partials, no merge), or two, four or five to eight workgroups take an equal share of it
   // each and the last to finish combines them (2, 4, 5 .. 8); sparse_count <= kAttnHeadBlockTokens, from five on the share of it. 0: the split units.
   int32_t head_block_units;
-  unsigned* sync;             // set by the launcher: this launch's counters, null for a second-launch merge
+  // This launch's counters (AttnCounters): four words per (sequence, 16 heads) where workgroups share units, two per (head group,
+  // sequence) for a merge in the launch, else null.
+  unsigned* sync;
   // Host-known lengths of a small batch travel here instead of through device memory: no upload,
   // no launch for it, and the kernels' first dependent load is gone. inline_count = 0: unused.
   int32_t inline_count;
@@ -218,6 +220,8 @@ hipError_t LaunchStoreWords(const int32_t* host_words, int count, int32_t* dst, 
 // slots from the block (host_words[0 .. num_tokens) is the slot mapping) instead of from memory.
 hipError_t LaunchAppendWithWords(const AppendArgs& args, const int32_t* host_words, int count, int32_t* dst, const int32_t* host_pairs,
                                  int pairs, int32_t* scatter_dst, hipStream_t stream);
+// `words` counters for launches with this workspace on the current device, null where there are none left (SyncRegions).
+hipError_t AttnCounters(const void* workspace, uint64_t workspace_bytes, int64_t words, unsigned** counters);
 hipError_t LaunchAttnDecode(const AttnArgs& args, hipStream_t stream);
 hipError_t LaunchMxQuant(const MxQuantArgs& args, hipStream_t stream);
 hipError_t LaunchIndexer(const IndexerArgs& args, hipStream_t stream);

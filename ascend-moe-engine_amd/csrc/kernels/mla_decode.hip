@@ -57,6 +57,7 @@
 
 #include "kernel_arguments.h"
 #include "kernels.h"
+#include "sync_regions.h"
 
 #include <cstddef>
 #include "mx_quant_device.h"
@@ -2511,30 +2512,13 @@ hipError_t LaunchByCache(const AttnArgs& args, const dim3& grid, hipStream_t str
   return args.fp8 ? Launch<true, 0, MXQ, false>(args, grid, stream) : Launch<false, 0, MXQ, false>(args, grid, stream);
 }
 
-// Meeting points of the in-launch merge: two words per (head group, sequence), all zero between
-// launches (the last contributor to leave a sequence clears its words). A launch takes the next of kSyncRegions
-// regions, so that launches running side by side on different streams do not share counters.
-constexpr int kSyncRegions = 16;
+// Meeting points of launches whose workgroups wait for or count one another: two words per (head group, sequence) for the
+// in-launch merge, four per (sequence, 16 heads) for units that several workgroups share, all zero between launches
+// (the last contributor clears what it used). A region belongs to a workspace (SyncRegions). Most launches that meet
+// are of few sequences and need few words, so those regions are many.
+constexpr int kFewSyncWords = 512, kFewSyncRegions = 4096, kSyncRegions = 64;
+static __device__ __align__(256) unsigned int few_sync_words[kFewSyncRegions][kFewSyncWords];
 static __device__ __align__(256) unsigned int sync_words[kSyncRegions][kAttnSyncSequences * 2];
-
-hipError_t SyncRegion(unsigned** region) {
-  constexpr int kMaxDevices = 64;
-  static std::mutex guard;
-  static unsigned* per_device[kMaxDevices] = {};
-  static unsigned next[kMaxDevices] = {};
-  int device = 0;
-  if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
-  if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
-  std::lock_guard<std::mutex> lock(guard);
-  if (per_device[device] == nullptr) {
-    void* resolved = nullptr;
-    if (hipError_t e = hipGetSymbolAddress(&resolved, HIP_SYMBOL(sync_words)); e != hipSuccess) return e;
-    if (resolved == nullptr) return hipErrorInvalidSymbol;
-    per_device[device] = static_cast<unsigned*>(resolved);
-  }
-  *region = per_device[device] + static_cast<size_t>(next[device]++ % kSyncRegions) * (kAttnSyncSequences * 2);
-  return hipSuccess;
-}
 
 }  // namespace
 
@@ -2560,6 +2544,39 @@ hipError_t PrepareAttnKernels() {
     if (e != hipSuccess) return e;
   }
   once.state[device] = 1;
+  return hipSuccess;
+}
+
+hipError_t AttnCounters(const void* workspace, uint64_t workspace_bytes, int64_t words, unsigned** counters) {
+  constexpr int kMaxDevices = 64;
+  struct Device {
+    std::mutex guard;
+    unsigned *few = nullptr, *many = nullptr;
+    SyncRegions<kFewSyncRegions> few_regions;
+    SyncRegions<kSyncRegions> many_regions;
+  };
+  static Device devices[kMaxDevices];
+  *counters = nullptr;
+  int device = 0;
+  if (hipError_t e = hipGetDevice(&device); e != hipSuccess) return e;
+  if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
+  Device& d = devices[device];
+  {
+    std::lock_guard<std::mutex> lock(d.guard);
+    if (d.few == nullptr || d.many == nullptr) {
+      void *few = nullptr, *many = nullptr;
+      if (hipError_t e = hipGetSymbolAddress(&few, HIP_SYMBOL(few_sync_words)); e != hipSuccess) return e;
+      if (hipError_t e = hipGetSymbolAddress(&many, HIP_SYMBOL(sync_words)); e != hipSuccess) return e;
+      if (few == nullptr || many == nullptr) return hipErrorInvalidSymbol;
+      d.few = static_cast<unsigned*>(few);
+      d.many = static_cast<unsigned*>(many);
+    }
+  }
+  if (words > kAttnSyncSequences * 2) return hipSuccess;
+  const uint64_t name = WorkspaceName(workspace, workspace_bytes);
+  const bool fits_few = words <= kFewSyncWords;
+  const int region = fits_few ? d.few_regions.Of(name) : d.many_regions.Of(name);
+  if (region >= 0) *counters = fits_few ? d.few + int64_t{region} * kFewSyncWords : d.many + int64_t{region} * kAttnSyncSequences * 2;
   return hipSuccess;
 }
 
@@ -2596,22 +2613,17 @@ bool AnySequenceSplit(const AttnArgs& a) {
   return false;
 }
 
-// Whole-selection units of 16 heads, taken by one, two or four workgroups each (head_block_units).
-static hipError_t LaunchHeadBlockUnits(AttnArgs& args, hipStream_t stream) {
-  const int sequences_per_xcd = (args.batch + kXcds - 1) / kXcds;
-  const int64_t pairs = static_cast<int64_t>(args.batch) * (args.heads / 16);
-  // The workgroups of a unit meet on four words each of this launch's counters and leave their
+// Whole-selection units of 16 heads, taken by one, two, four or five to eight workgroups each (head_block_units).
+static hipError_t LaunchHeadBlockUnits(const AttnArgs& args, hipStream_t stream) {
+  const int sequences_per_xcd = (args.batch + kXcds - 1) / kXcds, parts = args.head_block_units;
+  // The workgroups of a unit meet on four words each of the launch's counters and leave their
   // partials in the first parts x 16 x pairs rows of the workspace, the LSEs behind them (the caller
-  // has checked that the workspace holds them).
-  const bool together = args.head_block_units > 1 && pairs * 4 <= kAttnSyncSequences * 2 && args.partial_out != nullptr;
-  const int parts = together ? args.head_block_units : 1;
-  if (together) {
-    if (hipError_t sync_error = SyncRegion(&args.sync); sync_error != hipSuccess) return sync_error;
-  }
-  if (args.head_block_units > 4) {
-    // (a share is what a workgroup can stage, and there is nothing to fall back to here)
+  // has checked that the counters and the workspace hold them).
+  if (parts > 1 && (args.sync == nullptr || args.partial_out == nullptr)) return hipErrorInvalidValue;
+  if (parts > 4) {
+    // (a share is what a workgroup can stage)
     const int tiles = (args.sparse_count + kTileTokens - 1) / kTileTokens;
-    if (parts > 8 || parts <= 1 || (tiles + parts - 1) / parts * kTileTokens > kAttnHeadBlockTokens) return hipErrorInvalidValue;
+    if (parts > 8 || (tiles + parts - 1) / parts * kTileTokens > kAttnHeadBlockTokens) return hipErrorInvalidValue;
     const dim3 shares(kXcds * (args.heads / 16) * ((args.batch * parts + kXcds - 1) / kXcds));
     return args.fp8 ? LaunchHeadBlock<8, true>(args, shares, stream) : LaunchHeadBlock<8, false>(args, shares, stream);
   }
@@ -2628,10 +2640,10 @@ hipError_t LaunchAttnDecode(const AttnArgs& args_in, hipStream_t stream) {
   if (args.batch <= 0) return hipSuccess;
   if (hipError_t e = PrepareAttnKernels(); e != hipSuccess) return e;
   const int head_groups = (args.heads + 63) / 64;
-  const bool merge_in_launch = args.merge_in_launch && static_cast<int64_t>(args.batch) * head_groups <= kAttnSyncSequences;
-  args.sync = nullptr;
-  if (merge_in_launch) {
-    if (hipError_t e = SyncRegion(&args.sync); e != hipSuccess) return e;
+  const bool merge_in_launch = args.merge_in_launch;
+  if (merge_in_launch && args.head_block_units == 0 &&
+      (args.sync == nullptr || static_cast<int64_t>(args.batch) * head_groups > kAttnSyncSequences)) {
+    return hipErrorInvalidValue;
   }
   const dim3 grid(args.work_groups, head_groups);
   const bool quantise = args.out_codes != nullptr;

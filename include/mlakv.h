@@ -164,13 +164,18 @@ mlakvStatus mlakvCopyBlocks(const mlakvCacheView* cache, int32_t layer_begin, in
  * (MLAKV_ATTN_MERGE_IN_LAUNCH: contributors meet on counters the library keeps in a static device
  * array, with a bounded wait; measured no faster on MI355X, kept for callers that want one
  * launch). seq_lens[b] is read as min(max(seq_lens[b], 0), max_seq_len).
- * Limits of MLAKV_ATTN_MERGE_IN_LAUNCH: the counters are 16 regions per GPU, handed to the launches
- * of a process in turn. Launches that are ordered (one stream, or streams joined by events) can be
- * of any number; of launches that may run side by side on unordered streams at most 16 may be in
- * flight on one GPU, or two of them share counters and merge wrongly. A region's words are zero
- * between launches because the last contributor of every sequence clears them: a launch that is
+ * Counters: what meets inside a launch (MLAKV_ATTN_MERGE_IN_LAUNCH, and units of 16 heads that several workgroups share,
+ * below, also in plans whose merge_mode is _SECOND_LAUNCH) meets on words of the library's, a region for each workspace.
+ * Launches whose workspaces overlap have to be ordered (one stream, or streams joined by events), as they
+ * have to be for their partials; any number of others may run side by side, eagerly or replayed from a recording, which
+ * holds on to the region of its workspace. A region stays with the memory it was first asked for until the
+ * process ends: per GPU 4096 for launches of up to 128 (sequence, 16 heads) pairs or 256 to merge (workspaces from
+ * 16 MiB on count once per 8 MiB of memory they begin in, smaller ones once per address), 64 for larger ones.
+ * A launch that finds none left does without: one workgroup per unit, the 64-head kernel where one does not take the
+ * tokens, or the second-launch merge.
+ * A region's words are zero between launches because the last contributor clears them: a launch that is
  * torn down midway (device reset, process kill) leaves them as they are for the next user of that
- * region in the same process. The second-launch merge has neither limit. */
+ * region in the same process. */
 #define MLAKV_ATTN_MERGE_AUTO 0
 #define MLAKV_ATTN_MERGE_IN_LAUNCH 1
 #define MLAKV_ATTN_MERGE_SECOND_LAUNCH 2
@@ -206,9 +211,8 @@ mlakvStatus mlakvAttnPlanInit(int32_t batch, int32_t heads, int32_t max_seq_len,
  * HEAD_BLOCK_HALVES: the same unit shared by two workgroups, half of the selection's tiles each (a
  *   plan in which AUTO chose it shares a unit between four, a quarter each, while four per unit fit the
  *   CUs once: its `reserved` is 3); each leaves a partial (16 rows) in the workspace and counts
- *   itself on a word of the library's counters (those of MLAKV_ATTN_MERGE_IN_LAUNCH, with their
- *   limit on launches in flight); the last to finish combines them inside the launch, nobody
- *   waits. Up to 2048 (sequence, 16 heads) pairs.
+ *   itself on a word of the library's counters (those of MLAKV_ATTN_MERGE_IN_LAUNCH, see there);
+ *   the last to finish combines them inside the launch, nobody waits. Up to 2048 (sequence, 16 heads) pairs.
  * AUTO, unless chunk_tiles, work_groups or merge_mode ask for properties of the split, takes what
  * was measured ahead. bf16 caches: HEAD_BLOCK_HALVES from 257 to 768 selected tokens while two
  * workgroups per unit fit the CUs once; else HEAD_BLOCK up to 512 selected tokens while batch x

@@ -129,3 +129,75 @@ def test_a_captured_decode_step_replays_like_eager_calls():
             assert np.abs(got - expected).max() <= 2e-2 * np.abs(expected).max()
         # eager work of the program's own between replays
         torch.zeros(1 << 20, device="cuda").sum().item()
+
+
+def test_recorded_steps_side_by_side_share_no_counters():
+    """Two recorded steps of more layers than the library ever had regions handed out in turn, each with a workspace of
+    its own, replayed on two streams without an order between them: every launch in them is of workgroups that meet on
+    counters (units of 16 heads shared by four and by five to eight, whole contexts and selections, and the merge inside the launch).
+    Every replay gives the bits of the same calls made one after the other."""
+    lib, bs, heads, layers = ffi.load(), 64, 64, 20
+    ctxs = [1900, 1100, 33, 1500, 1, 1024]
+    batch = len(ctxs)
+    blocks = sum(-(-n // bs) for n in ctxs) + 2
+    table = kt.build_tables(ctxs, bs, blocks, seed=421, max_blocks=32).table()
+    cache = kt.PagedCache(1, blocks, bs)
+    kt.append(cache, kt.randn_bf16((1, sum(ctxs), LATENT), seed=422).cuda(), kt.randn_bf16((1, sum(ctxs), ROPE), seed=423).cuda(),
+              kt.dev_i32(kt.slots_for(table, ctxs, bs)))
+    rng = np.random.default_rng(424)
+    table_d, lens = kt.dev_i32(table), [kt.dev_i32(ctxs), kt.dev_i32([min(n, 700) for n in ctxs])]
+    selections = {}
+    for k in (700, 1100):
+        chosen = np.full((batch, k), -1, dtype=np.int32)
+        for s, n in enumerate(ctxs):
+            chosen[s, :min(n, k)] = rng.permutation(n)[:k]
+        selections[k] = kt.dev_i32(chosen)
+    plans = [kt.make_plan(batch, heads, 1900, bs, False), kt.make_plan(batch, heads, 700, bs, False),
+             kt.make_plan(batch, heads, 1900, bs, False, merge_mode=ffi.ATTN_MERGE_IN_LAUNCH, merge_spin_us=-1)]
+    sparse_plans = {k: kt.make_plan(batch, heads, k, bs, False, selection=True) for k in selections}
+    row = (LATENT + ROPE) * 2
+
+    class Step:
+        def __init__(self, seed):
+            self.q = kt.randn_bf16((layers, batch, heads, LATENT + ROPE), seed=seed).cuda()
+            self.out = torch.zeros(layers, 5, batch, heads, LATENT, dtype=torch.bfloat16, device="cuda")
+            size = max(int(p.workspace_bytes) for p in plans + list(sparse_plans.values()))
+            self.workspace = torch.empty(size, dtype=torch.uint8, device="cuda")
+
+        def calls(self):
+            stream = kt.stream_ptr()
+            for layer in range(layers):
+                q = self.q[layer].data_ptr()
+                head = (C.byref(cache.view), 0, q, heads * row, row, q + LATENT * 2, heads * row, row, table_d.data_ptr(), table_d.shape[1])
+
+                def tail(n):
+                    return (SCALE, self.out[layer, n].data_ptr(), heads * LATENT * 2, LATENT * 2, None, self.workspace.data_ptr(),
+                            self.workspace.numel(), stream)
+
+                for n, plan in enumerate(plans):
+                    ffi.check(lib.mlakvAttnDecode(C.byref(plan), *head, lens[n % 2].data_ptr(), *tail(n)))
+                for n, (k, chosen) in enumerate(selections.items()):
+                    ffi.check(lib.mlakvAttnDecodeSparse(C.byref(sparse_plans[k]), *head, lens[0].data_ptr(), chosen.data_ptr(), k, *tail(3 + n)))
+
+    steps = [Step(425), Step(426)]
+    want, graphs, streams = [], [], [torch.cuda.Stream(), torch.cuda.Stream()]
+    for step in steps:
+        step.calls()
+        torch.cuda.synchronize()
+        want.append(step.out.clone())
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step.calls()
+        graphs.append(graph)
+    assert torch.isfinite(want[0].float()).all()
+    for _ in range(6):
+        for step in steps:
+            step.out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for graph, stream in zip(graphs, streams):
+            with torch.cuda.stream(stream):
+                graph.replay()
+                graph.replay()
+        torch.cuda.synchronize()
+        for step, expected in zip(steps, want):
+            assert torch.equal(step.out, expected)
