@@ -401,20 +401,62 @@ int32_t SharedUnitParts(int32_t batch, int32_t heads, int32_t tokens, int32_t dt
 
 // Workgroups of a unit of 16 heads over more tokens than quarters are for: as many as fit the CUs once, five to eight; 0
 // where fewer fit or the split is ahead. The head blocks of a part are on one XCD, the parts go round them.
-// The line is where the tiles of a share outgrow what the split spends on its larger query, its partials and their merge.
-// Measured, append and attention of a layer, us, split / so: whole contexts of 1100, 1600, 2400 tokens: 4 x 64 heads 20.8 / 18.3, 20.8 /
-// 20.2, 21.4 / 22.1; FP8 22.2 / 19.2, 22.1 / 21.6, 23.1 / 23.1; 8 x 64 23.0 / 19.8, 23.5 / 20.6, 24.4 / 23.0; 12 x 64 24.0 / 20.3,
-// 24.7 / 21.2, 24.4 / 25.6; 2 x 128 20.9 / 18.6, 21.2 / 19.9, 21.4 / 21.7; 32 x 16 22.2 / 20.7, 23.4 / 22.9, 31.1 / 29.1.
-// Selections of 1100, 1500, 2048 tokens (with index keys and selection): 1 x 64 29.6 / 27.2, 29.6 / 28.4, 30.4 / 29.6; 9 x 64 32.8 / 30.2,
-// 33.3 / 31.0, 35.7 / 33.7; FP8 32.8 / 31.6, 33.7 / 32.3, 35.2 / 34.3; 32 x 16 FP8 37.8 / 35.2, 41.7 / 37.2, 44.1 / 40.2; 4 x 128, whose
-// eight head blocks all fetch the same rows, 32.7 / 30.4, 32.1 / 31.7, 33.1 / 33.8, FP8 32.9 / 31.6, 32.5 / 32.9, 33.3 / 35.1.
+// The lines are where the tiles of a share outgrow what the split spends on its larger query, its partials and their merge.
+// They lie lower
+//  - for 32, 80 and 96 heads: half or more of the split's last 64 heads do not exist, which makes it faster, while every
+//    head block here fetches all rows for itself (with 16 heads there is one, and the split is behind throughout);
+//  - for eight parts on more than a quarter of the CUs: a batch that leaves eight has so few rows that the split is in its smallest
+//    units (four tiles, of a selection two), which take no longer for more tokens, while a part here does;
+//  - for selections, whose rows the split locates while the query is on its way.
+// (One process and the next differ by up to 0.5 us where both sides are the split: the lines leave out what loses by more.)
+// Measured, us a layer, split / so, equal lengths (ragged ones gain 1 to 5 us wherever they were tried, their longest at 1100 to 1900).
+// Whole contexts with their append, recorded, of 1100, 1500, 1700, 1900 tokens: 12 x 64 heads (five) 23.2 / 20.6, 24.7 / 22.1, 24.5 / 23.1,
+// 24.9 / 24.6, FP8 24.2 / 22.2, 25.3 / 23.5, 25.0 / 24.3, 25.5 / 25.8; 6 x 128 FP8 (five) 24.0 / 21.7, 25.1 / 23.0, 24.7 / 23.7, 25.1 / 25.4; 13 x 48 FP8
+// (six) 23.9 / 21.1, 24.1 / 22.7, 24.2 / 24.4, 24.2 / 24.8; 10 x 64 (six) 22.3 / 19.6, 23.8 / 21.3, 24.4 / 22.7, 25.1 / 23.3; 9 x 64 (seven) 24.2 / 20.3,
+// 23.4 / 21.0, 23.8 / 21.9, 24.2 / 22.8; 8 x 64 (eight) 21.9 / 20.2, 22.3 / 20.8, 22.6 / 21.1, 23.5 / 22.2; 2 x 128 19.8 / 18.4, 20.0 / 19.9, 20.4 / 20.1,
+// 20.5 / 20.5 (1800: 20.2 / 20.8); 1 x 64 18.9 / 16.1, 19.0 / 17.6, 19.1 / 17.9, 19.4 / 18.2; 51 x 16 FP8 27.1 / 22.5, 31.9 / 24.2, 33.2 / 25.1, 33.5 / 26.1;
+// 25 x 32 (five) 23.7 / 21.5, 25.2 / 24.3, 25.9 / 26.9, 26.7 / 29.4, FP8 23.5 / 22.2, 25.5 / 23.6, 27.1 / 24.5, 27.4 / 25.8; 8 x 96 (five) 21.7 / 21.1, 22.2 / 21.9,
+// 22.2 / 22.4, 22.6 / 23.9; 6 x 80 (eight) 20.5 / 20.1, 20.9 / 21.4, 20.7 / 21.6, 20.9 / 21.4 (1300: 20.6 / 21.7). The quantising entry point, which follows
+// with a launch of its own, is level where lengths are equal (12 x 64, 1100, 1500, 1800 tokens: 24.2 / 22.9, 26.1 / 24.7, 26.0 / 26.4; 4 x 64 21.1 / 20.8,
+// 21.5 / 22.4, 21.9 / 23.2) and ahead where they are ragged (24.8 / 20.6, 23.3 / 21.8; 20.7 / 18.9, 21.1 / 20.0).
+// Selections of 1100, 1400, 1700, 2048 tokens with index keys and selection: 12 x 64 (five) 32.3 / 31.0, 35.2 / 32.8, 35.9 / 35.0, 37.7 / 37.5, FP8
+// 32.8 / 32.1, 35.6 / 32.3, 34.9 / 34.2, 36.4 / 36.3; 9 x 64 (seven) of up to 32768 tokens, 2048: 44.7 / 44.3, FP8 44.4 / 43.9; 25 x 32 (five) 40.1 / 37.4, 41.9 / 40.1,
+// 43.6 / 43.9, 45.6 / 47.2, FP8 39.3 / 36.6, 41.2 / 38.2, 43.1 / 39.8, 44.9 / 41.6; 8 x 64 (eight) 31.2 / 30.1, 31.8 / 30.7, 32.2 / 31.8, 32.7 / 33.6, FP8
+// 31.8 / 30.4, 32.2 / 31.6, 32.4 / 32.7, 32.7 / 34.6; 8 x 32 28.7 / 29.2, 29.4 / 29.8, 29.5 / 30.8, 29.9 / 32.0; 1 x 64 27.9 / 26.7, 28.3 / 28.1, 28.4 / 28.8,
+// 28.7 / 30.1; 1 x 16 FP8 26.7 / 26.3, 26.8 / 27.5, 27.1 / 28.4; 32 x 16 (eight) 40.2 / 38.4, 42.4 / 40.1, 45.5 / 41.8, 46.0 / 44.0. Of 1100, 1250, 1400:
+// 6 x 128 (five) 33.1 / 32.4, 33.5 / 33.0, 34.4 / 32.7; 4 x 128 (eight) 32.2 / 31.8, 32.6 / 33.2, 32.6 / 32.3, FP8 32.7 / 32.7, 33.0 / 34.3, 33.0 / 33.3.
 // (Contexts of up to 1024 tokens that quarters do not take keep to the split, as plans of that length always have.)
-int32_t ManyUnitParts(int32_t batch, int32_t heads, int32_t tokens, bool selection) {
+int32_t ManyUnitParts(int32_t batch, int32_t heads, int32_t tokens, int32_t dtype, bool selection) {
   constexpr int32_t kXcds = 8;
-  if (tokens > (selection ? (heads > 64 ? 1408 : 2048) : 1984)) return 0;
-  const int64_t groups = static_cast<int64_t>(kXcds) * (ComputeUnits() / kXcds / (heads / 16));
+  const int32_t blocks = heads / 16;
+  const int64_t cus = ComputeUnits(), groups = static_cast<int64_t>(kXcds) * (cus / kXcds / blocks);
   const int32_t parts = static_cast<int32_t>(std::min<int64_t>(8, groups / batch));
-  return parts >= 5 ? parts : 0;
+  if (parts < 5) return 0;
+  const int64_t used = static_cast<int64_t>(batch) * blocks * parts;  // CUs
+  const bool half_empty = blocks > 1 && (blocks % 4 == 1 || blocks % 4 == 2), bf16 = dtype == MLAKV_DTYPE_BF16;
+  int32_t most = 0;
+  if (selection) {
+    if (parts < 8) {
+      most = heads > 64 ? 1408 : (bf16 && parts < 7 && (blocks == 2 || blocks == 3) ? 1664 : 2048);
+    } else if (4 * used <= cus) {
+      most = blocks <= 2 ? 1280 : 1408;
+    } else if (blocks == 1) {
+      most = 2 * used >= cus ? 2048 : 1280;
+    } else if (blocks == 4 && 2 * used > cus) {
+      most = 1536;
+    }
+  } else if (half_empty && parts != 7) {
+    if (parts == 8) {
+      most = 8 * used > 7 * cus ? 1152 : 1760;
+    } else {
+      most = bf16 ? 1536 : (blocks == 2 ? 1984 : 1664);
+    }
+  } else if (blocks > 1 && (parts == 5 || (parts == 8 && 4 * used > cus))) {
+    most = bf16 && blocks > 4 ? 1664 : 1760;
+  } else {
+    most = parts == 6 && !bf16 && blocks > 1 ? 1856 : 1984;
+  }
+  return tokens <= most ? parts : 0;
 }
 
 // How a whole-context launch whose longest context is `bound` tokens cuts its work: 0 = the
@@ -429,7 +471,7 @@ int32_t ManyUnitParts(int32_t batch, int32_t heads, int32_t tokens, bool selecti
 // included: 8 x 800 21.3 / 17.7 for the 64-head kernel / four, 8 x 1024 22.3 / 18.8, FP8 22.6 / 18.7, 16 x 1024 24.5 / 20.5.)
 int32_t ShortContextUnits(const mlakvAttnPlan* plan, int32_t bound) {
   if (plan->selection_units == MLAKV_ATTN_UNITS_SPLIT) return 0;
-  if (bound > MLAKV_ATTN_HEAD_BLOCK_TOKENS) return plan->selection_units == MLAKV_ATTN_UNITS_AUTO ? ManyUnitParts(plan->batch, plan->heads, bound, false) : 0;
+  if (bound > MLAKV_ATTN_HEAD_BLOCK_TOKENS) return plan->selection_units == MLAKV_ATTN_UNITS_AUTO ? ManyUnitParts(plan->batch, plan->heads, bound, plan->dtype, false) : 0;
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK) return 1;
   if (plan->selection_units == MLAKV_ATTN_UNITS_HEAD_BLOCK_HALVES) return 2;
   const int64_t pairs = static_cast<int64_t>(plan->batch) * (plan->heads / 16);
@@ -544,7 +586,7 @@ mlakvStatus AttnPlanImpl(const char* who, int32_t batch, int32_t heads, int32_t 
     plan->reserved = kPlanSelectionQuarters;
   }
   if (sparse && plan->selection_units == MLAKV_ATTN_UNITS_SPLIT && chosen.selection_units == MLAKV_ATTN_UNITS_AUTO && !split_asked &&
-      ManyUnitParts(batch, heads, max_seq_len, true) != 0) {
+      ManyUnitParts(batch, heads, max_seq_len, dtype, true) != 0) {
     plan->reserved = kPlanSelectionEighths;
   }
   plan->workspace_bytes = shape.workspace;
@@ -759,7 +801,7 @@ mlakvStatus AttnDecodeImpl(const char* who, const mlakvAttnPlan* plan, const mla
     return status;
   };
   if (plan->reserved == kPlanSelectionQuarters) args.head_block_units = 4;
-  if (plan->reserved == kPlanSelectionEighths) args.head_block_units = ManyUnitParts(plan->batch, plan->heads, plan->max_seq_len, true);
+  if (plan->reserved == kPlanSelectionEighths) args.head_block_units = ManyUnitParts(plan->batch, plan->heads, plan->max_seq_len, plan->dtype, true);
   if (sparse) {
     if (const hipError_t settled = settle_units(); settled != hipSuccess) return HipFail(settled, who);
   }

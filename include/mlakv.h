@@ -220,14 +220,15 @@ mlakvStatus mlakvAttnPlanInit(int32_t batch, int32_t heads, int32_t max_seq_len,
  * HEAD_BLOCK_HALVES from 257 selected tokens while two workgroups per unit fit the CUs once; else
  * HEAD_BLOCK while the units fit the CUs four times (beyond that up to 256 selected tokens); else
  * SPLIT. Where that leaves SPLIT and five workgroups or more per unit of 16 heads fit the CUs once, the plan (its
- * `reserved` is 5) shares the units between as many as fit, eight at most, as HEAD_BLOCK_HALVES does between two: bf16 caches
- * from 769 selected tokens on, FP8 from 1025, up to 1408 with more than 64 heads.
+ * `reserved` is 5) shares the units between as many as fit, eight at most, as HEAD_BLOCK_HALVES does between two, where that was
+ * measured ahead: bf16 caches from 769 selected tokens on, FP8 from 1025, up to a line of 1280 to 2048 that goes by the
+ * heads and by how many share a unit.
  * Whole-context plans (mlakvAttnPlanInit[Ex] without `selection`) use the same units for short
  * contexts: a unit then takes every position of its sequence. AUTO decides at every launch from
  * the longest context the launch can see -- the lengths themselves with mlakvAttnDecodeHostLens,
  * the plan's max_seq_len with lengths in device memory: while two workgroups per unit fit the CUs
  * once, HEAD_BLOCK up to 256 tokens and HEAD_BLOCK_HALVES (with four workgroups per unit while those
- * fit) up to 768, and from 1025 to 1984 shared by five to eight while those fit; while one per unit fits,
+ * fit) up to 768, and from 1025 tokens up to a line of 1152 to 1984 shared by five to eight while those fit; while one per unit fits,
  * HEAD_BLOCK up to 512; while they fit twice, up to 256; the 64-head kernel otherwise and whenever
  * chunk_tiles, work_groups or merge_mode ask for properties of the split. SPLIT keeps the 64-head
  * kernel always; HEAD_BLOCK and HEAD_BLOCK_HALVES ask for the units (max_seq_len up to

@@ -321,41 +321,69 @@ def test_half_tiles_in_blocks_of_their_own(bs, fp8):
             assert not isinstance(got, kt.torch.Tensor) or kt.torch.equal(got, want)
 
 
-# Units of 16 heads shared by five to eight workgroups (whole contexts of 1025 to 1984 tokens; selections from 769 on, FP8 from 1025;
-# seen in the workspace and the plan): sequences of fewer tiles than workgroups, empty ones, shares of different sizes, the
-# batches with the fewest and the most workgroups per unit (12, 9 and 8 x 64 heads: five, seven, eight) and the first that keeps
-# to the split (13). The rows of the workspace behind those of eight stay as they are.
+# Units of 16 heads shared by five to eight workgroups, whole contexts: sequences of fewer tiles than workgroups, empty ones,
+# shares of different sizes, the batches with the fewest and the most workgroups per unit (12, 9 and 8 x 64 heads: five, seven,
+# eight), and every line of the rule from both sides. The workspace shows them: eight leave what lies behind their rows as it was,
+# the split (13 x 64: four do not fit; lengths beyond a line) gives the bits of a plan that asks for it.
 @pytest.mark.skipif(not kt.torch.cuda.is_available() or kt.torch.cuda.get_device_properties(0).multi_processor_count != 256,
                     reason="the sizes are those of 256 CUs")
 @pytest.mark.parametrize("ctxs,heads,bs,fp8,many", [
-    ([1984, 1, 0, 33, 1025, 257, 1500, 31], 64, 64, False, True), ([1025], 16, 48, True, True), ([1100, 40, 224], 128, 16, True, True),
-    ([1300 - 100 * i for i in range(12)], 64, 64, False, True), ([1030 + 31 * i for i in range(9)], 64, 128, True, True),
-    ([1300 - 90 * i for i in range(13)], 64, 64, True, False), ([1985, 5], 64, 64, False, False), ([1024, 700], 64, 64, False, False)])
-def test_units_shared_by_five_to_eight_workgroups(ctxs, heads, bs, fp8, many):
+    ([1760, 1, 0, 33, 1025, 257, 1500, 31], 64, 64, False, True), ([1761, 1, 0, 33, 1025, 257, 1500, 31], 64, 64, False, False),
+    ([1760, 900, 40], 128, 16, True, True), ([1664, 900, 40], 128, 64, False, True), ([1665, 900, 40], 128, 64, False, False),
+    ([1984, 5], 64, 64, False, True), ([1985, 5], 64, 64, False, False), ([1025], 16, 48, True, True), ([1024, 700], 64, 64, False, False),
+    ([1100, 40, 224], 128, 16, True, True), ([1300 - 100 * i for i in range(12)], 64, 64, False, True),
+    ([1760] + [50] * 11, 64, 64, True, True), ([1761] + [50] * 11, 64, 64, True, False), ([1856] + [70] * 9, 64, 64, True, True),
+    ([1857] + [70] * 9, 64, 64, True, False), ([1984] + [70] * 9, 64, 64, False, True), ([1030 + 31 * i for i in range(9)], 64, 128, True, True),
+    ([1300 - 90 * i for i in range(13)], 64, 64, True, False), ([1152, 3, 1100, 700, 65, 32], 80, 64, False, True),
+    ([1153, 3, 1100, 700, 65, 32], 80, 64, False, False), ([1760, 900, 33], 80, 64, False, True), ([1536] + [60] * 24, 32, 64, False, True),
+    ([1537] + [60] * 24, 32, 64, False, False), ([1984] + [60] * 24, 32, 64, True, True), ([1664] + [60] * 7, 96, 64, True, True),
+    ([1665] + [60] * 7, 96, 64, True, False), ([1984] + [60] * 50, 16, 64, False, True)])
+def test_contexts_in_units_shared_by_five_to_eight_workgroups(ctxs, heads, bs, fp8, many):
     cache, table = _cache(ctxs, bs, seed=1301, fp8=fp8)
+    _check(cache, table, ctxs, heads, seed=1305, fp8=fp8)
     if many:
         _, workspace = _workspace_after(cache, table, ctxs, heads)
         used = 16512 * len(ctxs) * heads
         assert bool((workspace[8256 * len(ctxs) * heads:used] != SENTINEL).any())
         assert (workspace[used:] == SENTINEL).all()
-    _check(cache, table, ctxs, heads, seed=1305, fp8=fp8)
-    rng = np.random.default_rng(1307)
-    for k in (769, 1025, 1400, 2048):
-        sparse = np.full((len(ctxs), k), -1, dtype=np.int32)
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1305).cuda()
+    out, split = [kt.attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), SCALE, selection_units=units)[0]
+                  for units in (ffi.ATTN_UNITS_AUTO, ffi.ATTN_UNITS_SPLIT)]
+    assert kt.torch.equal(out, split) == (not many)
+
+
+# The same of selections: which plans share their units so (`reserved` 5; 3: between four, 1: otherwise), at the lines of the rule
+# from both sides, and what the units and the split give for sequences shorter than the selection, empty ones and full ones.
+@pytest.mark.skipif(not kt.torch.cuda.is_available() or kt.torch.cuda.get_device_properties(0).multi_processor_count != 256,
+                    reason="the sizes are those of 256 CUs")
+@pytest.mark.parametrize("batch,heads,fp8,expected", [
+    (8, 64, False, {512: 3, 768: 3, 769: 5, 1536: 5, 1537: 1, 2048: 1}), (8, 64, True, {1024: 3, 1025: 5, 1536: 5, 1537: 1}),
+    (4, 64, False, {769: 1, 1100: 1}), (2, 64, False, {769: 5, 1408: 5, 1409: 1}), (1, 16, True, {1024: 3, 1025: 5, 1280: 5, 1281: 1}),
+    (9, 64, True, {1025: 5, 2048: 5}), (12, 64, False, {769: 5, 2048: 5}), (13, 64, False, {769: 1, 2048: 1}),
+    (25, 32, False, {769: 5, 1664: 5, 1665: 1}), (25, 32, True, {2048: 5}), (8, 32, False, {1100: 1}), (16, 16, False, {2048: 5}),
+    (12, 16, False, {1280: 5, 1281: 1}), (6, 128, False, {769: 5, 1408: 5, 1409: 1}), (4, 128, False, {1100: 1}), (9, 80, True, {1408: 5, 1409: 1})])
+def test_selections_in_units_shared_by_five_to_eight_workgroups(batch, heads, fp8, expected):
+    assert {k: kt.make_plan(batch, heads, k, 64, fp8, selection=True).reserved for k in expected} == expected
+    ctxs = [2100 - 150 * i for i in range(min(batch, 12))] + [33] * (batch - 12)
+    ctxs[batch // 2] = 0 if batch > 2 else ctxs[batch // 2]
+    cache, table = _cache(ctxs, 64, seed=1307, fp8=fp8)
+    rng = np.random.default_rng(1309)
+    for k in (min(expected), max(k for k, how in expected.items() if how == max(expected.values()))):
+        sparse = np.full((batch, k), -1, dtype=np.int32)
         for s, n in enumerate(ctxs):
             sparse[s, :min(n, k)] = rng.permutation(n)[:k]
-        plan = kt.make_plan(len(ctxs), heads, k, bs, fp8, selection=True)
-        fits = len(ctxs) * heads <= 12 * 64 and (heads <= 64 or k <= 1408)
-        assert plan.reserved == (5 if fits and k > (1024 if fp8 else 768) else plan.reserved) and (fits or plan.reserved != 5)
-        _check(cache, table, ctxs, heads, seed=1309, fp8=fp8, sparse=sparse)
+        _check(cache, table, ctxs, heads, seed=1311, fp8=fp8, sparse=sparse)
+        plan, workspace = _workspace_after(cache, table, ctxs, heads, sparse)
+        if plan.reserved == 5:
+            assert (workspace[16512 * batch * heads:] == SENTINEL).all()
 
 
 # The slices of up to eight parts are fp32: no further from float64 than the split units' bf16 partials, over rows that grow
 # along the context (the parts' weights lie far apart).
 @pytest.mark.parametrize("fp8", [False, True])
 def test_many_workgroups_are_as_precise_as_the_split(fp8):
-    ctxs, heads = [1900, 1200, 1025, 300], 64
-    cache, table = _cache(ctxs, 64, seed=1321, fp8=fp8, grow=lambda at: 0.1 + 4.0 * at / 1900)
+    ctxs, heads = [1700, 1200, 1025, 300], 64
+    cache, table = _cache(ctxs, 64, seed=1321, fp8=fp8, grow=lambda at: 0.1 + 4.0 * at / 1700)
     q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1323).cuda()
     expected, _ = kt.oracle_attention(cache, 0, q, table, ctxs, SCALE)
     errors = []
