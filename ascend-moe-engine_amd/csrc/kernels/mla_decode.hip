@@ -851,16 +851,15 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
   // Every wave walks the batch itself: the total number of tiles fixes the cut of the flat axis.
   // On the way the empty sequences (no tile, so no unit) get their zeros, spread over the workgroups.
   SeqWindow<SPARSE> win;
-  // The lengths of a window are asked for before those of the one ahead of it are looked at, and the window that the
-  // first unit begins in is not fetched again if it is the last one or the first: of a batch of 65 to 128 sequences a
-  // workgroup fetches the lengths in one memory trip, where it made three or four. (Append and attention of a layer, us: 100
-  // x 300..700 tokens 38.2 -> 36.9, 128 x 1000..2000 over an FP8 cache 61.5 -> 60.6, 70 x 2000..4000 69.9 -> 69.3.)
-  const int first_asked = SeqWindow<SPARSE>::Ask(a, lane0, 0);
-  int next_asked = a.batch > 64 ? SeqWindow<SPARSE>::Ask(a, lane0, 64) : 0;
-  int carry_tiles = 0, carry_live = 0;  // in front of the last window
-  win.Take(a, lane0, first_asked, 0, 0, 0);
+  // A batch of up to 64 sequences is one window. Beyond that the lengths of a window are asked for before those of the one
+  // ahead of it are looked at, and the window that the first unit begins in is not fetched again if it is the last one or
+  // the first: of 65 to 128 sequences a workgroup fetches the lengths in one memory trip, where it made three or four.
+  // (Append and attention of a layer, us: 100 x 300..700 tokens 38.2 -> 36.9, 128 x 1000..2000 over an FP8 cache 61.5 -> 60.6, 70 x
+  // 2000..4000 69.9 -> 69.3. The one window goes by itself, its code in front: as the first round of the same loop it cost every
+  // launch of a small batch up to 0.4 us, 32 x 1500 tokens 29.8 against 29.5, 4 x 5000..8000 over an FP8 cache 24.6 against 24.2.)
+  int first_asked = 0, carry_tiles = 0, carry_live = 0;  // in front of the last window
   int common_tiles = 0;  // the tile count all sequences with tiles share; -1 when they differ
-  for (;;) {
+  const auto look = [&]() __attribute__((always_inline)) {
     if constexpr (!SPARSE) {
       u64 empties = __builtin_amdgcn_ballot_w64(win.base + lane0 < a.batch && win.tiles == 0);
       while (empties != 0) {
@@ -871,12 +870,23 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
     }
     const int here = win.CommonTiles();
     if (here != 0) common_tiles = common_tiles == 0 || common_tiles == here ? here : -1;
-    if (win.base + 64 >= a.batch) break;
-    const int asked = next_asked;
-    if (win.base + 128 < a.batch) next_asked = SeqWindow<SPARSE>::Ask(a, lane0, win.base + 128);
-    carry_tiles = win.EndTiles();
-    carry_live = win.EndLive();
-    win.Take(a, lane0, asked, win.base + 64, carry_tiles, carry_live);
+  };
+  if (__builtin_expect(a.batch <= 64, 1)) {
+    win.Take(a, lane0, SeqWindow<SPARSE>::Ask(a, lane0, 0), 0, 0, 0);
+    look();
+  } else {
+    first_asked = SeqWindow<SPARSE>::Ask(a, lane0, 0);
+    int next_asked = SeqWindow<SPARSE>::Ask(a, lane0, 64);
+    win.Take(a, lane0, first_asked, 0, 0, 0);
+    for (;;) {
+      look();
+      if (win.base + 64 >= a.batch) break;
+      const int asked = next_asked;
+      if (win.base + 128 < a.batch) next_asked = SeqWindow<SPARSE>::Ask(a, lane0, win.base + 128);
+      carry_tiles = win.EndTiles();
+      carry_live = win.EndLive();
+      win.Take(a, lane0, asked, win.base + 64, carry_tiles, carry_live);
+    }
   }
   const Cut cut = MakeCut(a, win.EndTiles(), win.EndLive(), common_tiles, work_groups);
   const int tiles_per_unit = cut.tiles_per_unit, total_tiles = cut.total, pad = cut.pad;
@@ -1644,13 +1654,10 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
   }
   int first_unit = 0, partials = 0;
   if (WAYS == 1 || wave == 0) {
-    // (a window's lengths are asked for before those of the one ahead of it are looked at)
+    // (as in the kernel above: one window by itself, the lengths of several asked for ahead)
     SeqWindow<SPARSE> win;
-    const int first_asked = SeqWindow<SPARSE>::Ask(a, lane, 0);
-    int next_asked = a.batch > 64 ? SeqWindow<SPARSE>::Ask(a, lane, 64) : 0;
-    win.Take(a, lane, first_asked, 0, 0, 0);
     int end_tiles = 0, end_live = 0, seq_tiles = 0, common_tiles = 0;
-    for (;;) {
+    const auto look = [&]() __attribute__((always_inline)) {
       if (seq >= win.base && seq < win.base + 64) {
         end_tiles = win.End(seq, 0);
         end_live = win.End(seq, 1) - end_tiles;
@@ -1658,10 +1665,21 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
       }
       const int here = win.CommonTiles();
       if (here != 0) common_tiles = common_tiles == 0 || common_tiles == here ? here : -1;
-      if (win.base + 64 >= a.batch) break;
-      const int asked = next_asked;
-      if (win.base + 128 < a.batch) next_asked = SeqWindow<SPARSE>::Ask(a, lane, win.base + 128);
-      win.Take(a, lane, asked, win.base + 64, win.EndTiles(), win.EndLive());
+    };
+    if (__builtin_expect(a.batch <= 64, 1)) {
+      win.Take(a, lane, SeqWindow<SPARSE>::Ask(a, lane, 0), 0, 0, 0);
+      look();
+    } else {
+      const int first_asked = SeqWindow<SPARSE>::Ask(a, lane, 0);
+      int next_asked = SeqWindow<SPARSE>::Ask(a, lane, 64);
+      win.Take(a, lane, first_asked, 0, 0, 0);
+      for (;;) {
+        look();
+        if (win.base + 64 >= a.batch) break;
+        const int asked = next_asked;
+        if (win.base + 128 < a.batch) next_asked = SeqWindow<SPARSE>::Ask(a, lane, win.base + 128);
+        win.Take(a, lane, asked, win.base + 64, win.EndTiles(), win.EndLive());
+      }
     }
     if (seq_tiles != 0) {
       const Cut cut = MakeCut(a, win.EndTiles(), win.EndLive(), common_tiles, a.work_groups);
