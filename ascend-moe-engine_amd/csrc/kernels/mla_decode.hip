@@ -1232,7 +1232,7 @@ __global__ __launch_bounds__(kThreads) void MlaDecodeKernel(AttnArgs a) {
             for (int ks = 0; ks < kKSteps; ++ks) asm volatile("" ::"v"(q[ks]));
             for (; issued < G::kRing - 1 && issued < ntiles; ++issued) {
               if constexpr (kSoloPrologue) {
-                map.Begin(issued);  // keeps the cursor in step with the tiles this wave does not issue
+                map.Begin(tile_begin + issued);  // keeps the cursor in step with the tiles this wave does not issue
               } else {
                 if (!issue(issued)) last_unknown = issued;
               }
