@@ -1956,7 +1956,8 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
       const int i = tid + kHbThreads * j;
       if (i < min(own, kAttnHeadBlockTokens)) stage(i, selected ? listed[staged_from + i] : staged_from + i);
     }
-    if (lane == 0) words[kHbWaves + wave] = __builtin_amdgcn_ballot_w64(any_outside) != 0 ? 1 : 0;
+    const bool outside_here = __builtin_amdgcn_ballot_w64(any_outside) != 0;  // (asked of all lanes, not of the one that writes)
+    if (lane == 0) words[kHbWaves + wave] = outside_here ? 1 : 0;
 #pragma unroll
     for (int c = 0; c < kQSteps; ++c) asm volatile("" ::"v"(q[c]));  // (as below)
     __syncthreads();
@@ -1972,9 +1973,10 @@ __global__ __launch_bounds__(kHbThreads) void MlaSelectedHeadBlockKernel(AttnArg
       if (bad != 0) wave_end = min(wave_end, kHbThreads * j + 64 * wave + static_cast<int>(__builtin_ctzll(bad)));
       if (good && i < kAttnHeadBlockTokens) stage(i, index[j]);
     }
+    const bool outside_here = __builtin_amdgcn_ballot_w64(any_outside) != 0;  // (as above)
     if (lane == 0) {
       end_lds[wave] = wave_end;
-      end_lds[kHbWaves + wave] = __builtin_amdgcn_ballot_w64(any_outside) != 0 ? 1 : 0;
+      end_lds[kHbWaves + wave] = outside_here ? 1 : 0;
     }
     // Every role passes this statement with the query in hand: a wait of the compiler's for it further
     // down would not know of the tile loads issued from inline assembly, and would wait for them all.

@@ -394,6 +394,44 @@ def test_many_workgroups_are_as_precise_as_the_split(fp8):
     assert errors[0] <= 1.02 * errors[1]
 
 
+# Block-table entries that name no block, in units of 16 heads of one, two, four and eight workgroups, in blocks so small that a
+# hole is some of a wavefront's rows and not all: in the first, the last and a middle share, over a whole share, at the ends of a
+# sequence and in all of a short one; in a selection wherever its tokens lie. A table that names a block of
+# zeros gives the same bits.
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("bs", [16, 64, 48, 8])
+@pytest.mark.parametrize("parts", [1, 2, 4, 8])
+def test_holes_in_units_of_16_heads(parts, bs, fp8):
+    heads = 64
+    ctxs = {1: [256, 200, 33, 129, 1], 2: [768, 257, 33, 640], 4: [768, 257, 33, 640], 8: [1700, 1025, 33, 640, 1311, 1696]}[parts]
+    k = {1: 200, 2: 600, 4: 600, 8: 1100}[parts]
+    options = {"selection_units": ffi.ATTN_UNITS_HEAD_BLOCK_HALVES} if parts == 2 else {}
+    cache, table = _cache(ctxs, bs, seed=1341, fp8=fp8)
+    spare = sorted(set(range(cache.blocks)) - {int(b) for s, n in enumerate(ctxs) for b in table[s, :-(-n // bs)]})[0]
+    broken, zeroed = table.copy(), table.copy()
+    for s, n in enumerate(ctxs):
+        holes = [(20, n // 2, n - 1), (n - 1,), (0, n - 1), (), range(n // 8, n // 4), (n // 3, n // 2, n // 2 + 1, n - 5)][s]
+        for at, position in enumerate(holes):
+            broken[s, position // bs] = (-1, cache.blocks, 2 ** 31 - 1)[at % 3]
+            zeroed[s, position // bs] = spare
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1343).cuda()
+    rng = np.random.default_rng(1345)
+    sparse = np.full((len(ctxs), k), -1, dtype=np.int32)
+    for s, n in enumerate(ctxs):
+        sparse[s, :min(n, k)] = rng.permutation(n)[:k]
+    lens, chosen = kt.dev_i32(ctxs), kt.dev_i32(sparse)
+    expected, expected_lse = kt.oracle_attention(cache, 0, q, zeroed, ctxs, SCALE)
+    got = [kt.attention(cache, 0, q, kt.dev_i32(t), lens, SCALE, **options)[:2] for t in (broken, zeroed)]
+    split = kt.attention(cache, 0, q, kt.dev_i32(zeroed), lens, SCALE, selection_units=ffi.ATTN_UNITS_SPLIT)[0]
+    assert not kt.torch.equal(got[1][0], split)  # (the units ran)
+    assert np.abs(got[0][0].float().cpu().numpy() - expected).max() <= (TOL_FP8 if fp8 else TOL_BF16) * np.abs(expected).max()
+    assert np.abs(got[0][1].cpu().numpy() - expected_lse).max() <= 2e-2
+    assert kt.torch.equal(got[0][0], got[1][0]) and kt.torch.equal(got[0][1], got[1][1])
+    got = [kt.sparse_attention(cache, 0, q, kt.dev_i32(t), lens, chosen, SCALE, **options) for t in (broken, zeroed)]
+    assert got[0][2].reserved == {1: 1, 2: 1, 4: 3, 8: 5}[parts]
+    assert kt.torch.equal(got[0][0], got[1][0]) and kt.torch.equal(got[0][1], got[1][1])
+
+
 # Batches at the edges of a window of 64 sequences and with a window in the middle, whose lengths a workgroup asks for
 # ahead: units that begin in every window (one workgroup goes through all of them, 300 take a few tiles each), empty
 # sequences at the edges, a window without any tile. The same for selections, whose lengths are all the list's.
