@@ -1706,9 +1706,9 @@ __global__ __launch_bounds__(kMergeHeads * 64) void MlaMergeKernel(AttnArgs a) {
     // One wave per head takes few partials in groups of four or six: a padded group fetches its last row again and
     // again, 1 KB each from the L1, and with up to 8192 waves that is most of what the launch moves. (Groups of eight / so,
     // append and attention of a layer, us: 100 x 300..700 tokens 37.9 / 35.9, 128 x 1000..2000 over an FP8 cache 60.9 / 59.2, 70 x
-    // 2000..4000 69.8 / 69.3; with groups of two as well the first two take 35.9 and 59.0. Launches that share heads have
-    // little to pad, and the tests cost them 0.3 %: 20 x 2000..5000 tokens 34.6 / 34.7. Eight is tested first: tested last, 32 x
-    // 2048 tokens, which have eight partials, lost 0.4 %.)
+    // 2000..4000 69.8 / 69.3; with groups of two as well the first two take 35.9 and 59.0. The instantiations that share heads
+    // have little to pad and are built without the choice: the tests cost them 0.3 %, 20 x 2000..5000 tokens 34.7 with them, 34.6
+    // without. Eight is tested first: tested last, 32 x 2048 tokens, which have eight partials, lost 0.4 %.)
     const auto take = [&](auto size) __attribute__((always_inline)) {
       TakePartials<false, decltype(size)::value>(a, h >> 6, h & 63, a.max_units + seq, first_unit, 0, 1, partials, lane, state);
     };
@@ -1805,7 +1805,7 @@ hipError_t LaunchMerge(const AttnArgs& args, hipStream_t stream) {
 // are zero between launches (the last to arrive clears its word). A selection of fewer tiles than
 // parts is taken by the first of them, one tile each.
 // PARTS 8 stands for five to eight, as many as fit the CUs once (head_block_units), for more tokens than quarters are
-// ahead with or than a workgroup can stage: it stages its own share only, and the last part's waves take the slices in
+// ahead with or than a workgroup can stage: the parts go round the XCDs, each stages its own share only, and the last part's waves take the slices in
 // four at a time. Append and attention of a layer, us, split units and merge / so: 1 x 1100 tokens of 64 heads 19.3 / 15.9,
 // 8 x 1100 23.0 / 19.8, 8 x 1600 23.5 / 20.6 (FP8 24.6 / 23.4), 4 x 1600 20.8 / 20.2, 4 x 2400 21.4 / 22.1.
 constexpr int kHbWaves = kWaves, kHbThreads = kHbWaves * 64;

@@ -9,6 +9,7 @@ import pytest
 
 import kv_testing as kt
 import mlakv_ffi as ffi
+import oracle_ffi as orc
 
 pytestmark = pytest.mark.gpu
 
@@ -259,7 +260,7 @@ def test_rows_of_zeros_inside_long_segments(bs, fp8):
     the tiles they reach are staged with an unknown number of loads, full waits until they have landed, and
     the counted waits of whole tiles resume behind them. Holes in the first tiles, alone, in a row, a ring
     apart and a few tiles before the end. A table that names a block of zeros instead gives the same bits (blocks
-    of 16 slots: half a tile each; over an FP8 cache every tile is staged row by row there)."""
+    of 16 slots: half a tile each)."""
     heads, tile = 64, 32
     ctxs = [1700, 900, 3000, 70, 640, 1311]
     cache, table = _cache(ctxs, bs, seed=1101, fp8=fp8)
@@ -394,6 +395,28 @@ def test_many_workgroups_are_as_precise_as_the_split(fp8):
     assert errors[0] <= 1.02 * errors[1]
 
 
+# The same of selections, whose rows the split locates one by one: over rows that grow or fall along the selection, and equal ones.
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("shape", ["grow", "fall", "equal"])
+def test_selections_of_many_workgroups_are_as_precise_as_the_split(shape, fp8):
+    ctxs, heads, k = [2100, 1500, 1400, 1700, 1450, 900, 1600, 33, 2000], 64, 1400
+    factor = {"grow": lambda at: 0.1 + at / 500.0, "fall": lambda at: 4.3 - at / 500.0, "equal": None}[shape]
+    cache, table = _cache(ctxs, 64, seed=1331, fp8=fp8, grow=factor)
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1333).cuda()
+    rng = np.random.default_rng(1335)
+    sparse = np.full((len(ctxs), k), -1, dtype=np.int32)
+    for s, n in enumerate(ctxs):
+        sparse[s, :min(n, k)] = np.sort(rng.permutation(n)[:k])
+    expected, _ = kt.oracle_attention(cache, 0, q, table, ctxs, SCALE, sparse_indices=sparse)
+    errors, reserved = [], []
+    for options in ({}, {"selection_units": ffi.ATTN_UNITS_SPLIT}):
+        out, _, plan = kt.sparse_attention(cache, 0, q, kt.dev_i32(table), kt.dev_i32(ctxs), kt.dev_i32(sparse), SCALE, **options)
+        errors.append(np.linalg.norm(out.double().cpu().numpy() - expected) / np.linalg.norm(expected))
+        reserved.append(plan.reserved)
+    assert reserved == [5, 1]
+    assert errors[0] <= errors[1], errors
+
+
 # Block-table entries that name no block, in units of 16 heads of one, two, four and eight workgroups, in blocks so small that a
 # hole is some of a wavefront's rows and not all: in the first, the last and a middle share, over a whole share, at the ends of a
 # sequence and in all of a short one; in a selection wherever its tokens lie. A table that names a block of
@@ -430,6 +453,71 @@ def test_holes_in_units_of_16_heads(parts, bs, fp8):
     got = [kt.sparse_attention(cache, 0, q, kt.dev_i32(t), lens, chosen, SCALE, **options) for t in (broken, zeroed)]
     assert got[0][2].reserved == {1: 1, 2: 1, 4: 3, 8: 5}[parts]
     assert kt.torch.equal(got[0][0], got[1][0]) and kt.torch.equal(got[0][1], got[1][1])
+
+
+# A NaN query head gives a NaN row and a NaN cache row spoils its own sequence, whichever share of it holds the row; the others
+# keep their bits. Units shared by eight workgroups, whole contexts and selections.
+@pytest.mark.parametrize("fp8", [False, True])
+def test_units_shared_by_five_to_eight_workgroups_keep_a_nan(fp8):
+    ctxs, heads, k = [1700, 1300, 1025, 1400, 40, 1200], 64, 1100
+    cache, table = _cache(ctxs, 64, seed=1351, fp8=fp8)
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1353).cuda()
+    sparse = np.stack([np.r_[:min(n, k), [-1] * (k - min(n, k))] for n in ctxs]).astype(np.int32)
+    arguments = (kt.dev_i32(table), kt.dev_i32(ctxs))
+
+    def both(query):
+        return [kt.attention(cache, 0, query, *arguments, SCALE)[:2], kt.sparse_attention(cache, 0, query, *arguments, kt.dev_i32(sparse), SCALE)[:2]]
+
+    clean = both(q)
+    spoiled = q.clone()
+    spoiled[1, 5] = float("nan")
+    for (out, lse), (want, want_lse) in zip(both(spoiled), clean):
+        assert kt.torch.isnan(out[1, 5].float()).all() and kt.torch.isnan(lse[1, 5])
+        out[1, 5], lse[1, 5] = want[1, 5], want_lse[1, 5]
+        assert kt.torch.equal(out, want) and kt.torch.equal(lse, want_lse)
+    if fp8:
+        cache.scale[0, int(table[3, 900 // 64]), 900 % 64] = float("nan")
+    else:
+        cache.latent[0, int(table[3, 900 // 64]), 900 % 64] = float("nan")
+    others = [s for s in range(len(ctxs)) if s != 3]
+    for (out, lse), (want, want_lse) in zip(both(q), clean):
+        assert kt.torch.isnan(out[3].float()).all()
+        assert kt.torch.equal(out[others], want[others]) and kt.torch.equal(lse[others], want_lse[others])
+
+
+# Every way to say how long the contexts are leads to the same units shared by eight workgroups, and so does the quantising entry
+# point: the lengths by value and a bound of them under a plan for 8192 tokens, a plan of the longest context, and the
+# codes of that output with and without it.
+@pytest.mark.parametrize("fp8", [False, True])
+def test_units_shared_by_five_to_eight_workgroups_from_every_entry_point(fp8):
+    lib, bs, heads = ffi.load(), 64, 64
+    ctxs = [1700, 1, 0, 1030, 512]
+    table = kt.build_tables(ctxs, bs, sum(-(-n // bs) for n in ctxs) + 3, seed=1361, max_blocks=8192 // bs).table()
+    cache = kt.PagedCache(1, sum(-(-n // bs) for n in ctxs) + 3, bs, fp8=fp8)
+    kt.append(cache, kt.randn_bf16((1, sum(ctxs), LATENT), seed=1362).cuda(), kt.randn_bf16((1, sum(ctxs), ROPE), seed=1363).cuda(),
+              kt.dev_i32(kt.slots_for(table, ctxs, bs)))
+    q = kt.randn_bf16((len(ctxs), heads, LATENT + ROPE), seed=1364).cuda()
+    table_d, lens_d, row = kt.dev_i32(table), kt.dev_i32(ctxs), (LATENT + ROPE) * 2
+    want, want_lse, _ = kt.attention(cache, 0, q, table_d, lens_d, SCALE)
+    split = kt.attention(cache, 0, q, table_d, lens_d, SCALE, selection_units=ffi.ATTN_UNITS_SPLIT)[0]
+    assert not kt.torch.equal(want, split)
+    plan = kt.make_plan(len(ctxs), heads, 8192, bs, fp8)
+    workspace = kt.torch.empty(int(plan.workspace_bytes), dtype=kt.torch.uint8, device="cuda")
+    host = (C.c_int32 * len(ctxs))(*ctxs)
+    head = (C.byref(plan), C.byref(cache.view), 0, q.data_ptr(), heads * row, row, q.data_ptr() + LATENT * 2, heads * row, row,
+            table_d.data_ptr(), table_d.shape[1])
+    for call, lengths in ((lib.mlakvAttnDecodeHostLens, (C.cast(host, C.c_void_p),)), (lib.mlakvAttnDecodeBounded, (lens_d.data_ptr(), 1700))):
+        out, lse = kt.torch.full_like(want, float("nan")), kt.torch.full_like(want_lse, float("nan"))
+        ffi.check(call(*head, *lengths, SCALE, out.data_ptr(), heads * LATENT * 2, LATENT * 2, lse.data_ptr(), workspace.data_ptr(),
+                       workspace.numel(), kt.stream_ptr()))
+        kt.torch.cuda.synchronize()
+        assert kt.torch.equal(out, want) and kt.torch.equal(lse, want_lse)
+    want_codes, want_scales = orc.mx_quant_rows(kt.bits16(want).reshape(-1, LATENT))
+    for want_out in (False, True):
+        out, lse, _, codes, scales = kt.attention(cache, 0, q, table_d, lens_d, SCALE, quant=True, want_out=want_out)
+        assert (out is None or kt.torch.equal(out, want)) and kt.torch.equal(lse, want_lse)
+        assert np.array_equal(codes.cpu().numpy().reshape(-1, LATENT), want_codes)
+        assert np.array_equal(scales.cpu().numpy().reshape(-1, LATENT // 32), want_scales)
 
 
 # Batches at the edges of a window of 64 sequences and with a window in the middle, whose lengths a workgroup asks for
