@@ -408,7 +408,7 @@ int32_t SharedUnitParts(int32_t batch, int32_t heads, int32_t tokens, int32_t dt
 //  - for eight parts on more than a quarter of the CUs: a batch that leaves eight has so few rows that the split is in its smallest
 //    units (four tiles, of a selection two), which take no longer for more tokens, while a part here does;
 //  - for selections, whose rows the split locates while the query is on its way.
-// (One process and the next differ by up to 0.5 us where both sides are the split: the lines leave out what loses by more.)
+// (One process and the next differ by up to 0.5 us, once by 1, where both sides are the split: the lines leave out what loses by more.)
 // Measured, us a layer, split / so, equal lengths (ragged ones gain 1 to 5 us wherever they were tried, their longest at 1100 to 1900).
 // Whole contexts with their append, recorded, of 1100, 1500, 1700, 1900 tokens: 12 x 64 heads (five) 23.2 / 20.6, 24.7 / 22.1, 24.5 / 23.1,
 // 24.9 / 24.6, FP8 24.2 / 22.2, 25.3 / 23.5, 25.0 / 24.3, 25.5 / 25.8; 6 x 128 FP8 (five) 24.0 / 21.7, 25.1 / 23.0, 24.7 / 23.7, 25.1 / 25.4; 13 x 48 FP8
